@@ -188,6 +188,7 @@ _SIGNATURES = {
     "Rotate": ([_I, _I], _I),
     "RotateNew": ([_I, _I], _I),
     "RotateAdd": ([_I, _I], _I),
+    "RotateAddMany": ([_I, _PI, _I], _I),
     "RotateInto": ([_I, _I, _I], _I),
     "Conjugate": ([_I], _I),
     "ConjugateNew": ([_I], _I),

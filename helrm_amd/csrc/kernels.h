@@ -60,6 +60,55 @@ struct KeyMacArgs {
   u64 ka[HCK_MAXDIG];
 };
 
+// One key switch's key product (keymac1_kernel): at most HCK_KM1_DIG digits,
+// each with its own unrolled instantiation.  perm gathers every operand and
+// so applies the automorphism to the outputs (nullptr: identity).
+#define HCK_KM1_DIG 8
+struct KeyMac1Args {
+  const u64* digits;     // [dn][nqp][N]
+  const u64* own;        // the decomposed polynomial (NTT, Q rows)
+  const u64* key;        // [dnum][2][L+K][N], Montgomery form
+  const uint32_t* perm;
+  const u64 *add0, *add1;  // Q rows added to the parts (nullptr: none)
+  u64 *out0, *out1;      // [nqp][N] each
+  const ModC* mods;
+  int N, l, L, K, nqp, dn;
+  int seeded;            // the key's a halves are regenerated (ka) instead of read
+  u64 ka[HCK_MAXDIG];
+  // fold step (c0 set): out0's Q rows are not written; instead
+  //   c0_out = c + perm(c) + P^-1 * (part 0),  c = c0 (+ e0)
+  const u64 *c0, *e0;
+  u64* c0_out;
+  const u64 *pinv, *pinvp;
+};
+
+// From the product of one key switch to the digits of the next, in the
+// coefficient domain (link_kernel): per batch entry, with z the coefficients
+// of the QP polynomial x1 (level l) and M = (z - [z]_P) * P^-1 its ModDown,
+//   c1 = M (+ c1, with acc), and every digit of c1 extended to its other QP rows.
+// With x0p (P rows of a second QP polynomial) also e0 = -[x0p]_P * P^-1 on
+// the Q rows.  ginv: 0, or the inverse of the Galois element whose
+// automorphism x0p and x1 already carry: ModDown rounds down, so at the
+// positions where the automorphism changed the sign it is taken of the
+// negated word and the result is negated.
+struct LinkArgs {
+  const u64* x1; size_t x1_bstride;    // [nqp][N]
+  const u64* x0p;                      // [K][N] or nullptr (batch 1 only)
+  u64* c1; size_t c1_bstride;          // [l+1][N]
+  u64* e0;                             // [l+1][N]
+  u64* digits; size_t dig_bstride;     // [dn][nqp][N]
+  const struct BConvTable* ptab;       // P -> Q
+  const struct BConvTable* dtab[HCK_MAXDIG];  // per digit
+  const u64 *pinv, *pinvp;
+  const ModC* mods;
+  int N, l, L, K, nqp, dn, acc;
+  uint32_t ginv;
+};
+// LDS bytes of a link launch; at most LINK_LDS_MAX (K <= 8, dn <= HCK_MAXDIG) can be launched
+#define LINK_LDS_MAX 65536
+size_t link_lds_bytes(int l, int K, int dn);
+void launch_link(const LinkArgs& a, int batch, hipStream_t st);
+
 struct GiantAccArgs {
   const u64* digits;  // [ng][dn][nqp][N]
   size_t dig_bstride;
@@ -117,18 +166,19 @@ void launch_ntt(u64* data, size_t bstride, int batch, RowMap rm, int logN, bool 
 // Out-of-place: the transform of src's rows is written to the same rows of dst.
 void launch_ntt(const u64* src, size_t sstride, u64* dst, size_t dstride, int batch, RowMap rm, int logN, bool forward,
                 const NttTables& tw, hipStream_t st);
-// In-place NTT / inverse NTT of an explicit list of limbs: list is a device
-// array of nlimbs {int64 word offset from data, int modulus index, int pad}.
+// NTT / inverse NTT of an explicit list of limbs: list is a device array of
+// nlimbs {int64 word offset from data, int modulus index, int source: the
+// limb is read `source` limbs (of N words) past its offset, 0 in place}.
 void launch_ntt_list(u64* data, const void* list, int nlimbs, int logN, bool forward, const NttTables& tw, hipStream_t st);
 // Forward NTT of the Q rows 0..l of ext (the extension of [x]_P to Q) fused
 // with the ModDown combine: out[b][i][perm_inv^-1...] -- for every position p,
 // out[b][i][perm_inv[p]] = (x[b][i][p] - NTT(ext)[b][i][p]) * P^-1 (+ add[b][i][p]
 // for b < add_batches) (+ acc[b][i][perm_inv[p]] if acc, a buffer other than
-// out); ext itself is left in an intermediate state.
+// out); batch entries below x_from take x = 0; ext itself is left in an intermediate state.
 void launch_ntt_moddown(u64* ext, size_t ext_bstride, int batch, int l, int logN, const u64* x, size_t x_bstride,
                         u64* out, size_t o_bstride, const u64* add, size_t a_bstride, int add_batches,
                         const uint32_t* perm_inv, const u64* pinv, const u64* pinvp, const NttTables& tw, hipStream_t st,
-                        const u64* acc = nullptr, size_t c_bstride = 0);
+                        const u64* acc = nullptr, size_t c_bstride = 0, int x_from = 0);
 // Two scaled rescales of one ciphertext x at level l (l output rows) in one
 // forward transform: batch
 // entry b = 2 g + p (p the part) ends in
@@ -178,7 +228,11 @@ struct BConvJob {
   size_t out_off;  // word offset of the group's output inside a batch entry
 };
 #define HCK_MAXJOBS 16
-struct BConvJobs { BConvJob j[HCK_MAXJOBS]; int n, rows_per_block; };
+// ginv: 0, or the inverse of a Galois element whose automorphism the source
+// already carries (LinkArgs): at the positions whose sign it changed the
+// extension is taken of the negated sources and negated (launches of the
+// shared-source form only).
+struct BConvJobs { BConvJob j[HCK_MAXJOBS]; int n, rows_per_block; uint32_t ginv; };
 // Basis extension of every job for every batch entry, in one launch.
 void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, size_t out_bstride, int batch,
                   const ModC* mods, int N, hipStream_t st);
@@ -187,6 +241,7 @@ void launch_bconv(const u64* in, size_t in_bstride, int ns, const BConvTable* dt
                   const RowMap& rm, const ModC* mods, int N, bool force_v0, hipStream_t st);
 void launch_moddown_combine(u64* out, size_t o_bstride, const u64* x, size_t x_bstride, const u64* ext, size_t e_bstride, const u64* add, size_t a_bstride, int add_batches, const uint32_t* perm, const u64* pinv, const u64* pinvp, int qrows, int batch, const ModC* mods, int N, hipStream_t st);
 void launch_keymac(const KeyMacArgs& a, int batch, hipStream_t st);
+void launch_keymac1(const KeyMac1Args& a, hipStream_t st);
 void launch_giant_acc(const GiantAccArgs& a, hipStream_t st);
 void launch_diag_mac(const DiagMacArgs& a, hipStream_t st);
 void launch_rescale_spread(u64* t, const u64* u, int l, u64 half, const ModC* mods, int N, hipStream_t st);

@@ -329,6 +329,7 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
   u64* outb = out + (size_t)b * out_bstride + J.out_off;
   const RowMap rm = J.rm;
   const int nrows = rm.nact();
+  const bool flip = ((uint32_t)x * jobs.ginv & (uint32_t)(2 * N - 1)) >= (uint32_t)N;  // never with ginv = 0
   __shared__ u64 sy[MAXS][BCL_X];
   __shared__ double st[MAXS][BCL_X];
   __shared__ u64 svs[HCK_MAXMOD * (MAXS + 1)];
@@ -339,7 +340,8 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
     const BConvSrc s = tab->src[i];
     const bool act = i < ns;
     const u64 xi = inb[(size_t)(act ? i : 0) * N + x];
-    const u64 yi = shoup_mul(xi, s.hinv, s.hinvp, s.q);
+    u64 yi = shoup_mul(xi, s.hinv, s.hinvp, s.q);
+    if (flip && yi) yi = s.q - yi;
     const double t = (double)yi / s.qd;
     sy[i][lane] = act ? yi : 0;
     st[i][lane] = act ? t : 0.0;
@@ -367,8 +369,143 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
     const int m = rm.mod(row);
     const ModC mc = mods[m];
     const u64* __restrict__ h = hat + (size_t)m * ns;
-    outb[(size_t)row * N + x] = bconv_word8([&](int i) { return y[i]; }, h, mc.q, mc.qinv, svs[r * (ns + 1) + v]);
+    const u64 e = bconv_word8([&](int i) { return y[i]; }, h, mc.q, mc.qinv, svs[r * (ns + 1) + v]);
+    outb[(size_t)row * N + x] = flip && e ? mc.q - e : e;
   }
+}
+
+// From one key switch's product to the next one's digits (LinkArgs).  The
+// ModDown of the first, the automorphism's sum and the ModUp of the second
+// are all coefficient-wise, so one launch does them without a transform in
+// between: a rotation chain then runs the inverse transform of the product's
+// Q rows where it ran the forward transform of the ModDown's extension and
+// the inverse transform of the sum, and six launches a step instead of
+// eleven.  VALU-bound as the basis extensions it is made of (2 (l+1) + dn nqp
+// rows of 8 products a coefficient).  Shape as bconv_lds_kernel: 64
+// coefficients a workgroup, four waves; a wave computes every fourth row and
+// the rows' source terms meet in LDS.  At N = 2^16 with 23 Q and 8 P rows it
+// takes 43 us where the two extensions took 38 and the transforms between
+// them 46; a fold step goes from 190 to 161 us (11 steps at 11 Q rows: 134 to
+// 100 us a step).
+__global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
+  extern __shared__ u64 sm[];
+  const int lane = threadIdx.x & (BCL_X - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / BCL_X);
+  const int N = a.N, K = a.K, nq = a.l + 1, nqp = a.nqp, b = blockIdx.y;
+  const int x = blockIdx.x * BCL_X + lane;
+  const u64* x1 = a.x1 + (size_t)b * a.x1_bstride + x;
+  u64* c1 = a.c1 + (size_t)b * a.c1_bstride + x;
+  u64* digits = a.digits + (size_t)b * a.dig_bstride + x;
+  const bool two = a.x0p != nullptr;
+  const bool flip = ((uint32_t)x * a.ginv & (uint32_t)(2 * N - 1)) >= (uint32_t)N;
+  // LDS: source terms (P rows: y and y / p of both polynomials, 8 slots each;
+  // then the Q rows' y and y / q), then v * S mod t of every extended row
+  u64* U = sm;
+  u64* svs = sm + max(4 * 8, 2 * nq) * BCL_X;
+  const BConvTable* __restrict__ pt = a.ptab;
+  for (int part = two ? 0 : 1; part < 2; part++) {
+    const u64* src = part ? x1 + (size_t)nq * N : a.x0p + x;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const int i = w + 4 * k;
+      const BConvSrc s = pt->src[i];
+      const bool act = i < K;
+      u64 yi = shoup_mul(src[(size_t)(act ? i : 0) * N], s.hinv, s.hinvp, s.q);
+      if (flip && yi) yi = s.q - yi;
+      const double t = (double)yi / s.qd;
+      U[(part * 16 + i) * BCL_X + lane] = act ? yi : 0;
+      U[(part * 16 + 8 + i) * BCL_X + lane] = act ? (u64)__double_as_longlong(t) : 0;
+    }
+  }
+  for (int e = threadIdx.x; e < nq * (K + 1); e += blockDim.x) svs[e] = pt->vS[e];  // Q row r is modulus r
+  u64* svd = svs + nq * (K + 1);
+  for (int d = 0; d < a.dn; d++) {
+    const int st0 = d * K, ns = min(st0 + K, nq) - st0, wd = ns + 1, n = (nqp - ns) * wd;
+    const u64* __restrict__ vS = a.dtab[d]->vS;
+    for (int e = threadIdx.x; e < n; e += blockDim.x) {
+      const int rr = e / wd, row = rr < st0 ? rr : rr + ns;
+      svd[e] = vS[(size_t)(row < nq ? row : a.L + row - nq) * wd + (e - rr * wd)];
+    }
+    svd += n;
+  }
+  __syncthreads();
+  u64 y0[8], y1[8];
+  double v0f = 0.0, v1f = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    y1[i] = U[(16 + i) * BCL_X + lane];
+    v1f += __longlong_as_double((long long)U[(24 + i) * BCL_X + lane]);
+    if (two) {
+      y0[i] = U[i * BCL_X + lane];
+      v0f += __longlong_as_double((long long)U[(8 + i) * BCL_X + lane]);
+    }
+  }
+  const int v1 = (int)(u64)v1f, v0 = (int)(u64)v0f;
+  __syncthreads();
+  // a row's words are loaded while the row before it is computed
+  u64 zn = w < nq ? x1[(size_t)w * N] : 0, cn = a.acc && w < nq ? c1[(size_t)w * N] : 0;
+  for (int r = w; r < nq; r += 4) {
+    const ModC mc = a.mods[r];
+    const u64* __restrict__ h = pt->hat + (size_t)r * K;
+    const u64 pi = a.pinv[r], pip = a.pinvp[r];
+    const u64 z = zn, c = cn;
+    const int rn = min(r + 4, nq - 1);
+    zn = x1[(size_t)rn * N];
+    if (a.acc) cn = c1[(size_t)rn * N];
+    const u64 e1 = bconv_word8([&](int i) { return y1[i]; }, h, mc.q, mc.qinv, svs[r * (K + 1) + v1]);
+    const u64 m = shoup_mul(flip ? add_mod(z, e1, mc.q) : sub_mod(z, e1, mc.q), pi, pip, mc.q);
+    const u64 s = add_mod(c, m, mc.q);
+    c1[(size_t)r * N] = s;
+    const BConvSrc sd = a.dtab[r / K]->src[r % K];
+    const u64 yi = shoup_mul(s, sd.hinv, sd.hinvp, sd.q);
+    U[r * BCL_X + lane] = yi;
+    U[(nq + r) * BCL_X + lane] = (u64)__double_as_longlong((double)yi / sd.qd);
+    if (two) {
+      u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, mc.q, mc.qinv, svs[r * (K + 1) + v0]);
+      e0 = shoup_mul(e0, pi, pip, mc.q);
+      a.e0[(size_t)r * N + x] = flip || e0 == 0 ? e0 : mc.q - e0;
+    }
+  }
+  __syncthreads();
+  svd = svs + nq * (K + 1);
+  int first = w;  // this wave's first row of the digit: rows are dealt round robin over all digits
+  for (int d = 0; d < a.dn; d++) {
+    const int st0 = d * K, ns = min(st0 + K, nq) - st0, nrows = nqp - ns;
+    const BConvTable* __restrict__ dt = a.dtab[d];
+    u64 y[8];
+    double vf = 0.0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      const int r = st0 + (i < ns ? i : 0);
+      const u64 yi = U[r * BCL_X + lane];
+      const double t = __longlong_as_double((long long)U[(nq + r) * BCL_X + lane]);
+      y[i] = i < ns ? yi : 0;
+      vf += i < ns ? t : 0.0;
+    }
+    const int v = ns == 1 ? 0 : (int)(u64)vf;  // a digit of one modulus is spread without an overflow count
+    int rr = first;
+    for (; rr < nrows; rr += 4) {
+      const int row = rr < st0 ? rr : rr + ns;
+      const int m = row < nq ? row : a.L + row - nq;
+      const ModC mc = a.mods[m];
+      const u64* __restrict__ h = dt->hat + (size_t)m * ns;
+      digits[((size_t)d * nqp + row) * N] =
+          bconv_word8([&](int i) { return y[i]; }, h, mc.q, mc.qinv, svd[rr * (ns + 1) + v]);
+    }
+    first = rr - nrows;
+    svd += nrows * (ns + 1);
+  }
+}
+size_t link_lds_bytes(int l, int K, int dn) {
+  const int nq = l + 1, nqp = nq + K;
+  size_t words = (size_t)std::max(4 * 8, 2 * nq) * BCL_X + (size_t)nq * (K + 1);
+  for (int d = 0; d < dn; d++) {
+    const int ns = std::min(d * K + K, nq) - d * K;
+    words += (size_t)(nqp - ns) * (ns + 1);
+  }
+  return words * 8;
+}
+void launch_link(const LinkArgs& a, int batch, hipStream_t st) {
+  hipLaunchKernelGGL(link_kernel, dim3(a.N / BCL_X, batch), dim3(256), link_lds_bytes(a.l, a.K, a.dn), st, a);
 }
 void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, size_t out_bstride, int batch,
                   const ModC* mods, int N, hipStream_t st) {
@@ -516,6 +653,79 @@ void launch_keymac(const KeyMacArgs& a, int batch, hipStream_t st) {
   if (batch <= 0) return;
   hipLaunchKernelGGL(keymac_kernel, dim3(a.N / 256, a.nqp, batch), dim3(256), 0, st, a);
 }
+
+// The key product of one key switch.  DN digits unrolled, so that a word's
+// 2 DN (3 DN with the a halves read) loads are in flight together; with the
+// sum's bound DN q < 2^64 its high word needs no folding before the REDC.
+template <int DN, bool SEEDED, bool FOLD>
+__global__ __launch_bounds__(256) void keymac1_kernel(KeyMac1Args a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = blockIdx.y, N = a.N;
+  const bool qrow = k <= a.l;
+  const int src = a.perm ? (int)a.perm[i] : i;
+  const int kl = qrow ? k : a.L + (k - a.l - 1);
+  const ModC mc = a.mods[kl];
+  const int own_d = qrow ? k / a.K : -1;
+  const size_t kstride = (size_t)(a.L + a.K) * N, ro = (size_t)k * N;
+  u64 x[DN], kb[DN], ka[DN];
+#pragma unroll
+  for (int d = 0; d < DN; d++) {
+    const u64* dg = d == own_d ? a.own + ro : a.digits + (size_t)d * a.nqp * N + ro;
+    const u64* key = a.key + (size_t)d * 2 * kstride + (size_t)kl * N + src;
+    x[d] = dg[src];
+    kb[d] = __builtin_nontemporal_load(key);
+    if (!SEEDED) ka[d] = __builtin_nontemporal_load(key + kstride);
+  }
+  u64 add0 = 0, add1 = 0, c = 0;
+  if (qrow) {
+    if (FOLD) {
+      u64 ci = a.c0[ro + i], cs = a.c0[ro + src];
+      if (a.e0) {
+        ci = add_mod(ci, a.e0[ro + i], mc.q);
+        cs = add_mod(cs, a.e0[ro + src], mc.q);
+      }
+      c = add_mod(ci, cs, mc.q);
+    } else {
+      if (a.add0) add0 = a.add0[ro + src];
+      if (a.add1) add1 = a.add1[ro + src];
+    }
+  }
+  Acc128 A0, A1;
+  acc_zero(A0); acc_zero(A1);
+#pragma unroll
+  for (int d = 0; d < DN; d++) {
+    acc_mac(A0, x[d], kb[d]);
+    acc_mac(A1, x[d], SEEDED ? key_a_word(a.ka[d], (u64)kl * N + src, mc.q) : ka[d]);
+  }
+  // at most 8 products of words below q < 2^61: the sum stays below q * 2^64
+  u64 lo0, hi0, lo1, hi1;
+  acc_value(A0, lo0, hi0);
+  acc_value(A1, lo1, hi1);
+  // add0 enters the high word (v*2^64 == v*R mod q), so the REDC returns sum + add0
+  const u64 r0 = redc(lo0, add_mod(hi0, add0, mc.q), mc.q, mc.qinv);
+  u64 r1;
+  if (SEEDED) r1 = add_mod(mont_mul(redc(lo1, hi1, mc.q, mc.qinv), mc.r2, mc.q, mc.qinv), add1, mc.q);
+  else r1 = redc(lo1, add_mod(hi1, add1, mc.q), mc.q, mc.qinv);
+  if (FOLD && qrow) a.c0_out[ro + i] = add_mod(c, shoup_mul(r0, a.pinv[k], a.pinvp[k], mc.q), mc.q);
+  else a.out0[ro + i] = r0;
+  a.out1[ro + i] = r1;
+}
+template <int DN>
+static void launch_keymac1_t(const KeyMac1Args& a, hipStream_t st) {
+  if (DN < a.dn) {
+    if constexpr (DN < HCK_KM1_DIG) launch_keymac1_t<DN + 1>(a, st);
+    return;
+  }
+  const dim3 grid(a.N / 256, a.nqp), block(256);
+  if (a.c0) {
+    if (a.seeded) hipLaunchKernelGGL((keymac1_kernel<DN, true, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((keymac1_kernel<DN, false, true>), grid, block, 0, st, a);
+  } else {
+    if (a.seeded) hipLaunchKernelGGL((keymac1_kernel<DN, true, false>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((keymac1_kernel<DN, false, false>), grid, block, 0, st, a);
+  }
+}
+void launch_keymac1(const KeyMac1Args& a, hipStream_t st) { launch_keymac1_t<1>(a, st); }
 
 // Giant-step accumulation of the BSGS linear transform: for every QP row and
 // output position i, sum over giant groups g of

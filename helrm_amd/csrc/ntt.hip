@@ -239,6 +239,7 @@ struct ModDownEpi {
   const uint32_t* perm_inv;             // nullptr: identity
   const u64 *pinv, *pinvp;              // [mod] P^-1 mod q and its Shoup companion
   const u64* acc; size_t c_bstride;     // nullptr, or added at the output position (out != acc)
+  int x_from;                           // batch entries below it take x = 0
   // scaled pair (launch_ntt_rescale_pair): batch entry b = 2 g + p reads part
   // p of x, multiplies it by ks's K_g of its row, adds C_g to part 0 and
   // writes group g to out (g = 0) or out2 (g = 1); ks == nullptr: off
@@ -277,7 +278,7 @@ __device__ __forceinline__ LimbRef limb_ref(const NttArgs& a, int y) {
 }
 // src offset of the same limb (first pass of an out-of-place transform)
 __device__ __forceinline__ int64_t limb_src_off(const NttArgs& a, int y, const LimbRef& l) {
-  if (a.list) return l.off;
+  if (a.list) return l.off + ((int64_t)l.pad << a.logN);
   return (int64_t)l.pad * (int64_t)a.sstride + (l.off - (int64_t)l.pad * (int64_t)a.bstride);
 }
 
@@ -428,7 +429,7 @@ __device__ __forceinline__ void row_fwd_tail(const NttArgs& a, const u64* srow, 
     u64 xv[16], av[16];
     uint32_t dst[16];
 #pragma unroll
-    for (int i = 0; i < 16; i++) xv[i] = __builtin_nontemporal_load(&xr[j + P * i]);
+    for (int i = 0; i < 16; i++) xv[i] = b < a.e.x_from ? 0 : __builtin_nontemporal_load(&xr[j + P * i]);
     if (ar) {
 #pragma unroll
       for (int i = 0; i < 16; i++) av[i] = __builtin_nontemporal_load(&ar[j + P * i]);
@@ -819,7 +820,7 @@ __device__ __forceinline__ void row8_fwd_tail(const NttArgs& a, const u64* srow,
     u64 xv[8], av[8];
     uint32_t dst[8];
 #pragma unroll
-    for (int i = 0; i < 8; i++) xv[i] = __builtin_nontemporal_load(&xr[w8_elem(L0, t, i)]);
+    for (int i = 0; i < 8; i++) xv[i] = b < a.e.x_from ? 0 : __builtin_nontemporal_load(&xr[w8_elem(L0, t, i)]);
     if (ar) {
 #pragma unroll
       for (int i = 0; i < 8; i++) av[i] = __builtin_nontemporal_load(&ar[w8_elem(L0, t, i)]);
@@ -1143,7 +1144,7 @@ void launch_ntt(const u64* src, size_t sstride, u64* data, size_t bstride, int b
 void launch_ntt_moddown(u64* ext, size_t ext_bstride, int batch, int l, int logN, const u64* x, size_t x_bstride,
                         u64* out, size_t o_bstride, const u64* add, size_t a_bstride, int add_batches,
                         const uint32_t* perm_inv, const u64* pinv, const u64* pinvp, const NttTables& tw, hipStream_t st,
-                        const u64* acc, size_t c_bstride) {
+                        const u64* acc, size_t c_bstride, int x_from) {
   const RowMap rm{l + 1, l + 1, 0, 0, 0, 0};
   NttArgs a{};
   a.list = nullptr;
@@ -1154,7 +1155,7 @@ void launch_ntt_moddown(u64* ext, size_t ext_bstride, int batch, int l, int logN
   a.twr = reinterpret_cast<const uint4*>(tw.twr);
   a.epi = 1;
   a.e = ModDownEpi{x, x_bstride, out, o_bstride, add, a_bstride, add_batches, perm_inv, pinv, pinvp, acc, c_bstride,
-                   nullptr, 0, nullptr};
+                   x_from, nullptr, 0, nullptr};
   ntt_launch(a, (l + 1) * batch, true, st);
 }
 void launch_ntt_rescale_pair(u64* t, size_t t_bstride, int l, int logN, const u64* x, size_t x_bstride, u64* out0,
@@ -1169,7 +1170,7 @@ void launch_ntt_rescale_pair(u64* t, size_t t_bstride, int l, int logN, const u6
   a.tw = reinterpret_cast<const uint4*>(tw.tw);
   a.twr = reinterpret_cast<const uint4*>(tw.twr);
   a.epi = 1;
-  a.e = ModDownEpi{x, x_bstride, out0, o_bstride, nullptr, 0, 0, nullptr, rsinv, rsinvp, nullptr, 0, ks, l, out1};
+  a.e = ModDownEpi{x, x_bstride, out0, o_bstride, nullptr, 0, 0, nullptr, rsinv, rsinvp, nullptr, 0, 0, ks, l, out1};
   ntt_launch(a, l * 4, true, st);
 }
 

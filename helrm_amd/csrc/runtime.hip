@@ -361,6 +361,7 @@ struct Scheme {
   std::map<std::pair<int, int>, std::unique_ptr<BConvHost>> bconv;
   std::map<u64, DevArray<uint32_t>> perms, perm_invs;
   std::map<std::tuple<int, int, size_t>, std::unique_ptr<struct DigitRows>> digit_rows;
+  std::map<int, std::unique_ptr<struct FoldRows>> fold_rows;  // per level
   // Galois keys this library generated (a halves a function of the seed, the
   // key's stream and the word's position, regenerated by the kernels); a
   // loaded key is read whole
@@ -555,15 +556,18 @@ const DigitRows& digit_rows(int l, int batch, size_t dstride) {
   auto it = s.digit_rows.find(key);
   if (it != s.digit_rows.end()) return *it->second;
   const int N = s.N, K = s.K, nqp = l + 1 + K, dn = (l + 1 + K - 1) / K;
-  // modulus-major, so that consecutive limbs share their twiddle tables in L2
+  // modulus-major, so that consecutive limbs share their twiddle tables in
+  // L2; the P rows (integer butterflies) first, as in RowMap launches
   std::vector<LimbRefH> v;
-  for (int k = 0; k < nqp; k++)
+  for (int i = 0, k; i < nqp; i++) {
+    k = i < K ? l + 1 + i : i - K;
     for (int b = 0; b < batch; b++)
       for (int d = 0; d < dn; d++) {
         const int st0 = d * K, en = std::min(st0 + K, l + 1);
         if (k < st0 || k >= en)
           v.push_back(LimbRefH{(int64_t)((size_t)b * dstride + ((size_t)d * nqp + k) * N), qp_mod(l, k), 0});
       }
+  }
   auto dr = std::make_unique<DigitRows>();
   dr->n = (int)v.size();
   dr->list = DevArray<LimbRefH>(v.size());
@@ -1079,6 +1083,39 @@ void ct_drop_to(Cipher& c, int level) {
 // ============================================================================
 // evaluator operations
 // ============================================================================
+// The per-digit stream keys of a Galois key generated here, in ka (nullptr: a
+// loaded key, read whole).
+const u64* seeded_keys(u64 galel, int dn, u64 (&ka)[HCK_MAXDIG]) {
+  if (!sch().seeded_gk.count(galel)) return nullptr;
+  for (int d = 0; d < dn; d++) ka[d] = stream_key(ST_GK_A(galel, (u64)d));
+  return ka;
+}
+// dd[part][nqp][N] = the product of the decomposition (digits, own rows own)
+// with key (+ add0, add1 on the Q rows).  Up to HCK_KM1_DIG digits take the
+// unrolled kernel, longer decompositions the looping one.
+void key_product(int l, const u64* digits, const u64* own, const u64* key, const u64* ka, const u64* add0, const u64* add1,
+                 u64* dd) {
+  Scheme& s = sch();
+  const int N = s.N, K = s.K, nqp = l + 1 + K, dn = (l + 1 + K - 1) / K;
+  if (dn <= HCK_KM1_DIG) {
+    KeyMac1Args a{};
+    a.digits = digits; a.own = own; a.key = key; a.add0 = add0; a.add1 = add1;
+    a.out0 = dd; a.out1 = dd + (size_t)nqp * N; a.mods = s.d_mods.p;
+    a.N = N; a.l = l; a.L = s.L; a.K = K; a.nqp = nqp; a.dn = dn;
+    a.seeded = ka ? 1 : 0;
+    if (ka) std::copy(ka, ka + dn, a.ka);
+    launch_keymac1(a, s.st);
+    return;
+  }
+  KeyMacArgs a{};
+  a.digits = digits; a.key1 = key; a.add0 = add0; a.add1 = add1; a.own = own;
+  a.out0 = dd; a.out1 = dd + (size_t)nqp * N; a.mods = s.d_mods.p;
+  a.N = N; a.l = l; a.L = s.L; a.K = K; a.nqp = nqp; a.dn = dn;
+  a.seeded = ka ? 1 : 0;
+  if (ka) std::copy(ka, ka + dn, a.ka);
+  launch_keymac(a, 1, s.st);
+}
+
 // Key-switched automorphism of ct into out (2 (l+1) N words, out != ct):
 // c1 decomposed and extended to QP, key product fused with nothing else,
 // ModDown of both parts with sigma applied in its epilogue and c0 added.
@@ -1108,17 +1145,8 @@ void automorphism_core(const Cipher& ct, u64 galel, const u64* key, const uint32
     digits = digits_buf.p; dd = dd_buf.p;
   }
   decompose_modup(l, ct.d.p + (size_t)(l + 1) * N, 0, 1, digits, false, coef);
-  KeyMacArgs a{};
-  a.digits = digits; a.dig_bstride = 0; a.digits_per_batch = 0; a.key = nullptr; a.perm = nullptr;
-  a.key1 = key; a.perm1 = nullptr; a.add0 = nullptr;
-  a.own = ct.d.p + (size_t)(l + 1) * N; a.own_bstride = 0;
-  a.out0 = dd; a.out1 = dd + (size_t)nqp * N; a.out_bstride = 0; a.mods = s.d_mods.p;
-  a.N = N; a.l = l; a.L = s.L; a.K = K; a.nqp = nqp; a.dn = dn;
-  if (s.seeded_gk.count(galel)) {
-    a.seeded = 1;
-    for (int d = 0; d < dn; d++) a.ka[d] = stream_key(ST_GK_A(galel, (u64)d));
-  }
-  launch_keymac(a, 1, s.st);
+  u64 ka[HCK_MAXDIG];
+  key_product(l, digits, ct.d.p + (size_t)(l + 1) * N, key, seeded_keys(galel, dn, ka), nullptr, nullptr, dd);
   mod_down(l, dd, (size_t)nqp * N, 2, out, (size_t)(l + 1) * N, ct.d.p, 0, 1, perm_inv, md, acc);
 }
 std::unique_ptr<Cipher> automorphism(const Cipher& ct, u64 galel, bool lt_keyset) {
@@ -1126,6 +1154,129 @@ std::unique_ptr<Cipher> automorphism(const Cipher& ct, u64 galel, bool lt_keyset
   auto out = new_ct(ct.level, ct.scale); out->logslots = ct.logslots;
   timed("rotate", [&] { automorphism_core(ct, galel, key, perm_inv_for(galel), out->d.p, nullptr); });
   return out;
+}
+// The limbs of a fold step's transforms at level l, offsets into the fold's
+// workspace (fold_ws): forward, every digit's extended rows, the new c1 (read
+// from its coefficients) and e0; inverse, the key product's part 1 and the P
+// rows of part 0.
+struct FoldRows { DevArray<LimbRefH> fwd, inv; int nfwd = 0, ninv = 0; };
+struct FoldWs { size_t digits, c1n, coef, e0, dd, c0a, c0b, words; };
+FoldWs fold_ws(int l) {
+  Scheme& s = sch();
+  const size_t N = s.N, K = s.K, nq = l + 1, nqp = nq + K, dn = (nq + K - 1) / K;
+  FoldWs w{};
+  size_t o = 0;
+  auto take = [&](size_t rows) { const size_t at = o; o += rows * N; return at; };
+  // c0a, c0b ahead of c1n: the last step's epilogue reads both as one batch
+  w.c0a = take(nq); w.c0b = take(nq); w.c1n = take(nq); w.coef = take(nq);
+  w.e0 = take(nq); w.dd = take(2 * nqp); w.digits = take(dn * nqp);
+  w.words = o;
+  return w;
+}
+const FoldRows& fold_rows(int l) {
+  Scheme& s = sch();
+  auto it = s.fold_rows.find(l);
+  if (it != s.fold_rows.end()) return *it->second;
+  const int N = s.N, K = s.K, nq = l + 1, nqp = nq + K, dn = (nq + K - 1) / K;
+  const FoldWs w = fold_ws(l);
+  // modulus-major, P rows first, as digit_rows
+  std::vector<LimbRefH> f, b;
+  for (int i = 0; i < nqp; i++) {
+    const int k = i < K ? nq + i : i - K, m = qp_mod(l, k);
+    for (int d = 0; d < dn; d++)
+      if (k >= nq || k / K != d) f.push_back(LimbRefH{(int64_t)(w.digits + ((size_t)d * nqp + k) * N), m, 0});
+    if (k < nq) {
+      f.push_back(LimbRefH{(int64_t)(w.c1n + (size_t)k * N), m, (int)((w.coef - w.c1n) / N)});
+      f.push_back(LimbRefH{(int64_t)(w.e0 + (size_t)k * N), m, 0});
+    } else {
+      b.push_back(LimbRefH{(int64_t)(w.dd + (size_t)k * N), m, 0});
+    }
+    b.push_back(LimbRefH{(int64_t)(w.dd + (size_t)(nqp + k) * N), m, 0});
+  }
+  auto fr = std::make_unique<FoldRows>();
+  fr->nfwd = (int)f.size(); fr->ninv = (int)b.size();
+  fr->fwd = DevArray<LimbRefH>(f.size()); upload(fr->fwd.p, f.data(), f.size());
+  fr->inv = DevArray<LimbRefH>(b.size()); upload(fr->inv.p, b.data(), b.size());
+  const FoldRows& ref = *fr;
+  s.fold_rows[l] = std::move(fr);
+  return ref;
+}
+// ct += Rotate(ct) by each Galois element of ge in turn (a Linear's output
+// fold), word for word what one automorphism_core with acc per step computes.
+// Between two steps c1 is needed in both domains: its coefficients feed the
+// next decomposition, its transform the next key product's own rows.  So the
+// key product's part 1 is taken to the coefficient domain whole (not only its
+// P rows) and link_kernel goes from there to the next digits: one forward and
+// one inverse transform a step, where a step by itself runs two of each one
+// after the other.  The automorphism is applied by the key product's gather;
+// c0 stays in the NTT domain, one transform (e0) behind.
+void fold_rotations(Cipher& ct, const std::vector<u64>& ge) {
+  Scheme& s = sch();
+  const int l = ct.level, N = s.N, K = s.K, nq = l + 1, nqp = nq + K, dn = (nq + K - 1) / K;
+  const size_t qs = (size_t)nq * N;
+  const FoldWs w = fold_ws(l);
+  const FoldRows& fr = fold_rows(l);
+  const DigitRows& dr = digit_rows(l, 1, (size_t)dn * nqp * N);
+  DU64 ws_buf(w.words);
+  u64* ws = ws_buf.p;
+  u64 *digits = ws + w.digits, *coef = ws + w.coef, *dd = ws + w.dd, *c0cur = ws + w.c0a, *c0nxt = ws + w.c0b;
+  u64* ddp = dd + qs;  // P rows of part 0; those of part 1 nqp rows on
+  const u64 *c0 = ct.d.p, *own = ct.d.p + qs, *e0 = nullptr;
+  // the first decomposition
+  ntt_oop(own, 0, coef, 0, 1, rows_q(l), false);
+  BConvJobs jobs{};
+  jobs.n = dn;
+  LinkArgs lk{};
+  for (int d = 0; d < dn; d++) {
+    const int st0 = d * K, en = std::min(st0 + K, nq);
+    lk.dtab[d] = bconv_table_cached(st0, en).dtab.p;
+    jobs.j[d] = BConvJob{lk.dtab[d], st0, en - st0, en - st0 == 1 ? 1 : 0, 0, RowMap{nqp, nq, 0, s.L, st0, en}, (size_t)d * nqp * N};
+  }
+  launch_bconv(coef, 0, jobs, digits, 0, 1, s.d_mods.p, N, s.st);
+  launch_ntt_list(digits, dr.list.p, dr.n, s.logN, true, s.tw, s.st);
+  BConvHost& bt = bconv_table_cached(s.L, s.L + K);
+  lk.x1 = dd + (size_t)nqp * N; lk.x0p = ddp; lk.c1 = coef; lk.e0 = ws + w.e0; lk.digits = digits; lk.ptab = bt.dtab.p;
+  lk.pinv = s.pinv_w.p; lk.pinvp = s.pinv_wp.p; lk.mods = s.d_mods.p;
+  lk.N = N; lk.l = l; lk.L = s.L; lk.K = K; lk.nqp = nqp; lk.dn = dn; lk.acc = 1;
+  const u64 M = 2 * (u64)N;
+  for (size_t i = 0; i < ge.size(); i++) {
+    const uint32_t ginv = (uint32_t)invmod_odd(ge[i], M);
+    KeyMac1Args a{};
+    a.digits = digits; a.own = own; a.key = s.gkeys.at(ge[i])->p; a.perm = perm_for(ge[i]);
+    a.out0 = dd; a.out1 = dd + (size_t)nqp * N; a.mods = s.d_mods.p;
+    a.N = N; a.l = l; a.L = s.L; a.K = K; a.nqp = nqp; a.dn = dn;
+    a.seeded = seeded_keys(ge[i], dn, a.ka) ? 1 : 0;
+    a.c0 = c0; a.e0 = e0; a.c0_out = c0nxt; a.pinv = s.pinv_w.p; a.pinvp = s.pinv_wp.p;
+    launch_keymac1(a, s.st);
+    std::swap(c0cur, c0nxt);
+    if (i + 1 == ge.size()) {
+      // the last ModDown ends in the NTT domain: c0 = c0cur - NTT(ext0) P^-1,
+      // c1 = own + (x1 - NTT(ext1)) P^-1
+      ntt(ddp, (size_t)nqp * N, 2, rows_p(), false);
+      BConvJobs pj{};
+      pj.n = 1; pj.ginv = ginv;
+      pj.j[0] = BConvJob{bt.dtab.p, 0, K, 0, 0, rows_q(l), 0};
+      launch_bconv(ddp, (size_t)nqp * N, pj, digits, qs, 2, s.d_mods.p, N, s.st);
+      auto out = new_ct(l, ct.scale);
+      launch_ntt_moddown(digits, qs, 2, l, s.logN, dd, (size_t)nqp * N, out->d.p, qs, c0cur, (size_t)(own - c0cur), 2, nullptr,
+                         s.pinv_w.p, s.pinv_wp.p, s.tw, s.st, nullptr, 0, 1);
+      std::swap(ct.d, out->d);
+      return;
+    }
+    launch_ntt_list(ws, fr.inv.p, fr.ninv, s.logN, false, s.tw, s.st);
+    lk.ginv = ginv;
+    launch_link(lk, 1, s.st);
+    launch_ntt_list(ws, fr.fwd.p, fr.nfwd, s.logN, true, s.tw, s.st);
+    own = ws + w.c1n; c0 = c0cur; e0 = ws + w.e0;
+  }
+}
+// Whether fold_rotations can run at level l: one source group of P and every
+// digit within the eight sources of a row, the links' terms in LDS.  A single
+// step has no link and is the plain rotation's.
+bool fold_chains(int l, size_t steps) {
+  Scheme& s = sch();
+  const int dn = (l + 1 + s.K - 1) / s.K;
+  return steps >= 2 && s.K <= 8 && dn <= HCK_KM1_DIG && link_lds_bytes(l, s.K, dn) <= LINK_LDS_MAX;
 }
 // ---- plaintext, scalar and ciphertext products (Lattigo ckks Evaluator
 // Mul / Add with a constant / MulRelin, restated for the GPU) ----
@@ -1207,18 +1358,10 @@ std::unique_ptr<Cipher> mul_relin_ct(const Cipher& a, const Cipher& b, bool resc
                 rescale ? s.pmod_w.p : nullptr, rescale ? s.pmod_wp.p : nullptr, s.d_mods.p, N, s.st);
   DU64 digits((size_t)dn * nqp * N), dd((size_t)2 * nqp * N);
   decompose_modup(l, d2, 0, 1, digits.p, false);
-  KeyMacArgs k{};
-  k.digits = digits.p; k.dig_bstride = 0; k.digits_per_batch = 0; k.key = nullptr; k.perm = nullptr;
-  k.key1 = s.rlk->p; k.perm1 = nullptr;
-  k.add0 = rescale ? d0 : nullptr; k.add1 = rescale ? d1 : nullptr;
-  k.own = d2; k.own_bstride = 0;
-  k.out0 = dd.p; k.out1 = dd.p + (size_t)nqp * N; k.out_bstride = 0; k.mods = s.d_mods.p;
-  k.N = N; k.l = l; k.L = s.L; k.K = K; k.nqp = nqp; k.dn = dn;
-  if (s.rlk_seeded) {
-    k.seeded = 1;
-    for (int d = 0; d < dn; d++) k.ka[d] = stream_key(ST_RLK_A((u64)d));
-  }
-  launch_keymac(k, 1, s.st);
+  u64 ka[HCK_MAXDIG];
+  if (s.rlk_seeded)
+    for (int d = 0; d < dn; d++) ka[d] = stream_key(ST_RLK_A((u64)d));
+  key_product(l, digits.p, d2, s.rlk->p, s.rlk_seeded ? ka : nullptr, rescale ? d0 : nullptr, rescale ? d1 : nullptr, dd.p);
   if (rescale) {
     auto out = new_ct(l - 1, a.scale * b.scale / (double)s.mod[l]); out->logslots = a.logslots;
     mod_down_rescale(l, dd.p, (size_t)nqp * N, 2, out->d.p, (size_t)l * N);
@@ -2114,6 +2257,31 @@ int RotateAdd(int ctID, int amount) {
 // rotation key must exist already.  A call on the other stream of the
 // scheme waits for the previous call's key switch; calls from several host
 // threads or processes sharing the GPU race on the array.
+int RotateAddMany(int ctID, const int* amounts, int lenAmounts) {
+  return guard([&] {
+    Scheme& s = sch();
+    Cipher& ct = get_ct(ctID);
+    REQUIRE(lenAmounts >= 0, "RotateAddMany: negative number of rotations");
+    std::vector<u64> ge;
+    for (int i = 0; i < lenAmounts; i++) {
+      ge.push_back(galois_element(amounts[i]));
+      ensure_galois_key(ge.back());
+      s.rot_keys.insert(ge.back());
+    }
+    timed("fold", [&] {
+      if (fold_chains(ct.level, ge.size())) {
+        fold_rotations(ct, ge);
+      } else {
+        for (u64 g : ge) {
+          auto out = new_ct(ct.level, ct.scale);
+          automorphism_core(ct, g, key_ptr(g, false), perm_inv_for(g), out->d.p, nullptr, ct.d.p);
+          std::swap(ct.d, out->d);
+        }
+      }
+    });
+    return ctID;
+  });
+}
 int RotateInto(int ctID, int amount, int outID) {
   return guard([&] {
     Scheme& s = sch();

@@ -335,6 +335,20 @@ class CipherTensor:
         rolled.free()
         return self
 
+    def fold(self, amounts):
+        """add_rolled by each amount in turn, in place: a Linear's whole output
+        fold (linear.py:115-117).  One backend call per ciphertext
+        (RotateAddMany) when the backend has it; else step by step."""
+        b = self.scheme.backend
+        amounts = [int(a) for a in amounts]
+        if hasattr(b, "RotateAddMany"):
+            for c in self.ids:
+                b.RotateAddMany(c, amounts)
+            return self
+        for a in amounts:
+            self.add_rolled(a)
+        return self
+
     def free(self):
         for c in self.ids:
             self.scheme.backend.DeleteCiphertext(c)
@@ -456,8 +470,7 @@ class LinearLayer:
     def forward(self, x):
         out = self.evaluate_lt(x)
         slots = self.scheme.params.get_slots()
-        for i in range(1, self.output_rotations + 1):
-            out.add_rolled(slots // (2 ** i))
+        out.fold(slots // (2 ** i) for i in range(1, self.output_rotations + 1))
         out += self.on_bias_ptxt
         return out
 

@@ -100,6 +100,11 @@ int RotateNew(int ciphertextID, int amount); /* evaluator.go:89-101 */
  * the add done in the key switch's last pass.  Same words as RotateNew +
  * AddCiphertext.  Returns ciphertextID. */
 int RotateAdd(int ciphertextID, int amount);
+/* [ext] RotateAdd by each amount in turn: a Linear's whole output fold in one
+ * call.  Same words as the single steps; the key switches of consecutive
+ * steps share their transforms.  Every key is made first, so a failure leaves
+ * the ciphertext as it was.  Returns ciphertextID. */
+int RotateAddMany(int ciphertextID, const int* amounts, int lenAmounts);
 /* [ext] No counterpart in the reference.  For callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops): RotateNew
  * written into the existing ciphertext outID (!= ciphertextID, with room for

@@ -16,6 +16,13 @@
 // values in [0, 2q); each pass's output is reduced to [0, q) only where the
 // transform ends, so the result equals the textbook NTT word for word.
 // Twiddles are (w, floor(w 2^64 / q)) pairs read as one 16-byte load.
+// In the 16-word kernels a round's 15 twiddle pairs (60 registers) are loaded
+// after the exchange that precedes it, never while the words of the round
+// before are still live, and the ModDown epilogue takes 8 words at a time:
+// 94 to 108 VGPRs (four or five waves per SIMD) instead of 124 to 168 (three).
+// At N = 2^16 and 744 limbs the epilogue's row pass takes 232 us instead of
+// 241 and the forward column pass 185 instead of 192; the batch of 1,536
+// float64 limbs stays at the rate of a copy (4.6 of 4.8 TB/s).
 //
 // Limbs whose modulus is at most FP_QMAX (the 40- and 50-bit primes) run the
 // same passes on float64 words instead: exact products by the float64
@@ -226,7 +233,7 @@ __device__ __forceinline__ int swz(int col) { return col ^ ((col >> 4) & 15); }
 // One limb of a batched transform: word offset from the data base and
 // modulus index.  Either listed explicitly (rows of several digits of a
 // decomposition in one launch) or derived from (RowMap, batch stride).
-struct LimbRef { int64_t off; int mod; int pad; };  // pad: batch entry (RowMap path)
+struct LimbRef { int64_t off; int mod; int pad; };  // pad: batch entry (RowMap path); source limb past off (list)
 
 // ModDown epilogue of a forward transform (the transform of the extension of
 // [x]_P to Q): instead of the transform v, the row pass writes
@@ -267,9 +274,12 @@ struct NttArgs {
 
 // Limbs of one modulus are consecutive (row-major over the batch) so that
 // the workgroups in flight share few twiddle tables and those stay in L2.
+// The P rows (integer butterflies, twice the work of a float64 limb) come
+// first: a launch of a few waves per SIMD then does not end on them.
 __device__ __forceinline__ LimbRef limb_ref(const NttArgs& a, int y) {
   if (a.list) return a.list[y];
-  const int ri = y / a.batch, b = y - ri * a.batch, r = a.rm.row(ri);
+  const int ri = y / a.batch, b = y - ri * a.batch, np = a.rm.n - a.rm.split;
+  const int r = a.rm.row(ri < np ? a.rows - np + ri : ri - np);
   LimbRef l;
   l.off = (int64_t)b * (int64_t)a.bstride + ((int64_t)r << a.logN);
   l.mod = a.rm.mod(r);
@@ -308,11 +318,11 @@ __device__ __forceinline__ void ntt_col_int(const NttArgs& a, u64* sm, const Lim
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = in[(size_t)(j + P * i) * C];
     ntt_round<true, 4>(v, T1, q);
-    RoundTw<S - 4> T2;
-    round_tw_load<true, S - 4>(T2, (u64)(16 * j) << SB, SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) sm[(j + P * i) * nsub + c] = v[i];
     __syncthreads();
+    RoundTw<S - 4> T2;
+    round_tw_load<true, S - 4>(T2, (u64)(16 * j) << SB, SB, Nn, tw);
     // round 2: rows 16*j + i, the remaining S-4 stages
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = sm[(16 * j + i) * nsub + c];
@@ -326,11 +336,11 @@ __device__ __forceinline__ void ntt_col_int(const NttArgs& a, u64* sm, const Lim
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = poly[(size_t)(16 * j + i) * C];
     ntt_round<false, S - 4>(v, T1, q);
-    RoundTw<4> T2;
-    round_tw_load<false, 4>(T2, 0, S - 4 + SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) sm[(16 * j + i) * nsub + c] = v[i];
     __syncthreads();
+    RoundTw<4> T2;
+    round_tw_load<false, 4>(T2, 0, S - 4 + SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = sm[(j + P * i) * nsub + c];
     ntt_round<false, 4>(v, T2, q);
@@ -367,11 +377,11 @@ __device__ __forceinline__ void ntt_col_fp(const NttArgs& a, u64* sm, const Limb
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = f_in(in[(size_t)(j + P * i) * C]);
     f_round_fwd<4, 16, R1>(v, [&](int, int, int sl) { return T1.t[sl]; }, fc);
-    RoundTw<S - 4> T2;
-    round_tw_load<true, S - 4>(T2, (u64)(16 * j) << SB, SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) sm[(j + P * i) * nsub + c] = f_bits(v[i]);
     __syncthreads();
+    RoundTw<S - 4> T2;
+    round_tw_load<true, S - 4>(T2, (u64)(16 * j) << SB, SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = f_val(sm[(16 * j + i) * nsub + c]);
     f_round_fwd<S - 4, 16, R2>(v, [&](int, int, int sl) { return T2.t[sl]; }, fc);
@@ -385,11 +395,11 @@ __device__ __forceinline__ void ntt_col_fp(const NttArgs& a, u64* sm, const Limb
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = f_val(poly[(size_t)(16 * j + i) * C]);
     f_round_inv<S - 4, 16, B0, false>(v, [&](int, int, int sl) { return T1.t[sl]; }, fc);
-    RoundTw<4> T2;
-    round_tw_load<false, 4>(T2, 0, S - 4 + SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) sm[(16 * j + i) * nsub + c] = f_bits(v[i]);
     __syncthreads();
+    RoundTw<4> T2;
+    round_tw_load<false, 4>(T2, 0, S - 4 + SB, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = f_val(sm[(j + P * i) * nsub + c]);
     f_round_inv<4, 16, B1, true>(v, [&](int, int, int sl) { return T2.t[sl]; }, fc);
@@ -413,6 +423,7 @@ template <int S, bool EPI>
 __device__ __forceinline__ void row_fwd_tail(const NttArgs& a, const u64* srow, const LimbRef& lr, int r, int j, u64* poly) {
   constexpr int P = 1 << (S - 4);
   constexpr int C = 1 << S;
+  constexpr int EH = 8;  // words of the epilogue in flight a thread
   const int m = lr.mod;
   const u64 q = a.mods[m].q;
   if (EPI) {
@@ -424,48 +435,50 @@ __device__ __forceinline__ void row_fwd_tail(const NttArgs& a, const u64* srow, 
     const u64* ar = (a.e.add && b < a.e.add_batches) ? a.e.add + (size_t)b * a.e.a_bstride + rowoff : nullptr;
     u64* orow = (g ? a.e.out2 : a.e.out) + (size_t)part * a.e.o_bstride + ((size_t)row << a.logN);
     const u64 pi = a.e.pinv[m], pip = a.e.pinvp[m];
-    // every load of the epilogue is issued before the first use, so the
+    for (int i0 = 0; i0 < 16; i0 += EH) {
+    // the loads of EH words are issued before the first use, so that the
     // latencies overlap instead of adding up word by word
-    u64 xv[16], av[16];
-    uint32_t dst[16];
+    u64 xv[EH], av[EH];
+    uint32_t dst[EH];
 #pragma unroll
-    for (int i = 0; i < 16; i++) xv[i] = b < a.e.x_from ? 0 : __builtin_nontemporal_load(&xr[j + P * i]);
+    for (int i = 0; i < EH; i++) xv[i] = b < a.e.x_from ? 0 : __builtin_nontemporal_load(&xr[j + P * (i0 + i)]);
     if (ar) {
 #pragma unroll
-      for (int i = 0; i < 16; i++) av[i] = __builtin_nontemporal_load(&ar[j + P * i]);
+      for (int i = 0; i < EH; i++) av[i] = __builtin_nontemporal_load(&ar[j + P * (i0 + i)]);
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; i++) av[i] = 0;
+      for (int i = 0; i < EH; i++) av[i] = 0;
     }
     if (a.e.perm_inv) {
 #pragma unroll
-      for (int i = 0; i < 16; i++) dst[i] = a.e.perm_inv[r * C + j + P * i];
+      for (int i = 0; i < EH; i++) dst[i] = a.e.perm_inv[r * C + j + P * (i0 + i)];
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; i++) dst[i] = (uint32_t)(r * C + j + P * i);
+      for (int i = 0; i < EH; i++) dst[i] = (uint32_t)(r * C + j + P * (i0 + i));
     }
     if (a.e.acc) {
       // a sum of the result and acc: acc at the output position, gathered
       // through the same permutation as the stores
       const u64* crow = a.e.acc + (size_t)b * a.e.c_bstride + ((size_t)row << a.logN);
 #pragma unroll
-      for (int i = 0; i < 16; i++) av[i] = add_mod(av[i], crow[dst[i]], q);
+      for (int i = 0; i < EH; i++) av[i] = add_mod(av[i], crow[dst[i]], q);
     }
     if (a.e.ks) {
       const int R = a.e.ks_rows;
       const u64 kw = a.e.ks[(size_t)g * R + row], kwp = a.e.ks[(size_t)(2 + g) * R + row];
       const u64 cadd = part == 0 ? a.e.ks[(size_t)(4 + g) * R + row] : 0;
 #pragma unroll
-      for (int i = 0; i < 16; i++) {
+      for (int i = 0; i < EH; i++) {
         xv[i] = shoup_mul(xv[i], kw, kwp, q);
         av[i] = add_mod(av[i], cadd, q);
       }
     }
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int pos = j + P * i;
+    for (int i = 0; i < EH; i++) {
+      const int pos = j + P * (i0 + i);
       const u64 o = shoup_mul(sub_mod(xv[i], srow[swz(pos)], q), pi, pip, q);
       __builtin_nontemporal_store(add_mod(o, av[i], q), &orow[dst[i]]);
+    }
     }
   } else {
 #pragma unroll
@@ -522,17 +535,17 @@ __device__ __forceinline__ void ntt_row_int(const NttArgs& a, u64* sm, const Lim
     for (int i = 0; i < 16; i++) v[i] = __builtin_nontemporal_load(&in[j + P * i]);
 #pragma unroll
     for (int i = 0; i < 16; i++) srow[swz(j + P * i)] = v[i];
+    __syncthreads();
     RoundTw<S - 4> T1;
     round_tw_load_tab<S - 4>(T1, twr, P);
-    __syncthreads();
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = srow[swz(16 * j + i)];
     ntt_round<false, S - 4>(v, T1, q);
-    RoundTw<4> T2;
-    round_tw_load<false, 4>(T2, A, S - 4, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) srow[swz(16 * j + i)] = v[i];
     __syncthreads();
+    RoundTw<4> T2;
+    round_tw_load<false, 4>(T2, A, S - 4, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = srow[swz(j + P * i)];
     ntt_round<false, 4>(v, T2, q);
@@ -587,17 +600,17 @@ __device__ __forceinline__ void ntt_row_fp(const NttArgs& a, u64* sm, const Limb
     for (int i = 0; i < 16; i++) w[i] = __builtin_nontemporal_load(&in[j + P * i]);
 #pragma unroll
     for (int i = 0; i < 16; i++) srow[swz(j + P * i)] = w[i];
+    __syncthreads();
     RoundTw<S - 4> T1;
     round_tw_load_tab<S - 4>(T1, twr, P);
-    __syncthreads();
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = f_in(srow[swz(16 * j + i)]);
     f_round_inv<S - 4, 16, B0, false>(v, [&](int, int, int sl) { return T1.t[sl]; }, fc);
-    RoundTw<4> T2;
-    round_tw_load<false, 4>(T2, A, S - 4, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) srow[swz(16 * j + i)] = f_bits(v[i]);
     __syncthreads();
+    RoundTw<4> T2;
+    round_tw_load<false, 4>(T2, A, S - 4, Nn, tw);
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = f_val(srow[swz(j + P * i)]);
     f_round_inv<4, 16, B1, false>(v, [&](int, int, int sl) { return T2.t[sl]; }, fc);

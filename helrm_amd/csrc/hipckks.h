@@ -146,17 +146,21 @@ __device__ __forceinline__ void acc_mac_s(Acc128& A, u64 a, u64 b) {
 struct Acc61 { u64 s0, s1a, s1b, s2; uint32_t c0; };
 __device__ __forceinline__ void acc61_zero(Acc61& A) { A.s0 = A.s1a = A.s1b = A.s2 = 0; A.c0 = 0; }
 // the first product of an accumulator (and of its second middle half) sets
-// the columns instead of adding to zeros
-__device__ __forceinline__ void acc61_first_s(Acc61& A, u64 a, u64 b) {
+// the columns instead of adding to zeros; the accumulator starts from v * n,
+// v at most 8 and n < 2^61 (below 2^32 in the middle column, which four
+// products leave free)
+__device__ __forceinline__ void acc61_first_s(Acc61& A, uint32_t v, u64 n, u64 a, u64 b) {
   const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32), b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
-  u64 junk;
-  asm("v_mad_u64_u32 %[s0], %[j], %[b0], %[a0], 0\n\t"
-      "v_mad_u64_u32 %[s1], %[j], %[b1], %[a0], 0\n\t"
+  u64 junk, ca;
+  asm("v_mad_u64_u32 %[s0], %[j], %[n0], %[v], 0\n\t"
+      "v_mad_u64_u32 %[s1], %[j], %[n1], %[v], 0\n\t"
+      "v_mad_u64_u32 %[s0], %[ca], %[b0], %[a0], %[s0]\n\t"
+      "v_mad_u64_u32 %[s1], %[j], %[b1], %[a0], %[s1]\n\t"
       "v_mad_u64_u32 %[s1], %[j], %[b0], %[a1], %[s1]\n\t"
-      "v_mad_u64_u32 %[s2], %[j], %[b1], %[a1], 0"
-      : [s0] "=&v"(A.s0), [s1] "=&v"(A.s1a), [s2] "=&v"(A.s2), [j] "=&s"(junk)
-      : [a0] "v"(a0), [a1] "v"(a1), [b0] "s"(b0), [b1] "s"(b1));
-  A.c0 = 0;
+      "v_mad_u64_u32 %[s2], %[j], %[b1], %[a1], 0\n\t"
+      "v_cndmask_b32_e64 %[c0], 0, 1, %[ca]"
+      : [s0] "=&v"(A.s0), [s1] "=&v"(A.s1a), [s2] "=&v"(A.s2), [c0] "=&v"(A.c0), [ca] "=&s"(ca), [j] "=&s"(junk)
+      : [a0] "v"(a0), [a1] "v"(a1), [b0] "s"(b0), [b1] "s"(b1), [v] "v"(v), [n0] "s"((uint32_t)n), [n1] "s"((uint32_t)(n >> 32)));
 }
 __device__ __forceinline__ void acc61_first_half_s(Acc61& A, u64 a, u64 b) {
   const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32), b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
@@ -189,80 +193,69 @@ __device__ __forceinline__ void acc61_value(const Acc61& A, u64& lo, u64& hi) {
   lo = A.s0 + t;
   hi = A.s2 + A.c0 + (s1 >> 32) + (s1c << 32) + (lo < t ? 1 : 0);
 }
-// REDC(value of A) - sub mod q for an Acc61 whose value is below q * 2^64
-// (8 products of words below 2^61 and a column bound kept by the caller), sub
-// < q: the columns are combined, reduced and corrected in 32-bit carry
-// chains (about 33 VALU instructions where the 64-bit form takes ~47):
-//   s1 = s1a + s1b (carry s1c); lo = s0 + s1 * 2^32 (carry c1);
-//   hi = s2 + s1 / 2^32 + s1c * 2^32 + c0 + c1;
-//   m = lo * qinv mod 2^64 (qinv = -q^-1); t = hi + mulhi(m, q) + (lo != 0);
-//   r = t >= q ? t - q : t;  result = r - sub (+ q if it borrows).
-__device__ __forceinline__ u64 acc61_redc_sub(const Acc61& A, u64 q, u64 qinv, u64 sub) {
-  uint32_t lol, loh, hil, hih;
-  {
-    uint32_t s1l, s1h;
-    u64 k0, k1, k2, k3, s1c, c1;
-    asm("v_add_co_u32_e64 %[s1l], %[k0], %[al], %[bl]\n\t"
-        "v_addc_co_u32_e64 %[s1h], %[s1c], %[ah], %[bh], %[k0]\n\t"
-        "v_add_co_u32_e64 %[loh], %[c1], %[s0h], %[s1l]\n\t"
-        "v_add_co_u32_e64 %[hil], %[k1], %[s2l], %[s1h]\n\t"
-        "v_addc_co_u32_e64 %[hih], %[k1], %[s2h], 0, %[k1]\n\t"
-        "v_addc_co_u32_e64 %[hih], %[k1], %[hih], 0, %[s1c]\n\t"
-        "v_add_co_u32_e64 %[hil], %[k2], %[hil], %[c0]\n\t"
-        "v_addc_co_u32_e64 %[hih], %[k2], %[hih], 0, %[k2]\n\t"
-        "v_addc_co_u32_e64 %[hil], %[k3], %[hil], 0, %[c1]\n\t"
-        "v_addc_co_u32_e64 %[hih], %[k3], %[hih], 0, %[k3]"
-        : [s1l] "=&v"(s1l), [s1h] "=&v"(s1h), [loh] "=&v"(loh), [hil] "=&v"(hil), [hih] "=&v"(hih),
-          [k0] "=&s"(k0), [k1] "=&s"(k1), [k2] "=&s"(k2), [k3] "=&s"(k3), [s1c] "=&s"(s1c), [c1] "=&s"(c1)
-        : [al] "v"((uint32_t)A.s1a), [ah] "v"((uint32_t)(A.s1a >> 32)), [bl] "v"((uint32_t)A.s1b),
-          [bh] "v"((uint32_t)(A.s1b >> 32)), [s0h] "v"((uint32_t)(A.s0 >> 32)), [s2l] "v"((uint32_t)A.s2),
-          [s2h] "v"((uint32_t)(A.s2 >> 32)), [c0] "v"(A.c0));
-    lol = (uint32_t)A.s0;
-  }
-  const u64 lo = ((u64)loh << 32) | lol;
-  // m = lo * qinv mod 2^64
-  const uint32_t ql = (uint32_t)q, qh = (uint32_t)(q >> 32), il = (uint32_t)qinv, ih = (uint32_t)(qinv >> 32);
-  const u64 p0 = (u64)lol * il;
-  const uint32_t mh = (uint32_t)(p0 >> 32) + lol * ih + loh * il;
-  const u64 m = ((u64)mh << 32) | (uint32_t)p0;
-  const u64 mq = mulhi64(m, q);
-  uint32_t tl, th, rl, rh, dl, dh;
-  u64 cz, k4, b0, b1;
-  // t = hi + mq + (lo != 0); r = t - q unless that borrows; d = r - sub, + q if that borrows
-  asm("v_cmp_ne_u64_e64 %[cz], 0, %[lo]\n\t"
-      "v_addc_co_u32_e64 %[tl], %[k4], %[hil], %[mql], %[cz]\n\t"
-      "v_addc_co_u32_e64 %[th], %[k4], %[hih], %[mqh], %[k4]\n\t"
-      "v_sub_co_u32_e64 %[rl], %[b0], %[tl], %[ql]\n\t"
-      "v_subb_co_u32_e64 %[rh], %[b0], %[th], %[qh], %[b0]\n\t"
-      "v_cndmask_b32_e64 %[rl], %[rl], %[tl], %[b0]\n\t"
-      "v_cndmask_b32_e64 %[rh], %[rh], %[th], %[b0]\n\t"
-      "v_sub_co_u32_e64 %[dl], %[b1], %[rl], %[sl]\n\t"
-      "v_subb_co_u32_e64 %[dh], %[b1], %[rh], %[sh], %[b1]\n\t"
-      "v_cndmask_b32_e64 %[tl], 0, %[ql], %[b1]\n\t"
-      "v_cndmask_b32_e64 %[th], 0, %[qh], %[b1]\n\t"
-      "v_add_co_u32_e64 %[dl], %[k4], %[dl], %[tl]\n\t"
-      "v_addc_co_u32_e64 %[dh], %[k4], %[dh], %[th], %[k4]"
-      : [tl] "=&v"(tl), [th] "=&v"(th), [rl] "=&v"(rl), [rh] "=&v"(rh), [dl] "=&v"(dl), [dh] "=&v"(dh),
-        [cz] "=&s"(cz), [k4] "=&s"(k4), [b0] "=&s"(b0), [b1] "=&s"(b1)
-      : [lo] "v"(lo), [hil] "v"(hil), [hih] "v"(hih), [mql] "v"((uint32_t)mq), [mqh] "v"((uint32_t)(mq >> 32)),
-        [ql] "v"(ql), [qh] "v"(qh), [sl] "v"((uint32_t)sub), [sh] "v"((uint32_t)(sub >> 32)));
-  return ((u64)dh << 32) | dl;
+// REDC(value of A) for an Acc61 whose value is below q * 2^64, a 32-bit word
+// at a time on the columns as they are (21 VALU instructions; recombining the
+// 128-bit value first takes 33):
+//   m0 = s0 * qinv mod 2^32;  s1 = s1a + s1b + m0 q1 + (s0 + m0 q0) / 2^32
+//   m1 = s1 * qinv mod 2^32;  r  = s2 + m1 q1 + (s1 + m1 q0) / 2^32
+// with the carries out of s0 counted into s1's high word and those out of s1
+// (kb, k1, kd, k3) into r's; r < 2q, then r >= q ? r - q : r.
+__device__ __forceinline__ u64 acc61_redc(const Acc61& A, u64 q, u64 qinv) {
+  const uint32_t q0 = (uint32_t)q, q1 = (uint32_t)(q >> 32), qi = (uint32_t)qinv;
+  uint32_t m0, s1l, s1h, c0;
+  u64 t, k0, kb, kc;
+  asm("v_mul_lo_u32 %[m0], %[s0l], %[qi]\n\t"
+      "v_add_co_u32_e64 %[s1l], %[kc], %[al], %[bl]\n\t"
+      "v_mad_u64_u32 %[t], %[k0], %[m0], %[q0], %[s0]\n\t"
+      "v_addc_co_u32_e64 %[s1h], %[kb], %[ah], %[bh], %[kc]\n\t"
+      "v_addc_co_u32_e64 %[c0], %[kc], 0, %[c0i], %[k0]"
+      : [m0] "=&v"(m0), [t] "=&v"(t), [s1l] "=&v"(s1l), [s1h] "=&v"(s1h), [c0] "=&v"(c0), [k0] "=&s"(k0), [kb] "=&s"(kb),
+        [kc] "=&s"(kc)
+      : [s0l] "v"((uint32_t)A.s0), [s0] "v"(A.s0), [c0i] "v"(A.c0), [al] "v"((uint32_t)A.s1a), [ah] "v"((uint32_t)(A.s1a >> 32)),
+        [bl] "v"((uint32_t)A.s1b), [bh] "v"((uint32_t)(A.s1b >> 32)), [qi] "s"(qi), [q0] "s"(q0));
+  u64 s1 = ((u64)s1h << 32) | s1l, k1, kd;
+  asm("v_mad_u64_u32 %[s1], %[k1], %[m0], %[q1], %[s1]" : [s1] "+v"(s1), [k1] "=&s"(k1) : [m0] "v"(m0), [q1] "s"(q1));
+  asm("v_add_co_u32_e64 %[s1l], %[kc], %[il], %[th]\n\t"
+      "v_addc_co_u32_e64 %[s1h], %[kd], %[ih], %[c0], %[kc]"
+      : [s1l] "=&v"(s1l), [s1h] "=&v"(s1h), [kc] "=&s"(kc), [kd] "=&s"(kd)
+      : [il] "v"((uint32_t)s1), [ih] "v"((uint32_t)(s1 >> 32)), [th] "v"((uint32_t)(t >> 32)), [c0] "v"(c0));
+  s1 = ((u64)s1h << 32) | s1l;
+  uint32_t m1;
+  u64 r = A.s2, k3, junk;
+  asm("v_mul_lo_u32 %[m1], %[s1l], %[qi]\n\t"
+      "v_mad_u64_u32 %[t], %[k3], %[m1], %[q0], %[s1]\n\t"
+      "v_mad_u64_u32 %[r], %[j], %[m1], %[q1], %[r]"
+      : [m1] "=&v"(m1), [t] "=&v"(t), [r] "+v"(r), [k3] "=&s"(k3), [j] "=&s"(junk)
+      : [s1l] "v"(s1l), [s1] "v"(s1), [qi] "s"(qi), [q0] "s"(q0), [q1] "s"(q1));
+  uint32_t rl, rh;
+  asm("v_add_co_u32_e64 %[rl], %[j], %[il], %[th]\n\t"
+      "v_addc_co_u32_e64 %[rh], %[j], %[ih], 0, %[j]\n\t"
+      "v_addc_co_u32_e64 %[rh], %[j], %[rh], 0, %[kb]\n\t"
+      "v_addc_co_u32_e64 %[rh], %[j], %[rh], 0, %[k1]\n\t"
+      "v_addc_co_u32_e64 %[rh], %[j], %[rh], 0, %[kd]\n\t"
+      "v_addc_co_u32_e64 %[rh], %[j], %[rh], 0, %[k3]"
+      : [rl] "=&v"(rl), [rh] "=&v"(rh), [j] "=&s"(junk)
+      : [il] "v"((uint32_t)r), [ih] "v"((uint32_t)(r >> 32)), [th] "v"((uint32_t)(t >> 32)), [kb] "s"(kb), [k1] "s"(k1),
+        [kd] "s"(kd), [k3] "s"(k3));
+  return csub_b(((u64)rh << 32) | rl, q);
 }
 // One destination word of a basis extension from at most 8 sources:
-// REDC(sum_i y(i) * h[i]) - sub mod q, y(i) < 2^61 (zero past the job's
-// sources) and h[i] < q the row's table words (Montgomery form, read for all
-// 8 i: the table holds spare words past its last row).
+// REDC(sum_i y(i) * h[i] + v * n), y(i) < 2^61 (zero past the job's sources),
+// h[i] < q the row's table words and n < q that of -S (Montgomery form, h
+// read for all 8 i: the table holds spare words past its last row), v <= 8
+// the overflow count: the sum is at most (2^64 - 8)(q - 1) + 8 (q - 1), so
+// below q * 2^64 as the REDC needs.
 template <class Y>
-__device__ __forceinline__ u64 bconv_word8(Y y, const u64* __restrict__ h, u64 q, u64 qinv, u64 sub) {
+__device__ __forceinline__ u64 bconv_word8(Y y, const u64* __restrict__ h, uint32_t v, u64 n, u64 q, u64 qinv) {
   Acc61 A;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    if (i == 0) acc61_first_s(A, y(i), h[i]);
+    if (i == 0) acc61_first_s(A, v, n, y(i), h[i]);
     else if (i < 4) acc61_mac_s<0>(A, y(i), h[i]);
     else if (i == 4) acc61_first_half_s(A, y(i), h[i]);
     else acc61_mac_s<1>(A, y(i), h[i]);
   }
-  return acc61_redc_sub(A, q, qinv, sub);
+  return acc61_redc(A, q, qinv);
 }
 // the 128-bit value (lo, hi) of an accumulator
 __device__ __forceinline__ void acc_value(const Acc128& A, u64& lo, u64& hi) {

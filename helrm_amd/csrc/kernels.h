@@ -33,7 +33,7 @@ struct BConvSrc {
 struct BConvTable {
   BConvSrc src[HCK_MAXSRC];
   const u64* hat;  // [nmod][ns]   (S/s_i mod t) * R mod t  (Montgomery form)
-  const u64* vS;   // [nmod][ns+1] v*S mod t
+  const u64* nS;   // [nmod]       (-S mod t) * R mod t
   int rows_per_block;
 };
 
@@ -106,7 +106,7 @@ struct LinkArgs {
 };
 // LDS bytes of a link launch; at most LINK_LDS_MAX (K <= 8, dn <= HCK_MAXDIG) can be launched
 #define LINK_LDS_MAX 65536
-size_t link_lds_bytes(int l, int K, int dn);
+size_t link_lds_bytes(int l);
 void launch_link(const LinkArgs& a, int batch, hipStream_t st);
 
 struct GiantAccArgs {

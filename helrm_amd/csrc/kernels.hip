@@ -243,19 +243,6 @@ __global__ __launch_bounds__(256) void bconv_kernel(const u64* __restrict__ in, 
   // every source word in flight at once (rows past ns re-read row 0, unused)
 #pragma unroll
   for (int i = 0; i < MAXS; i++) y[i] = inb[(size_t)(i < ns ? i : 0) * N + x];
-  // v*S mod t of this workgroup's destination rows for every v = 0..ns,
-  // staged in LDS once: read per lane from memory inside the row loop it
-  // would put an L2 round trip on every destination row
-  __shared__ u64 svs[HCK_MAXMOD * (MAXS + 1)];
-  {
-    const u64* __restrict__ vS = tab->vS;
-    const int w = ns + 1, n = (r1 - r0) * w;
-    for (int e = threadIdx.x; e < n; e += blockDim.x) {
-      const int rr = e / w;
-      svs[e] = vS[(size_t)rm.mod(rm.row(r0 + rr)) * w + (e - rr * w)];
-    }
-  }
-  __syncthreads();
   // the source constants are read without a branch per source (entries past
   // ns are zero and their terms are selected away), so that their scalar
   // loads are issued together instead of one round trip per source
@@ -268,8 +255,9 @@ __global__ __launch_bounds__(256) void bconv_kernel(const u64* __restrict__ in, 
     y[i] = act ? yi : 0;
     vf += act ? t : 0.0;
   }
-  const int v = J.force_v0 ? 0 : (int)(u64)vf;
+  const uint32_t v = J.force_v0 ? 0 : (uint32_t)(u64)vf;
   const u64* __restrict__ hat = tab->hat;
+  const u64* __restrict__ nS = tab->nS;
   for (int r = r0; r < r1; r++) {
     const int row = rm.row(r);
     const int m = rm.mod(row);
@@ -278,9 +266,7 @@ __global__ __launch_bounds__(256) void bconv_kernel(const u64* __restrict__ in, 
     // exact column sums of 16 products (words < 2^62), folded below q
     u64 res;
     if (MAXS <= 8) {
-      // y[i] < q_i < 2^61 and h[i] < q < 2^61: 8 products sum below 2^64 q,
-      // so hi < q as the REDC needs (y[i] = 0 past ns)
-      res = bconv_word8([&](int i) { return y[i]; }, h, mc.q, mc.qinv, svs[(r - r0) * (ns + 1) + v]);
+      res = bconv_word8([&](int i) { return y[i]; }, h, v, nS[m], mc.q, mc.qinv);
     } else {
       u128 acc = 0;
 #pragma unroll
@@ -290,12 +276,12 @@ __global__ __launch_bounds__(256) void bconv_kernel(const u64* __restrict__ in, 
 #pragma unroll
         for (int i = i0; i < i0 + 16 && i < MAXS; i++)
           if (i < ns) acc_mac_s(A, y[i], h[i]);
+        if (i0 == 0) acc_mac_s(A, v, nS[m]);  // v < 2^6: nothing in the top column
         u64 lo, hi;
         acc_value(A, lo, hi);
         acc += ((u128)fold_hi4(hi, mc.q) << 64) | lo;
       }
       res = redc((u64)acc, fold_hi4((u64)(acc >> 64), mc.q), mc.q, mc.qinv);
-      res = sub_mod(res, svs[(r - r0) * (ns + 1) + v], mc.q);
     }
     outb[(size_t)row * N + x] = res;
   }
@@ -332,7 +318,6 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
   const bool flip = ((uint32_t)x * jobs.ginv & (uint32_t)(2 * N - 1)) >= (uint32_t)N;  // never with ginv = 0
   __shared__ u64 sy[MAXS][BCL_X];
   __shared__ double st[MAXS][BCL_X];
-  __shared__ u64 svs[HCK_MAXMOD * (MAXS + 1)];
   // sources w and w + 4 of this coefficient
 #pragma unroll
   for (int k = 0; k < 2; k++) {
@@ -346,14 +331,6 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
     sy[i][lane] = act ? yi : 0;
     st[i][lane] = act ? t : 0.0;
   }
-  {
-    const u64* __restrict__ vS = tab->vS;
-    const int wd = ns + 1, n = nrows * wd;
-    for (int e = threadIdx.x; e < n; e += blockDim.x) {
-      const int rr = e / wd;
-      svs[e] = vS[(size_t)rm.mod(rm.row(rr)) * wd + (e - rr * wd)];
-    }
-  }
   __syncthreads();
   u64 y[MAXS];
   double vf = 0.0;
@@ -362,14 +339,15 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
     y[i] = sy[i][lane];
     vf += st[i][lane];
   }
-  const int v = J.force_v0 ? 0 : (int)(u64)vf;
+  const uint32_t v = J.force_v0 ? 0 : (uint32_t)(u64)vf;
   const u64* __restrict__ hat = tab->hat;
+  const u64* __restrict__ nS = tab->nS;
   for (int r = w; r < nrows; r += 4) {
     const int row = rm.row(r);
     const int m = rm.mod(row);
     const ModC mc = mods[m];
     const u64* __restrict__ h = hat + (size_t)m * ns;
-    const u64 e = bconv_word8([&](int i) { return y[i]; }, h, mc.q, mc.qinv, svs[r * (ns + 1) + v]);
+    const u64 e = bconv_word8([&](int i) { return y[i]; }, h, v, nS[m], mc.q, mc.qinv);
     outb[(size_t)row * N + x] = flip && e ? mc.q - e : e;
   }
 }
@@ -398,9 +376,7 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   const bool two = a.x0p != nullptr;
   const bool flip = ((uint32_t)x * a.ginv & (uint32_t)(2 * N - 1)) >= (uint32_t)N;
   // LDS: source terms (P rows: y and y / p of both polynomials, 8 slots each;
-  // then the Q rows' y and y / q), then v * S mod t of every extended row
-  u64* U = sm;
-  u64* svs = sm + max(4 * 8, 2 * nq) * BCL_X;
+  // then the Q rows' y and y / q)
   const BConvTable* __restrict__ pt = a.ptab;
   for (int part = two ? 0 : 1; part < 2; part++) {
     const u64* src = part ? x1 + (size_t)nq * N : a.x0p + x;
@@ -412,61 +388,49 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
       u64 yi = shoup_mul(src[(size_t)(act ? i : 0) * N], s.hinv, s.hinvp, s.q);
       if (flip && yi) yi = s.q - yi;
       const double t = (double)yi / s.qd;
-      U[(part * 16 + i) * BCL_X + lane] = act ? yi : 0;
-      U[(part * 16 + 8 + i) * BCL_X + lane] = act ? (u64)__double_as_longlong(t) : 0;
+      sm[(part * 16 + i) * BCL_X + lane] = act ? yi : 0;
+      sm[(part * 16 + 8 + i) * BCL_X + lane] = act ? (u64)__double_as_longlong(t) : 0;
     }
-  }
-  for (int e = threadIdx.x; e < nq * (K + 1); e += blockDim.x) svs[e] = pt->vS[e];  // Q row r is modulus r
-  u64* svd = svs + nq * (K + 1);
-  for (int d = 0; d < a.dn; d++) {
-    const int st0 = d * K, ns = min(st0 + K, nq) - st0, wd = ns + 1, n = (nqp - ns) * wd;
-    const u64* __restrict__ vS = a.dtab[d]->vS;
-    for (int e = threadIdx.x; e < n; e += blockDim.x) {
-      const int rr = e / wd, row = rr < st0 ? rr : rr + ns;
-      svd[e] = vS[(size_t)(row < nq ? row : a.L + row - nq) * wd + (e - rr * wd)];
-    }
-    svd += n;
   }
   __syncthreads();
   u64 y0[8], y1[8];
   double v0f = 0.0, v1f = 0.0;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    y1[i] = U[(16 + i) * BCL_X + lane];
-    v1f += __longlong_as_double((long long)U[(24 + i) * BCL_X + lane]);
+    y1[i] = sm[(16 + i) * BCL_X + lane];
+    v1f += __longlong_as_double((long long)sm[(24 + i) * BCL_X + lane]);
     if (two) {
-      y0[i] = U[i * BCL_X + lane];
-      v0f += __longlong_as_double((long long)U[(8 + i) * BCL_X + lane]);
+      y0[i] = sm[i * BCL_X + lane];
+      v0f += __longlong_as_double((long long)sm[(8 + i) * BCL_X + lane]);
     }
   }
-  const int v1 = (int)(u64)v1f, v0 = (int)(u64)v0f;
+  const uint32_t v1 = (uint32_t)(u64)v1f, v0 = (uint32_t)(u64)v0f;
   __syncthreads();
   // a row's words are loaded while the row before it is computed
   u64 zn = w < nq ? x1[(size_t)w * N] : 0, cn = a.acc && w < nq ? c1[(size_t)w * N] : 0;
   for (int r = w; r < nq; r += 4) {
     const ModC mc = a.mods[r];
     const u64* __restrict__ h = pt->hat + (size_t)r * K;
-    const u64 pi = a.pinv[r], pip = a.pinvp[r];
+    const u64 pi = a.pinv[r], pip = a.pinvp[r], n = pt->nS[r];
     const u64 z = zn, c = cn;
     const int rn = min(r + 4, nq - 1);
     zn = x1[(size_t)rn * N];
     if (a.acc) cn = c1[(size_t)rn * N];
-    const u64 e1 = bconv_word8([&](int i) { return y1[i]; }, h, mc.q, mc.qinv, svs[r * (K + 1) + v1]);
+    const u64 e1 = bconv_word8([&](int i) { return y1[i]; }, h, v1, n, mc.q, mc.qinv);
     const u64 m = shoup_mul(flip ? add_mod(z, e1, mc.q) : sub_mod(z, e1, mc.q), pi, pip, mc.q);
     const u64 s = add_mod(c, m, mc.q);
     c1[(size_t)r * N] = s;
     const BConvSrc sd = a.dtab[r / K]->src[r % K];
     const u64 yi = shoup_mul(s, sd.hinv, sd.hinvp, sd.q);
-    U[r * BCL_X + lane] = yi;
-    U[(nq + r) * BCL_X + lane] = (u64)__double_as_longlong((double)yi / sd.qd);
+    sm[r * BCL_X + lane] = yi;
+    sm[(nq + r) * BCL_X + lane] = (u64)__double_as_longlong((double)yi / sd.qd);
     if (two) {
-      u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, mc.q, mc.qinv, svs[r * (K + 1) + v0]);
+      u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, v0, n, mc.q, mc.qinv);
       e0 = shoup_mul(e0, pi, pip, mc.q);
       a.e0[(size_t)r * N + x] = flip || e0 == 0 ? e0 : mc.q - e0;
     }
   }
   __syncthreads();
-  svd = svs + nq * (K + 1);
   int first = w;  // this wave's first row of the digit: rows are dealt round robin over all digits
   for (int d = 0; d < a.dn; d++) {
     const int st0 = d * K, ns = min(st0 + K, nq) - st0, nrows = nqp - ns;
@@ -476,12 +440,12 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
 #pragma unroll
     for (int i = 0; i < 8; i++) {
       const int r = st0 + (i < ns ? i : 0);
-      const u64 yi = U[r * BCL_X + lane];
-      const double t = __longlong_as_double((long long)U[(nq + r) * BCL_X + lane]);
+      const u64 yi = sm[r * BCL_X + lane];
+      const double t = __longlong_as_double((long long)sm[(nq + r) * BCL_X + lane]);
       y[i] = i < ns ? yi : 0;
       vf += i < ns ? t : 0.0;
     }
-    const int v = ns == 1 ? 0 : (int)(u64)vf;  // a digit of one modulus is spread without an overflow count
+    const uint32_t v = ns == 1 ? 0 : (uint32_t)(u64)vf;  // a digit of one modulus is spread without an overflow count
     int rr = first;
     for (; rr < nrows; rr += 4) {
       const int row = rr < st0 ? rr : rr + ns;
@@ -489,23 +453,14 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
       const ModC mc = a.mods[m];
       const u64* __restrict__ h = dt->hat + (size_t)m * ns;
       digits[((size_t)d * nqp + row) * N] =
-          bconv_word8([&](int i) { return y[i]; }, h, mc.q, mc.qinv, svd[rr * (ns + 1) + v]);
+          bconv_word8([&](int i) { return y[i]; }, h, v, dt->nS[m], mc.q, mc.qinv);
     }
     first = rr - nrows;
-    svd += nrows * (ns + 1);
   }
 }
-size_t link_lds_bytes(int l, int K, int dn) {
-  const int nq = l + 1, nqp = nq + K;
-  size_t words = (size_t)std::max(4 * 8, 2 * nq) * BCL_X + (size_t)nq * (K + 1);
-  for (int d = 0; d < dn; d++) {
-    const int ns = std::min(d * K + K, nq) - d * K;
-    words += (size_t)(nqp - ns) * (ns + 1);
-  }
-  return words * 8;
-}
+size_t link_lds_bytes(int l) { return (size_t)std::max(4 * 8, 2 * (l + 1)) * BCL_X * 8; }
 void launch_link(const LinkArgs& a, int batch, hipStream_t st) {
-  hipLaunchKernelGGL(link_kernel, dim3(a.N / BCL_X, batch), dim3(256), link_lds_bytes(a.l, a.K, a.dn), st, a);
+  hipLaunchKernelGGL(link_kernel, dim3(a.N / BCL_X, batch), dim3(256), link_lds_bytes(a.l), st, a);
 }
 void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, size_t out_bstride, int batch,
                   const ModC* mods, int N, hipStream_t st) {

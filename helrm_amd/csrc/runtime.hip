@@ -330,7 +330,7 @@ struct LinTrans {
   bool ptrs_ready = false;
 };
 
-struct BConvHost { int ns; BConvTable tab; DU64 hat, vS; DevArray<BConvTable> dtab; };
+struct BConvHost { int ns; BConvTable tab; DU64 hat, nS; DevArray<BConvTable> dtab; };
 
 struct Timing { bool on = false; std::map<std::string, std::vector<std::pair<hipEvent_t, hipEvent_t>>> ev; std::map<std::string, std::pair<long, double>> acc; };
 
@@ -456,7 +456,7 @@ BConvHost& bconv_table(int s0, int s1) {
   REQUIRE(ns >= 1 && ns <= HCK_MAXSRC, "basis conversion source too large");
   auto b = std::make_unique<BConvHost>();
   b->ns = ns;
-  std::vector<u64> hat((size_t)nm * ns), vS((size_t)nm * (ns + 1));
+  std::vector<u64> hat((size_t)nm * ns), nS(nm);
   for (int i = 0; i < ns; i++) {
     u64 si = s.mod[s0 + i], pr = 1;
     for (int j = 0; j < ns; j++) if (j != i) pr = mulmod(pr, s.mod[s0 + j] % si, si);
@@ -466,7 +466,7 @@ BConvHost& bconv_table(int s0, int s1) {
   for (int m = 0; m < nm; m++) {
     u64 t = s.mod[m], R = s.hmods[m].rmod, Sm = 1;
     for (int j = 0; j < ns; j++) Sm = mulmod(Sm, s.mod[s0 + j] % t, t);
-    for (int v = 0; v <= ns; v++) vS[(size_t)m * (ns + 1) + v] = mulmod((u64)v, Sm, t);
+    nS[m] = mulmod(Sm ? t - Sm : 0, R, t);
     for (int i = 0; i < ns; i++) {
       u64 pr = 1;
       for (int j = 0; j < ns; j++) if (j != i) pr = mulmod(pr, s.mod[s0 + j] % t, t);
@@ -475,8 +475,8 @@ BConvHost& bconv_table(int s0, int s1) {
   }
   hat.resize(hat.size() + 8, 0);  // spare words: the 8-source kernel reads h[ns..7] (times zero) past the last row
   b->hat = DU64(hat.size()); upload(b->hat.p, hat.data(), hat.size());
-  b->vS = DU64(vS.size()); upload(b->vS.p, vS.data(), vS.size());
-  b->tab.hat = b->hat.p; b->tab.vS = b->vS.p; b->tab.rows_per_block = 8;
+  b->nS = DU64(nS.size()); upload(b->nS.p, nS.data(), nS.size());
+  b->tab.hat = b->hat.p; b->tab.nS = b->nS.p; b->tab.rows_per_block = 8;
   b->dtab = DevArray<BConvTable>(1); upload(b->dtab.p, &b->tab, 1);
   auto& ref = *b;
   s.bconv[key] = std::move(b);
@@ -1276,7 +1276,7 @@ void fold_rotations(Cipher& ct, const std::vector<u64>& ge) {
 bool fold_chains(int l, size_t steps) {
   Scheme& s = sch();
   const int dn = (l + 1 + s.K - 1) / s.K;
-  return steps >= 2 && s.K <= 8 && dn <= HCK_KM1_DIG && link_lds_bytes(l, s.K, dn) <= LINK_LDS_MAX;
+  return steps >= 2 && s.K <= 8 && dn <= HCK_KM1_DIG && link_lds_bytes(l) <= LINK_LDS_MAX;
 }
 // ---- plaintext, scalar and ciphertext products (Lattigo ckks Evaluator
 // Mul / Add with a constant / MulRelin, restated for the GPU) ----

@@ -11,59 +11,131 @@
 // The forward NTT and the Montgomery conversion that follow are the library's
 // own kernels.
 //
-// Every floating-point operation is the one of the host restatement, in the
+// Decoding goes the other way: the centred CRT of each coefficient in multiword
+// integers, the nearest double of it over the scale, and the special FFT.
+//
+// Every floating-point operation is the one of the scalar restatement, in the
 // same order, with contraction into fused multiply-adds switched off, so the
-// coefficients are bit-identical to a scalar float64 evaluation of the
-// algorithm.  One thread per butterfly and one launch per FFT stage: encoding
-// is set-up work (diagonals are encoded once per compiled layer) and a stage
-// launch over a batch of plaintexts streams at HBM rate.
+// coefficients and the decoded values are bit-identical to a scalar float64
+// evaluation of the algorithm.  The FFT's log2(slots) stages run in two
+// launches through LDS: the stages inside aligned blocks of 256 values, and
+// those across blocks on 8 columns of the (slots / 256) x 256 view.  At 2^15
+// slots a launch a stage took 15 dependent launches for 512 KB of data.
 #include "hipckks.h"
 #include "kernels.h"
 
 namespace {
 
-// plaintext p, element k: data[src * slots + ((k + rot) mod slots)], or 0 past
-// nvals; complex input: (re, im) pairs at data[2k], data[2k + 1]
-__global__ void encode_load_kernel(double* __restrict__ re, double* __restrict__ im, size_t pstride,
-                                   const float* __restrict__ data, const EncodeSrc* __restrict__ src, int n, int nvals,
-                                   int complex_in) {
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  const int p = blockIdx.y;
-  if (k >= n) return;
-  const EncodeSrc e = src[p];
-  double v = 0.0, vi = 0.0;
-  if (k < nvals) {
-    if (complex_in) {
-      v = (double)data[2 * (size_t)k];
-      vi = (double)data[2 * (size_t)k + 1];
-    } else {
-      v = (double)data[(size_t)e.src * n + ((k + e.rot) & (n - 1))];
-    }
+constexpr int FFT_B = 256;   // values of a block (the stages len <= FFT_B)
+constexpr int FFT_CW = 8;    // columns of a workgroup of the stages above: 64-byte rows, n / 256 <= 128 rows in 16 KB
+struct FftArgs {
+  double *re, *im;
+  size_t pstride;
+  int n, M;
+  const int* rotgroup;
+  const double *rre, *rim;
+  // inverse: the column pass reads element k of plaintext p from
+  // data[src * n + ((k + rot) mod n)], or 0 past nvals; complex input: (re, im)
+  // pairs at data[2k], data[2k + 1]
+  const float* data;
+  const EncodeSrc* src;
+  int nvals, complex_in;
+  // forward: the column pass writes the real parts as float (mode 0) or double
+  // (1), or (re, im) pairs of float (2)
+  void* out;
+  int mode;
+};
+
+// one butterfly of stage len, root j: forward (u, v) -> (u + w v, u - w v),
+// inverse (u, v) -> (u + v, (u - v) conj(w))
+template <bool INV>
+__device__ __forceinline__ void fft_butterfly(const FftArgs& a, int len, int j, double& ur, double& ui, double& vr, double& vi) {
+#pragma clang fp contract(off)
+  const int lenq = len << 2, gap = a.M / lenq, r = a.rotgroup[j] & (lenq - 1);
+  const int idx = (INV ? lenq - r : r) * gap;
+  const double wr = a.rre[idx], wi = a.rim[idx];
+  if (INV) {
+    const double dr = ur - vr, di = ui - vi;
+    ur = ur + vr;
+    ui = ui + vi;
+    vr = dr * wr - di * wi;
+    vi = dr * wi + di * wr;
+  } else {
+    const double tr = vr * wr - vi * wi, ti = vr * wi + vi * wr;
+    vr = ur - tr;
+    vi = ui - ti;
+    ur = ur + tr;
+    ui = ui + ti;
   }
-  re[(size_t)p * pstride + k] = v;
-  im[(size_t)p * pstride + k] = vi;
 }
 
-// one DIF stage of the special inverse FFT: blocks of len, pairs (k, k + len/2)
-__global__ void special_ifft_stage_kernel(double* __restrict__ re, double* __restrict__ im, size_t pstride, int n, int len,
-                                          int M, const int* __restrict__ rotgroup, const double* __restrict__ rre,
-                                          const double* __restrict__ rim) {
-#pragma clang fp contract(off)
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (n >> 1)) return;
-  double* R = re + (size_t)blockIdx.y * pstride;
-  double* I = im + (size_t)blockIdx.y * pstride;
-  const int lenh = len >> 1, lenq = len << 2, gap = M / lenq, mask = lenq - 1;
-  const int j = t % lenh;
-  const int k = (t / lenh) * len + j;
-  const double ur = R[k], ui = I[k], vr = R[k + lenh], vi = I[k + lenh];
-  const int idx = (lenq - (rotgroup[j] & mask)) * gap;
-  const double wr = rre[idx], wi = rim[idx];
-  const double dr = ur - vr, di = ui - vi;
-  R[k] = ur + vr;
-  I[k] = ui + vi;
-  R[k + lenh] = dr * wr - di * wi;
-  I[k + lenh] = dr * wi + di * wr;
+// stages len <= FFT_B of one block: 128 threads, a butterfly each per stage
+template <bool INV>
+__global__ __launch_bounds__(FFT_B / 2) void fft_block_kernel(FftArgs a) {
+  __shared__ double sr[FFT_B], si[FFT_B];
+  const int t = threadIdx.x, base = blockIdx.x * FFT_B;
+  double* R = a.re + (size_t)blockIdx.y * a.pstride + base;
+  double* I = a.im + (size_t)blockIdx.y * a.pstride + base;
+  for (int k = t; k < FFT_B; k += FFT_B / 2) { sr[k] = R[k]; si[k] = I[k]; }
+  for (int len = INV ? FFT_B : 2; INV ? len >= 2 : len <= FFT_B; len = INV ? len >> 1 : len << 1) {
+    __syncthreads();
+    const int lenh = len >> 1, j = t & (lenh - 1), k = 2 * (t - j) + j;
+    fft_butterfly<INV>(a, len, j, sr[k], si[k], sr[k + lenh], si[k + lenh]);
+  }
+  __syncthreads();
+  for (int k = t; k < FFT_B; k += FFT_B / 2) { R[k] = sr[k]; I[k] = si[k]; }
+}
+
+// stages len > FFT_B: FFT_CW columns of the (n / FFT_B) x FFT_B view
+template <bool INV>
+__global__ __launch_bounds__(256) void fft_col_kernel(FftArgs a) {
+  constexpr int MAXE = 128 * FFT_CW;
+  __shared__ double sr[MAXE], si[MAXE];
+  const int rows = a.n / FFT_B, E = rows * FFT_CW, col0 = blockIdx.x * FFT_CW;
+  double* R = a.re + (size_t)blockIdx.y * a.pstride;
+  double* I = a.im + (size_t)blockIdx.y * a.pstride;
+  for (int e = threadIdx.x; e < E; e += 256) {
+    const int k = (e / FFT_CW) * FFT_B + col0 + e % FFT_CW;
+    double v = 0.0, vi = 0.0;
+    if (!INV) {
+      v = R[k];
+      vi = I[k];
+    } else if (k < a.nvals) {
+      if (a.complex_in) {
+        v = (double)a.data[2 * (size_t)k];
+        vi = (double)a.data[2 * (size_t)k + 1];
+      } else {
+        const EncodeSrc s = a.src[blockIdx.y];
+        v = (double)a.data[(size_t)s.src * a.n + ((k + s.rot) & (a.n - 1))];
+      }
+    }
+    sr[e] = v;
+    si[e] = vi;
+  }
+  for (int rl = INV ? rows : 2; INV ? rl >= 2 : rl <= rows; rl = INV ? rl >> 1 : rl << 1) {
+    __syncthreads();
+    const int rh = rl >> 1;
+    for (int u = threadIdx.x; u < E / 2; u += 256) {
+      const int c = u % FFT_CW, b = u / FFT_CW, jr = b & (rh - 1);
+      const int k = (2 * (b - jr) + jr) * FFT_CW + c, k2 = k + rh * FFT_CW;
+      fft_butterfly<INV>(a, rl * FFT_B, jr * FFT_B + col0 + c, sr[k], si[k], sr[k2], si[k2]);
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += 256) {
+    const int k = (e / FFT_CW) * FFT_B + col0 + e % FFT_CW;
+    if (INV) {
+      R[k] = sr[e];
+      I[k] = si[e];
+    } else if (a.mode == 0) {
+      ((float*)a.out)[k] = (float)sr[e];
+    } else if (a.mode == 1) {
+      ((double*)a.out)[k] = sr[e];
+    } else {
+      ((float*)a.out)[2 * (size_t)k] = (float)sr[e];
+      ((float*)a.out)[2 * (size_t)k + 1] = (float)si[e];
+    }
+  }
 }
 
 // fixed-point record of one coefficient (Lattigo SingleFloat64ToFixedPointCRT)
@@ -111,18 +183,136 @@ __global__ void encode_finish_kernel(u64* __restrict__ out, size_t out_pstride, 
   }
 }
 
+// The coefficient x of a plaintext at its level: the centred CRT value
+//   acc = sum_i y_i * (Q / q_i) - k Q,  y_i = x_i (Q / q_i)^-1 mod q_i,
+// k = floor(sum_i y_i / q_i) in float64 (off by at most one, corrected), then
+// Q - acc for acc >= floor(Q / 2), the nearest double of it (ties to even) over
+// the scale, stored at its bit-reversed place of the FFT.  One thread a
+// coefficient, acc in W words (2^(64 W) > 2^8 Q) held in registers up to 32
+// words; l + 1 passes of W multiply-adds over wave-uniform table words.  One
+// wave a SIMD at N = 2^16, so the next row's word is loaded a row ahead.
+// Decrypt and Decode of 23 limbs there took 7.5 ms with this sum on the host
+// (12 MB of residues fetched, 16 threads); 0.75 ms with it here, 0.65 of them
+// the caller's list of floats.
+template <int W>
+__global__ __launch_bounds__(256) void decode_crt_kernel(DecodeArgs d) {
+#pragma clang fp contract(off)
+  constexpr int UN = W <= 32 ? W : 1;
+  const int x = blockIdx.x * blockDim.x + threadIdx.x;
+  const int N = d.N, n = N >> 1;
+  u64 a[W];
+#pragma unroll UN
+  for (int w = 0; w < W; w++) a[w] = 0;
+  double est = 0.0;
+  u64 next = d.coef[x];
+  for (int i = 0; i < d.nl; i++) {
+    const BConvSrc s = d.src[i];
+    const u64 xi = next;
+    next = d.coef[(size_t)min(i + 1, d.nl - 1) * N + x];  // in flight while row i is multiplied
+    const u64 y = shoup_mul(xi, s.hinv, s.hinvp, s.q);
+    est += (double)y / s.qd;
+    const u64* h = d.hat + (size_t)i * W;
+    u64 c = 0;
+#pragma unroll UN
+    for (int w = 0; w < W; w++) {
+      const u128 t = (u128)h[w] * y + a[w] + c;
+      a[w] = (u64)t;
+      c = (u64)(t >> 64);
+    }
+  }
+  const u64* Q = d.hat + (size_t)d.nl * W;
+  const u64* Qh = Q + W;
+  const u64 k = (u64)est;
+  u64 c = 0, br = 0;
+#pragma unroll UN
+  for (int w = 0; w < W; w++) {
+    const u128 t = (u128)Q[w] * k + c;
+    c = (u64)(t >> 64);
+    const u128 s = (u128)a[w] - (u64)t - br;
+    a[w] = (u64)s;
+    br = (u64)(s >> 64) & 1;
+  }
+  // k one too large leaves acc - Q (negative), one too small acc + Q
+  const u64 neg = 0 - (a[W - 1] >> 63);
+  c = 0; br = 0;
+#pragma unroll UN
+  for (int w = 0; w < W; w++) {
+    const u128 t = (u128)a[w] + (Q[w] & neg) + c;
+    a[w] = (u64)t;
+    c = (u64)(t >> 64);
+    br = (u64)(((u128)a[w] - Q[w] - br) >> 64) & 1;
+  }
+  const u64 over = br - 1;  // all ones where acc >= Q
+  u64 brh = 0;
+  br = 0;
+#pragma unroll UN
+  for (int w = 0; w < W; w++) {
+    const u128 t = (u128)a[w] - (Q[w] & over) - br;
+    a[w] = (u64)t;
+    br = (u64)(t >> 64) & 1;
+    brh = (u64)(((u128)a[w] - Qh[w] - brh) >> 64) & 1;
+  }
+  const bool minus = brh == 0;
+  br = 0;
+#pragma unroll UN
+  for (int w = 0; w < W; w++) {
+    const u128 t = (u128)Q[w] - a[w] - br;
+    br = (u64)(t >> 64) & 1;
+    if (minus) a[w] = (u64)t;
+  }
+  // the top 64 bits, every bit below them in the last one
+  u64 hi = 0, lo = 0, rest = 0;
+  int top = -1;
+#pragma unroll UN
+  for (int w = W - 1; w >= 0; w--) {
+    if (top < 0) {
+      if (a[w]) { top = w; hi = a[w]; }
+    } else if (w == top - 1) {
+      lo = a[w];
+    } else {
+      rest |= a[w];
+    }
+  }
+  double v;
+  if (top <= 0) {
+    v = (double)hi;
+  } else {
+    const int lz = __clzll((long long)hi);
+    const u64 m = lz ? (hi << lz) | (lo >> (64 - lz)) : hi;
+    const u64 low = lz ? lo << lz : lo;
+    v = ldexp((double)(m | ((low | rest) ? 1 : 0)), 64 * top - lz);
+  }
+  if (minus) v = -v;
+  v = v / d.scale;
+  const int i = x < n ? x : x - n;
+  (x < n ? d.re : d.im)[brv_bits(i, d.logn)] = v;
+}
+
 }  // namespace
 
 void launch_encode_fft(u64* out, size_t out_pstride, RowMap rm, const float* data, const EncodeSrc* src, int np, int nvals,
                        double scale, double* re, double* im, size_t pstride, const int* rotgroup, const double* rre,
                        const double* rim, const ModC* mods, int logN, hipStream_t st, bool complex_in) {
-  const int N = 1 << logN, n = N >> 1, M = 2 * N, logn = logN - 1;
+  const int N = 1 << logN, n = N >> 1, logn = logN - 1;
   const int tpb = 256;
-  hipLaunchKernelGGL(encode_load_kernel, dim3((n + tpb - 1) / tpb, np), dim3(tpb), 0, st, re, im, pstride, data, src, n, nvals,
-                     complex_in ? 1 : 0);
-  for (int len = n; len >= 2; len >>= 1)
-    hipLaunchKernelGGL(special_ifft_stage_kernel, dim3((n / 2 + tpb - 1) / tpb, np), dim3(tpb), 0, st, re, im, pstride, n, len,
-                       M, rotgroup, rre, rim);
+  const FftArgs f{re, im, pstride, n, 2 * N, rotgroup, rre, rim, data, src, nvals, complex_in ? 1 : 0, nullptr, 0};
+  hipLaunchKernelGGL(fft_col_kernel<true>, dim3(FFT_B / FFT_CW, np), dim3(256), 0, st, f);
+  hipLaunchKernelGGL(fft_block_kernel<true>, dim3(n / FFT_B, np), dim3(FFT_B / 2), 0, st, f);
   hipLaunchKernelGGL(encode_finish_kernel, dim3((N + tpb - 1) / tpb, np), dim3(tpb), 0, st, out, out_pstride, rm, re, im,
                      pstride, n, logn, scale, mods, N);
+}
+
+void launch_decode_fft(const DecodeArgs& d, int words, const int* rotgroup, const double* rre, const double* rim, void* out,
+                       int mode, hipStream_t st) {
+  const int n = d.N / 2;
+  const dim3 grid(d.N / 256), block(256);
+  if (words <= 4) hipLaunchKernelGGL(decode_crt_kernel<4>, grid, block, 0, st, d);
+  else if (words <= 8) hipLaunchKernelGGL(decode_crt_kernel<8>, grid, block, 0, st, d);
+  else if (words <= 16) hipLaunchKernelGGL(decode_crt_kernel<16>, grid, block, 0, st, d);
+  else if (words <= 24) hipLaunchKernelGGL(decode_crt_kernel<24>, grid, block, 0, st, d);
+  else if (words <= 32) hipLaunchKernelGGL(decode_crt_kernel<32>, grid, block, 0, st, d);
+  else hipLaunchKernelGGL(decode_crt_kernel<DECODE_MAXW>, grid, block, 0, st, d);
+  const FftArgs f{d.re, d.im, 0, n, 2 * d.N, rotgroup, rre, rim, nullptr, nullptr, 0, 0, out, mode};
+  hipLaunchKernelGGL(fft_block_kernel<false>, dim3(n / FFT_B), dim3(FFT_B / 2), 0, st, f);
+  hipLaunchKernelGGL(fft_col_kernel<false>, dim3(FFT_B / FFT_CW), dim3(256), 0, st, f);
 }

@@ -265,6 +265,7 @@ void launch_moddown_rescale_spread(u64* ext, size_t e_bstride, const u64* xl, si
 void launch_sample_uniform(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, hipStream_t st);
 void launch_sample_cbd(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, bool add, hipStream_t st);
 void launch_signed_rows(u64* out, RowMap rm, const int8_t* v, const ModC* mods, int N, hipStream_t st);
+void launch_ternary_rows(u64* out, RowMap rm, const uint32_t* pos, int npos, const ModC* mods, int N, hipStream_t st);
 void launch_gk_combine(u64* b, const u64* a, const u64* soR, const u64* sR, int own0, int own1, const u64* pmod, int rows, const ModC* mods, int N, hipStream_t st);
 // Device encoder (encoder.hip): plaintext p of a batch takes element k from
 // data[src * slots + ((k + rot) mod slots)] (zero past nvals), runs the special
@@ -275,6 +276,27 @@ struct EncodeSrc { int src, rot; };
 void launch_encode_fft(u64* out, size_t out_pstride, RowMap rm, const float* data, const EncodeSrc* src, int np, int nvals,
                        double scale, double* re, double* im, size_t pstride, const int* rotgroup, const double* rre,
                        const double* rim, const ModC* mods, int logN, hipStream_t st, bool complex_in = false);
+// Device decoder: coefficients coef[nl][N] (rows q_0 .. q_{nl-1}), tables of the
+// level: src[i] (hinv of Q / q_i), hat [nl][W] words of Q / q_i, then Q and
+// floor(Q / 2); W the first of 4, 8, 16, 24, 32, DECODE_MAXW not below `words`
+// (words of 2^8 Q; decode_words).  re / im are work buffers of N / 2 doubles;
+// out takes the slots' real parts as float (mode 0) or double (1), or (re, im)
+// pairs of float (2).
+#define DECODE_MAXW 96
+struct DecodeArgs {
+  const u64* coef;
+  int nl, N, logn;
+  const BConvSrc* src;
+  const u64* hat;
+  double scale;
+  double *re, *im;
+};
+inline int decode_words(int words) {
+  for (int w : {4, 8, 16, 24, 32}) if (words <= w) return w;
+  return DECODE_MAXW;
+}
+void launch_decode_fft(const DecodeArgs& d, int words, const int* rotgroup, const double* rre, const double* rim, void* out,
+                       int mode, hipStream_t st);
 // multiplication by the imaginary unit (the monomial X^(N/2)) in the NTT domain:
 // slot x < N/2 times iu[m], slot x >= N/2 times q - iu[m] (Shoup pairs iu / iup, niu / niup)
 void launch_mul_i(u64* out, const u64* in, size_t bstride, int batch, RowMap rm, const u64* iu, const u64* iup,

@@ -1154,6 +1154,27 @@ __global__ void signed_rows_kernel(u64* __restrict__ out, RowMap rm, const int8_
 void launch_signed_rows(u64* out, RowMap rm, const int8_t* v, const ModC* mods, int N, hipStream_t st) {
   hipLaunchKernelGGL(signed_rows_kernel, dim3(N / 256, rm.nact(), 1), dim3(256), 0, st, out, rm, v, mods, N);
 }
+// The polynomial with coefficient +1 at pos[i] / 2 for even pos[i], -1 for odd
+// ones (distinct places) and 0 elsewhere, reduced into every row: 1024
+// coefficients of a row a workgroup, gathered in LDS.
+__global__ __launch_bounds__(256) void ternary_rows_kernel(u64* __restrict__ out, RowMap rm, const uint32_t* __restrict__ pos,
+                                                          int npos, const ModC* __restrict__ mods, int N) {
+  __shared__ int v[1024];
+  const int base = blockIdx.x * 1024;
+  for (int i = threadIdx.x; i < 1024; i += 256) v[i] = 0;
+  __syncthreads();
+  for (int i = threadIdx.x; i < npos; i += 256) {
+    const int x = (int)(pos[i] >> 1) - base;
+    if (x >= 0 && x < 1024) v[x] = pos[i] & 1 ? -1 : 1;
+  }
+  __syncthreads();
+  const int row = rm.row(blockIdx.y);
+  const u64 q = mods[rm.mod(row)].q;
+  for (int i = threadIdx.x; i < 1024; i += 256) out[(size_t)row * N + base + i] = v[i] < 0 ? q - 1 : (u64)v[i];
+}
+void launch_ternary_rows(u64* out, RowMap rm, const uint32_t* pos, int npos, const ModC* mods, int N, hipStream_t st) {
+  hipLaunchKernelGGL(ternary_rows_kernel, dim3(N / 1024, rm.nact(), 1), dim3(256), 0, st, out, rm, pos, npos, mods, N);
+}
 // Galois-key body: b = -a*s' + e (+ P*s on own rows), in place on b; a, s', s in
 // (a standard, sR/soR Montgomery), own rows [own0, own1) of the Q chain.
 __global__ void gk_combine_kernel(u64* __restrict__ b, const u64* __restrict__ a, const u64* __restrict__ soR,

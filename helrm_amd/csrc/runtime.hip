@@ -22,7 +22,6 @@
 #include <set>
 #include <stdexcept>
 #include <string>
-#include <thread>
 #include <unordered_map>
 #include <unordered_set>
 #include <vector>
@@ -161,17 +160,25 @@ inline u64 ST_RLK_E(u64 d) { return (10ULL << 56) | d; }
 constexpr u64 ST_SEED_A = 11ULL << 56;
 inline u64 ST_SEED_E(u64 e) { return (12ULL << 56) | e; }
 // ternary vector with exactly h entries +-1 (partial Fisher-Yates)
-std::vector<int8_t> ternary_hw(u64 seed, u64 stream, int N, int h) {
-  std::vector<int> idx(N);
-  for (int i = 0; i < N; i++) idx[i] = i;
-  std::vector<int8_t> out(N, 0);
+// The drawn positions in order, each as 2 * position + (1 for -1).  The
+// shuffle's array is kept only where a swap has touched it.
+std::vector<uint32_t> ternary_positions(u64 seed, u64 stream, int N, int h) {
+  std::unordered_map<int, int> moved;
+  auto at = [&](int i) { auto it = moved.find(i); return it == moved.end() ? i : it->second; };
   if (h > N) h = N;
+  std::vector<uint32_t> pos(h);
   for (int k = 0; k < h; k++) {
     u64 r = rand64(seed, stream, (u64)k);
     int j = k + (int)(((u128)r * (u64)(N - k)) >> 64);
-    std::swap(idx[k], idx[j]);
-    out[idx[k]] = (rand64(seed, stream, (1ULL << 32) + (u64)k) & 1) ? -1 : 1;
+    const int a = at(k), b = at(j);
+    moved[j] = a;  // place k is drawn and not read again
+    pos[k] = 2 * (uint32_t)b + (uint32_t)(rand64(seed, stream, (1ULL << 32) + (u64)k) & 1);
   }
+  return pos;
+}
+std::vector<int8_t> ternary_hw(u64 seed, u64 stream, int N, int h) {
+  std::vector<int8_t> out(N, 0);
+  for (uint32_t p : ternary_positions(seed, stream, N, h)) out[p >> 1] = p & 1 ? -1 : 1;
   return out;
 }
 
@@ -334,6 +341,13 @@ struct BConvHost { int ns; BConvTable tab; DU64 hat, nS; DevArray<BConvTable> dt
 
 struct Timing { bool on = false; std::map<std::string, std::vector<std::pair<hipEvent_t, hipEvent_t>>> ev; std::map<std::string, std::pair<long, double>> acc; };
 
+// the decoder's CRT tables of a level (decode_table)
+struct DecodeTable {
+  int words = 0;
+  DevArray<BConvSrc> src;
+  DU64 tab;
+};
+
 struct Scheme {
   int logN = 0, N = 0, L = 0, K = 0, dnum = 0, logscale = 0, h = 0;
   u64 seed = 0;
@@ -362,6 +376,7 @@ struct Scheme {
   std::map<u64, DevArray<uint32_t>> perms, perm_invs;
   std::map<std::tuple<int, int, size_t>, std::unique_ptr<struct DigitRows>> digit_rows;
   std::map<int, std::unique_ptr<struct FoldRows>> fold_rows;  // per level
+  std::map<int, DecodeTable> decode_tabs;                    // per level
   // Galois keys this library generated (a halves a function of the seed, the
   // key's stream and the word's position, regenerated by the kernels); a
   // loaded key is read whole
@@ -788,27 +803,6 @@ void init_encoder(Scheme& s) {
   s.d_rim = DevArray<double>(s.rim.size()); upload(s.d_rim.p, s.rim.data(), s.rim.size());
   s.d_rotgroup = DevArray<int>(slots); upload(s.d_rotgroup.p, s.rotgroup.data(), slots);
 }
-void bitrev(std::vector<double>& re, std::vector<double>& im, int n) {
-  int logn = 0; while ((1 << logn) < n) logn++;
-  for (int i = 0; i < n; i++) { int j = brv(i, logn); if (j > i) { std::swap(re[i], re[j]); std::swap(im[i], im[j]); } }
-}
-void special_fft(const Scheme& s, std::vector<double>& re, std::vector<double>& im, int n) {
-  const int M = 2 * s.N;
-  bitrev(re, im, n);
-  for (int len = 2; len <= n; len <<= 1) {
-    int lenh = len >> 1, lenq = len << 2, gap = M / lenq, mask = lenq - 1;
-    for (int i = 0; i < n; i += len)
-      for (int j = 0; j < lenh; j++) {
-        int k = i + j;
-        int idx = (s.rotgroup[j] & mask) * gap;
-        double wr = s.rre[idx], wi = s.rim[idx];
-        double ur = re[k], ui = im[k], xr = re[k + lenh], xi = im[k + lenh];
-        double vr = xr * wr - xi * wi, vi = xr * wi + xi * wr;
-        re[k] = ur + vr; im[k] = ui + vi;
-        re[k + lenh] = ur - vr; im[k + lenh] = ui - vi;
-      }
-  }
-}
 // Encode np plaintexts on the device: plaintext p reads data[src[p].src * slots
 // + ((k + src[p].rot) mod slots)] (zero past nvals), its residues go to rows
 // rm of out + p * out_pstride, then the forward NTT.  Batches of up to 64
@@ -837,87 +831,43 @@ void encode_device(const float* h_data, size_t ndata, const std::vector<EncodeSr
   sync();
 }
 
-// ---- big integers for the decoder's centred CRT ----
-struct Big { std::vector<u64> w; };
-void big_norm(Big& a) { while (!a.w.empty() && a.w.back() == 0) a.w.pop_back(); }
-void big_mul_small(Big& a, u64 m) {
+// ---- decoder ----
+// CRT tables of a level, in words little endian: Q / q_i for every i, Q and
+// floor(Q / 2), `words` each (launch_decode_fft).
+void big_mul_small(std::vector<u64>& a, u64 m) {
   u128 c = 0;
-  for (auto& x : a.w) { u128 t = (u128)x * m + c; x = (u64)t; c = t >> 64; }
-  if (c) a.w.push_back((u64)c);
-  big_norm(a);
+  for (auto& x : a) { u128 t = (u128)x * m + c; x = (u64)t; c = t >> 64; }
+  REQUIRE(c == 0, "decoder table overflow");
 }
-int big_cmp(const Big& a, const Big& b) {
-  if (a.w.size() != b.w.size()) return a.w.size() < b.w.size() ? -1 : 1;
-  for (size_t i = a.w.size(); i-- > 0;) if (a.w[i] != b.w[i]) return a.w[i] < b.w[i] ? -1 : 1;
-  return 0;
-}
-void big_add(Big& a, const Big& b) {
-  size_t n = std::max(a.w.size(), b.w.size()); a.w.resize(n, 0); u64 c = 0;
-  for (size_t i = 0; i < n; i++) { u128 t = (u128)a.w[i] + (i < b.w.size() ? b.w[i] : 0) + c; a.w[i] = (u64)t; c = (u64)(t >> 64); }
-  if (c) a.w.push_back(c);
-}
-void big_sub(Big& a, const Big& b) {  // a >= b
-  u64 br = 0;
-  for (size_t i = 0; i < a.w.size(); i++) { u128 t = (u128)a.w[i] - (i < b.w.size() ? b.w[i] : 0) - br; a.w[i] = (u64)t; br = (u64)(t >> 64) ? 1 : 0; }
-  big_norm(a);
-}
-double big_to_double(const Big& a) {  // nearest, ties to even
-  if (a.w.empty()) return 0.0;
-  int top = (int)a.w.size() - 1, lz = __builtin_clzll(a.w[top]);
-  int bitlen = top * 64 + (64 - lz);
-  if (bitlen <= 64) return (double)a.w[0];
-  int sh = bitlen - 64, wi = sh / 64, bi = sh % 64;
-  u64 hi = bi ? (a.w[wi] >> bi) | (a.w[wi + 1] << (64 - bi)) : a.w[wi];
-  bool sticky = bi && (a.w[wi] & ((1ULL << bi) - 1));
-  for (int i = 0; i < wi; i++) if (a.w[i]) sticky = true;
-  if (sticky) hi |= 1;
-  return std::ldexp((double)hi, sh);
-}
-// Lattigo Encoder.Decode (float64): centred CRT value / scale, SpecialFFT, real part
-std::vector<double> decode_host(const std::vector<u64>& coef, int level, double scale, std::vector<double>* imag = nullptr) {
+DecodeTable& decode_table(int level) {
   Scheme& s = sch();
-  const int N = s.N, slots = N / 2, nl = level + 1;
-  std::vector<double> vals(N);
-  if (level == 0) {
-    u64 q = s.mod[0];
-    for (int x = 0; x < N; x++) { u64 v = coef[x]; vals[x] = (v >= (q >> 1) ? -(double)(q - v) : (double)v) / scale; }
-  } else {
-    Big Q; Q.w = {1};
-    for (int i = 0; i < nl; i++) big_mul_small(Q, s.mod[i]);
-    Big Qh = Q;
-    for (size_t i = 0; i < Qh.w.size(); i++) Qh.w[i] = (Qh.w[i] >> 1) | (i + 1 < Qh.w.size() ? Qh.w[i + 1] << 63 : 0);
-    big_norm(Qh);
-    std::vector<Big> hat(nl); std::vector<u64> hinv(nl);
-    for (int i = 0; i < nl; i++) {
-      hat[i].w = {1}; u64 pr = 1;
-      for (int j = 0; j < nl; j++) if (j != i) { big_mul_small(hat[i], s.mod[j]); pr = mulmod(pr, s.mod[j] % s.mod[i], s.mod[i]); }
-      hinv[i] = invmod(pr, s.mod[i]);
+  auto it = s.decode_tabs.find(level);
+  if (it != s.decode_tabs.end()) return it->second;
+  const int nl = level + 1;
+  double bits = 8;  // below a word's rounding error for any number of moduli here
+  for (int i = 0; i < nl; i++) bits += std::log2((double)s.mod[i]) + 1e-9;
+  DecodeTable t;
+  t.words = decode_words((int)std::ceil(bits / 64));
+  const int W = t.words;
+  std::vector<u64> tab((size_t)(nl + 2) * W, 0);
+  std::vector<BConvSrc> src(nl);
+  for (int i = 0; i <= nl; i++) {  // i == nl: Q
+    std::vector<u64> h(W, 0); h[0] = 1;
+    for (int j = 0; j < nl; j++) if (j != i) big_mul_small(h, s.mod[j]);
+    std::copy(h.begin(), h.end(), tab.begin() + (size_t)i * W);
+    if (i == nl) {
+      for (int w = 0; w < W; w++) tab[(size_t)(nl + 1) * W + w] = (h[w] >> 1) | (w + 1 < W ? h[w + 1] << 63 : 0);
+    } else {
+      const u64 q = s.mod[i];
+      u64 pr = 1;
+      for (int j = 0; j < nl; j++) if (j != i) pr = mulmod(pr, s.mod[j] % q, q);
+      const u64 hi = invmod(pr, q);
+      src[i] = BConvSrc{q, hi, shoup(hi, q), (double)q};
     }
-    auto work = [&](int x0, int x1) {
-      for (int x = x0; x < x1; x++) {
-        Big acc;
-        for (int i = 0; i < nl; i++) {
-          u64 y = mulmod(coef[(size_t)i * N + x], hinv[i], s.mod[i]);
-          Big t = hat[i]; big_mul_small(t, y); big_add(acc, t);
-        }
-        while (big_cmp(acc, Q) >= 0) big_sub(acc, Q);
-        double d;
-        if (big_cmp(acc, Qh) >= 0) { Big t = Q; big_sub(t, acc); d = -big_to_double(t); }
-        else d = big_to_double(acc);
-        vals[x] = d / scale;
-      }
-    };
-    int nt = (int)std::min<unsigned>(16, std::max(1u, std::thread::hardware_concurrency()));
-    if (N < 4096) nt = 1;
-    std::vector<std::thread> th;
-    for (int t = 0; t < nt; t++) th.emplace_back(work, (int)((long)N * t / nt), (int)((long)N * (t + 1) / nt));
-    for (auto& t : th) t.join();
   }
-  std::vector<double> re(slots), im(slots);
-  for (int i = 0; i < slots; i++) { re[i] = vals[i]; im[i] = vals[i + slots]; }
-  special_fft(s, re, im, slots);
-  if (imag) *imag = im;
-  return re;
+  t.tab = DU64(tab.size()); upload(t.tab.p, tab.data(), tab.size());
+  t.src = DevArray<BConvSrc>(nl); upload(t.src.p, src.data(), src.size());
+  return s.decode_tabs.emplace(level, std::move(t)).first->second;
 }
 
 // ============================================================================
@@ -1850,17 +1800,16 @@ std::unique_ptr<Cipher> encrypt_pt(const Plain& pt) {
   REQUIRE(s.has_pk, "public key not generated");
   const int l = pt.level, N = s.N, nm = s.L + s.K, nr = l + 2;
   const u64 enc = s.enc_counter++;
-  std::vector<int8_t> u = ternary_hw(s.seed, ST_ENC_U(enc), N, s.h);
-  DevArray<int8_t> du(N); upload(du.p, u.data(), N);
+  std::vector<uint32_t> u = ternary_positions(s.seed, ST_ENC_U(enc), N, s.h);
+  DevArray<uint32_t> du(std::max<size_t>(u.size(), 1)); upload(du.p, u.data(), u.size());
   RowMap rm{nr, l + 1, 0, s.L, 0, 0};
-  DU64 uq((size_t)nr * N), pk((size_t)2 * nr * N), tt((size_t)2 * nr * N);
-  launch_signed_rows(uq.p, rm, du.p, s.d_mods.p, N, s.st);
+  DU64 uq((size_t)nr * N), tt((size_t)2 * nr * N);
+  launch_ternary_rows(uq.p, rm, du.p, (int)u.size(), s.d_mods.p, N, s.st);
   ntt(uq.p, 0, 1, rm, true);
-  for (int p = 0; p < 2; p++) {
-    d2d(pk.p + (size_t)p * nr * N, s.pkR.p + (size_t)p * nm * N, (size_t)(l + 1) * N * 8);
-    d2d(pk.p + (size_t)p * nr * N + (size_t)(l + 1) * N, s.pkR.p + (size_t)p * nm * N + (size_t)s.L * N, (size_t)N * 8);
-  }
-  launch_mont_mul(tt.p, (size_t)nr * N, uq.p, 0, pk.p, (size_t)nr * N, 2, rm, s.d_mods.p, N, false, s.st);
+  // pkR holds every modulus: rows q_0..q_l, then row p_0 of it
+  launch_mont_mul(tt.p, (size_t)nr * N, uq.p, 0, s.pkR.p, (size_t)nm * N, 2, rows_q(l), s.d_mods.p, N, false, s.st);
+  launch_mont_mul(tt.p + (size_t)(l + 1) * N, (size_t)nr * N, uq.p + (size_t)(l + 1) * N, 0, s.pkR.p + (size_t)s.L * N,
+                  (size_t)nm * N, 2, RowMap{1, 0, 0, s.L, 0, 0}, s.d_mods.p, N, false, s.st);
   ntt(tt.p, (size_t)nr * N, 2, rm, false);
   launch_sample_cbd(tt.p, rm, s.seed, ST_ENC_E0(enc), s.d_mods.p, N, true, s.st);
   launch_sample_cbd(tt.p + (size_t)nr * N, rm, s.seed, ST_ENC_E1(enc), s.d_mods.p, N, true, s.st);
@@ -1941,15 +1890,21 @@ std::unique_ptr<Plain> encode_complex_values(const float* v, int n, int level, d
   encode_device(buf.data(), buf.size(), {EncodeSrc{0, 0}}, n, scale, rows_q(level), p->d.p, 0, true);
   return p;
 }
-std::vector<double> decode_pt(const Plain& p, std::vector<double>* imag = nullptr) {
+// The slots of a plaintext: mode 0 real parts as float, 1 as double, 2 (re, im)
+// pairs of float, written to out (Lattigo Encoder.Decode in float64: centred
+// CRT value / scale, special FFT).
+void decode_pt(const Plain& p, int mode, void* out) {
   Scheme& s = sch();
   const int N = s.N, l = p.level;
-  DU64 tmp((size_t)(l + 1) * N);
-  d2d(tmp.p, p.d.p, tmp.bytes());
-  ntt(tmp.p, 0, 1, rows_q(l), false);
-  std::vector<u64> coef((size_t)(l + 1) * N);
-  download(coef.data(), tmp.p, coef.size());
-  return decode_host(coef, l, p.scale, imag);
+  DecodeTable& t = decode_table(l);
+  DU64 coef((size_t)(l + 1) * N);
+  ntt_oop(p.d.p, 0, coef.p, 0, 1, rows_q(l), false);
+  DevArray<double> re(N / 2), im(N / 2);
+  const size_t bytes = (size_t)(N / 2) * (mode == 0 ? 4 : 8);
+  DevArray<char> dout(bytes);
+  launch_decode_fft(DecodeArgs{coef.p, l + 1, N, s.logN - 1, t.src.p, t.tab.p, p.scale, re.p, im.p}, t.words, s.d_rotgroup.p,
+                    s.d_rre.p, s.d_rim.p, dout.p, mode, s.st);
+  download((char*)out, dout.p, bytes);
 }
 
 template <class T> T* c_array(const std::vector<T>& v) {
@@ -2140,22 +2095,26 @@ int Encode(const float* values, int lenValues, int level, unsigned long scale) {
     return push_pt(encode_values(values, lenValues, level, (double)scale));
   });
 }
-ArrayResultFloat Decode(int plaintextID) {
+static ArrayResultFloat decode_floats(int plaintextID, int mode) {
   ArrayResultFloat r{nullptr, 0};
   guard([&] {
-    std::vector<double> v = decode_pt(get_pt(plaintextID));
-    std::vector<float> f(v.begin(), v.end());
-    r.Data = c_array(f); r.Length = f.size();
+    const size_t n = (size_t)(sch().N / 2) * (mode == 2 ? 2 : 1);
+    const Plain& p = get_pt(plaintextID);
+    std::unique_ptr<float, void (*)(void*)> f((float*)std::malloc(n * sizeof(float)), std::free);
+    if (!f) throw Error("out of host memory");
+    decode_pt(p, mode, f.get());
+    r.Data = f.release(); r.Length = n;
     return 0;
   });
   return r;
 }
+ArrayResultFloat Decode(int plaintextID) { return decode_floats(plaintextID, 0); }
 int DecodeDouble(int plaintextID, double* out, int len) {
   return guard([&] {
-    std::vector<double> v = decode_pt(get_pt(plaintextID));
-    REQUIRE(len >= (int)v.size(), "output buffer too small");
-    std::copy(v.begin(), v.end(), out);
-    return (int)v.size();
+    const Plain& p = get_pt(plaintextID);
+    REQUIRE(len >= sch().N / 2, "output buffer too small");
+    decode_pt(p, 1, out);
+    return sch().N / 2;
   });
 }
 
@@ -2165,18 +2124,7 @@ int EncodeComplex(const float* values, int lenValues, int level, unsigned long s
     return push_pt(encode_complex_values(values, lenValues / 2, level, (double)scale));
   });
 }
-ArrayResultFloat DecodeComplex(int plaintextID) {
-  ArrayResultFloat r{nullptr, 0};
-  guard([&] {
-    std::vector<double> im;
-    std::vector<double> re = decode_pt(get_pt(plaintextID), &im);
-    std::vector<float> f(2 * re.size());
-    for (size_t i = 0; i < re.size(); i++) { f[2 * i] = (float)re[i]; f[2 * i + 1] = (float)im[i]; }
-    r.Data = c_array(f); r.Length = f.size();
-    return 0;
-  });
-  return r;
-}
+ArrayResultFloat DecodeComplex(int plaintextID) { return decode_floats(plaintextID, 2); }
 
 // ---- encryptor ----
 int NewEncryptor(void) { return guard([&] { sch().encryptor = true; return 0; }); }

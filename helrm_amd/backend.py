@@ -52,6 +52,12 @@ class HipFunction:
         self.checked = checked
 
     def __call__(self, *args):
+        out = self.array(*args)
+        return out.tolist() if isinstance(out, np.ndarray) else out
+
+    def array(self, *args):
+        """The call with a float array result left a float64 array: a list of
+        2^15 Python floats costs 0.4 ms to make and 0.9 ms to read back."""
         c_args = []
         for arg in args:
             typ = self.func.argtypes[len(c_args)]
@@ -79,10 +85,10 @@ class HipFunction:
                     msg = HipFunction.lib.GetLastError().decode()
                     if msg:
                         raise HipError(msg)
-                return []
+                return np.zeros(0) if isinstance(res, ArrayResultFloat) else []
             n = int(res.Length)
             if isinstance(res, ArrayResultFloat):
-                out = np.ctypeslib.as_array(res.Data, shape=(n,)).astype(np.float64).tolist()
+                out = np.ctypeslib.as_array(res.Data, shape=(n,)).astype(np.float64)
             else:
                 out = [int(res.Data[i]) for i in range(n)]
             HipFunction.lib.FreeCArray(ctypes.cast(res.Data, ctypes.c_void_p))

@@ -266,15 +266,13 @@ class Scheme:
         vec = np.concatenate([values, np.zeros(pad)]) if pad or len(values) == 0 else values
         if len(vec) == 0:
             vec = np.zeros(slots)
-        ids = [self.backend.Encode(vec[i * slots:(i + 1) * slots].tolist(), level, int(scale))
+        ids = [self.backend.Encode(vec[i * slots:(i + 1) * slots], level, int(scale))
                for i in range(len(vec) // slots)]
         return PlainTensor(self, ids, len(values))
 
     def decode(self, pt):
-        vals = []
-        for i in pt.ids:
-            vals.extend(self.backend.Decode(i))
-        return np.asarray(vals[: pt.n], dtype=np.float64)
+        vals = [self.backend.Decode.array(i) for i in pt.ids]
+        return np.concatenate(vals)[: pt.n] if vals else np.zeros(0)
 
     def encrypt(self, pt):
         return CipherTensor(self, [self.backend.Encrypt(i) for i in pt.ids], pt.n)

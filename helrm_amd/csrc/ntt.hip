@@ -1093,21 +1093,30 @@ void launch_ntt(u64* data, size_t bstride, int batch, RowMap rm, int logN, bool 
   launch_ntt(data, bstride, data, bstride, batch, rm, logN, forward, tw, st);
 }
 
-// Workgroup shape: 256-thread tiles (narrower tiles lose coalescing and
-// measured slower even for launches of a few limbs).
+// Workgroup shape: 256-thread tiles (column tiles narrower than 16 words lose
+// coalescing and measured slower even for launches of a few limbs).
 // Launches over at most this many limbs use the 8-word kernels (a launch of
 // few limbs leaves most SIMDs with one or two waves of the 16-word kernels).
 #ifndef NTT_W8_MAX_LIMBS
 #define NTT_W8_MAX_LIMBS 96
 #endif
 
+// The 8-word kernels' workgroups are halved, down to 16 columns or one wave of
+// rows, while the launch has fewer than this many: a pass over 4 limbs of
+// N = 2^13 then runs on 32 or 64 CUs instead of 8 or 16, and its waves have a
+// SIMD each instead of sharing one with another.  N = 2^13, 4 limbs and one
+// special modulus: a rotation 55 -> 46 us, a whole one-table lookup 456 -> 405
+// us; a bound of 512 measures the same, and N = 2^16 always has more.
+constexpr int W8_FILL = 256;
 static void ntt_launch(NttArgs a, int nlimbs, bool forward, hipStream_t st) {
   int SA, SB;
   ntt_split(a.logN, &SA, &SB);
   a.SA = SA; a.SB = SB;
   if (nlimbs <= NTT_W8_MAX_LIMBS) {
     const int TA = 1 << (SA - 3), TB = 1 << (SB - 3), C = 1 << SB, R = 1 << SA;
-    const int nsubA = std::min(512 / TA, C), nsubB = std::min(256 / TB, R);
+    int nsubA = std::min(512 / TA, C), nsubB = std::min(256 / TB, R);
+    while (nsubA > 16 && nlimbs * (C / nsubA) < W8_FILL) nsubA /= 2;
+    while (nsubB * TB > 64 && nlimbs * (R / nsubB) < W8_FILL) nsubB /= 2;
     NttArgs aA = a; aA.nsub = nsubA;
     NttArgs aB = a; aB.nsub = nsubB;
     if (forward) { aB.src = a.data; aB.sstride = a.bstride; } else { aA.src = a.data; aA.sstride = a.bstride; }

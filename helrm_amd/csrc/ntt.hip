@@ -1,8 +1,9 @@
 // ntt.hip -- negacyclic NTT / inverse NTT for gfx950.
 //
 // Transform of one limb of N = 2^logN words, N = R x C with R = 2^SA rows of
-// C = 2^SB columns (5 <= SA, SB <= 8).  Forward (Cooley-Tukey, distances
-// N/2 .. 1, twiddle W[(N + g) >> (lt + 1)] for the pair (g, g + 2^lt)):
+// C = 2^SB columns (6 <= SA, SB <= 8; 5 in the one-workgroup form).  Forward
+// (Cooley-Tukey, distances N/2 .. 1, twiddle W[(N + g) >> (lt + 1)] for the
+// pair (g, g + 2^lt)):
 //   pass A  distances N/2 .. C      (column sub-transforms of size R)
 //   pass B  distances C/2 .. 1      (row sub-transforms of size C)
 // Inverse (Gentleman-Sande, distances 1 .. N/2, then N^-1): pass B, pass A.
@@ -287,7 +288,7 @@ __device__ __forceinline__ LimbRef limb_ref(const NttArgs& a, int y) {
   return l;
 }
 // src offset of the same limb (first pass of an out-of-place transform)
-__device__ __forceinline__ int64_t limb_src_off(const NttArgs& a, int y, const LimbRef& l) {
+__device__ __forceinline__ int64_t limb_src_off(const NttArgs& a, const LimbRef& l) {
   if (a.list) return l.off + ((int64_t)l.pad << a.logN);
   return (int64_t)l.pad * (int64_t)a.sstride + (l.off - (int64_t)l.pad * (int64_t)a.bstride);
 }
@@ -311,7 +312,7 @@ __device__ __forceinline__ void ntt_col_int(const NttArgs& a, u64* sm, const Lim
   const uint4* tw = a.tw + (size_t)m * Nn;
   u64 v[16];
   if (FWD) {
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + col;
+    const u64* in = a.src + limb_src_off(a, lr) + col;
     // round 1: rows j + P*i, distances R/2 .. R/16 rows
     RoundTw<4> T1;
     round_tw_load<true, 4>(T1, 0, S - 4 + SB, Nn, tw);
@@ -371,7 +372,7 @@ __device__ __forceinline__ void ntt_col_fp(const NttArgs& a, u64* sm, const Limb
   if (FWD) {
     static_assert(fpb::ct_pass_ok(false, S, true), "float64 forward column pass out of bounds");
     constexpr bool R1 = fpb::ct_pass(false, S, true, 0, true), R2 = fpb::ct_pass(false, S, true, 1, true);
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + col;
+    const u64* in = a.src + limb_src_off(a, lr) + col;
     RoundTw<4> T1;
     round_tw_load<true, 4>(T1, 0, S - 4 + SB, Nn, tw);
 #pragma unroll
@@ -528,7 +529,7 @@ __device__ __forceinline__ void ntt_row_int(const NttArgs& a, u64* sm, const Lim
     __syncthreads();
     row_fwd_tail<S, EPI>(a, srow, lr, r, j, poly);
   } else {
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + (size_t)r * C;
+    const u64* in = a.src + limb_src_off(a, lr) + (size_t)r * C;
     // all 16 loads in flight before the LDS writes; the first round's
     // twiddles are issued behind them and arrive during the barrier
 #pragma unroll
@@ -594,7 +595,7 @@ __device__ __forceinline__ void ntt_row_fp(const NttArgs& a, u64* sm, const Limb
   } else {
     static_assert(fpb::gs_pass_ok(false, S, true), "float64 inverse row pass out of bounds");
     constexpr long B0 = fpb::gs_pass(false, S, true, 0), B1 = fpb::gs_pass(false, S, true, 1);
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + (size_t)r * C;
+    const u64* in = a.src + limb_src_off(a, lr) + (size_t)r * C;
     u64 w[16];
 #pragma unroll
     for (int i = 0; i < 16; i++) w[i] = __builtin_nontemporal_load(&in[j + P * i]);
@@ -706,7 +707,7 @@ __device__ __forceinline__ void ntt_col8_int(const NttArgs& a, u64* sm, const Li
   const uint4* tw = a.tw + (size_t)m * Nn;
   u64 v[8];
   if (FWD) {
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + col;
+    const u64* in = a.src + limb_src_off(a, lr) + col;
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = in[(size_t)w8_elem(w8_ls(S, 0), t, i) * C];
     w8_round<true, S, 0>(v, t, 0, SB, Nn, tw, q);
@@ -766,7 +767,7 @@ __device__ __forceinline__ void ntt_col8_fp(const NttArgs& a, u64* sm, const Lim
   const uint4* tw = a.tw + (size_t)m * Nn;
   double v[8];
   if (FWD) {
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + col;
+    const u64* in = a.src + limb_src_off(a, lr) + col;
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = f_in(in[(size_t)w8_elem(w8_ls(S, 0), t, i) * C]);
     w8_round_fp<true, S, 0, true>(v, t, 0, SB, Nn, tw, fc);
@@ -921,7 +922,7 @@ __device__ __forceinline__ void ntt_row8_int(const NttArgs& a, u64* sm, const Li
     __syncthreads();
     row8_fwd_tail<S, EPI>(a, srow, lr, r, t, poly);
   } else {
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + (size_t)r * C;
+    const u64* in = a.src + limb_src_off(a, lr) + (size_t)r * C;
 #pragma unroll
     for (int i = 0; i < 8; i++) v[i] = __builtin_nontemporal_load(&in[w8_elem(L0, t, i)]);
 #pragma unroll
@@ -989,7 +990,7 @@ __device__ __forceinline__ void ntt_row8_fp(const NttArgs& a, u64* sm, const Lim
     __syncthreads();
     row8_fwd_tail<S, EPI>(a, srow, lr, r, t, poly);
   } else {
-    const u64* in = a.src + limb_src_off(a, blockIdx.y, lr) + (size_t)r * C;
+    const u64* in = a.src + limb_src_off(a, lr) + (size_t)r * C;
     u64 w[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) w[i] = __builtin_nontemporal_load(&in[w8_elem(L0, t, i)]);
@@ -1025,10 +1026,260 @@ __global__ __launch_bounds__(256) void ntt_row8_kernel(NttArgs a) {
   else ntt_row8_int<FWD, S, EPI>(a, sm, lr);
 }
 
+// ---------------------------------------------------------------------------
+// Rings of at most 2^14 words: the whole limb in one workgroup's LDS.  The same
+// rounds as the 16-word passes above (columns, then rows; the inverse the other
+// way), N / 16 threads, the words between all rounds in LDS: one launch and one
+// pass over memory instead of two.  The LDS row pitch is 8 words past C, which
+// spreads the rows that a wave's row rounds touch over the banks.  A row's
+// threads are consecutive lanes of one wave, so its exchanges need no barrier.
+// ---------------------------------------------------------------------------
+template <int LOGN>
+struct LdsShape {
+  static constexpr int SA = LOGN / 2, SB = LOGN - SA, PA = 1 << (SA - 4), PB = 1 << (SB - 4);
+  static constexpr int C = 1 << SB, R = 1 << SA, CP = C + 8;
+};
+__device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+template <bool FWD, int LOGN, bool EPI>
+__device__ __forceinline__ void ntt_lds_int(const NttArgs& a, u64* sm, const LimbRef& lr) {
+  typedef LdsShape<LOGN> H;
+  constexpr int SA = H::SA, SB = H::SB, PA = H::PA, PB = H::PB, C = H::C, CP = H::CP;
+  const int tid = threadIdx.x, m = lr.mod;
+  const int c = tid & (C - 1), jc = tid >> SB;          // columns
+  const int j = tid & (PB - 1), r = tid >> (SB - 4);    // rows
+  const u64 q = a.mods[m].q;
+  constexpr u64 Nn = 1ull << LOGN;
+  u64* poly = a.data + lr.off;
+  const u64* in = a.src + limb_src_off(a, lr);
+  const uint4* tw = a.tw + (size_t)m * Nn;
+  constexpr int NSL = ntt_round_slots(SB - 4);
+  const uint4* twr = a.twr + (((size_t)m * H::R + r) * NSL) * PB + j;
+  u64* scol = sm + swz(c);
+  u64* srow = sm + r * CP;
+  u64 v[16];
+  if (FWD) {
+    {
+      RoundTw<4> T;
+      round_tw_load<true, 4>(T, 0, SA - 4 + SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = in[(jc + PA * i) * C + c];
+      ntt_round<true, 4>(v, T, q);
+#pragma unroll
+      for (int i = 0; i < 16; i++) scol[(jc + PA * i) * CP] = v[i];
+    }
+    __syncthreads();
+    {
+      RoundTw<SA - 4> T;
+      round_tw_load<true, SA - 4>(T, (u64)(16 * jc) << SB, SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = scol[(16 * jc + i) * CP];
+      ntt_round<true, SA - 4>(v, T, q);
+#pragma unroll
+      for (int i = 0; i < 16; i++) scol[(16 * jc + i) * CP] = v[i];
+    }
+    __syncthreads();
+    {
+      RoundTw<4> T;
+      round_tw_load<true, 4>(T, (u64)r * C, SB - 4, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = srow[swz(j + PB * i)];
+      ntt_round<true, 4>(v, T, q);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(j + PB * i)] = v[i];
+    }
+    wave_lds_sync();
+    {
+      RoundTw<SB - 4> T;
+      round_tw_load_tab<SB - 4>(T, twr, PB);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = srow[swz(16 * j + i)];
+      ntt_round<true, SB - 4>(v, T, q);
+      const u64 q2 = q + q;
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(16 * j + i)] = csub(csub(csub(v[i], q2 + q2), q2), q);
+    }
+    wave_lds_sync();
+    row_fwd_tail<SB, EPI>(a, srow, lr, r, j, poly + (size_t)r * C);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 16; i++) v[i] = in[r * C + j + PB * i];
+#pragma unroll
+    for (int i = 0; i < 16; i++) srow[swz(j + PB * i)] = v[i];
+    wave_lds_sync();
+    {
+      RoundTw<SB - 4> T;
+      round_tw_load_tab<SB - 4>(T, twr, PB);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = srow[swz(16 * j + i)];
+      ntt_round<false, SB - 4>(v, T, q);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(16 * j + i)] = v[i];
+    }
+    wave_lds_sync();
+    {
+      RoundTw<4> T;
+      round_tw_load<false, 4>(T, (u64)r * C, SB - 4, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = srow[swz(j + PB * i)];
+      ntt_round<false, 4>(v, T, q);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(j + PB * i)] = v[i];
+    }
+    __syncthreads();
+    {
+      RoundTw<SA - 4> T;
+      round_tw_load<false, SA - 4>(T, (u64)(16 * jc) << SB, SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = scol[(16 * jc + i) * CP];
+      ntt_round<false, SA - 4>(v, T, q);
+#pragma unroll
+      for (int i = 0; i < 16; i++) scol[(16 * jc + i) * CP] = v[i];
+    }
+    __syncthreads();
+    {
+      RoundTw<4> T;
+      round_tw_load<false, 4>(T, 0, SA - 4 + SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = scol[(jc + PA * i) * CP];
+      ntt_round<false, 4>(v, T, q);
+      const u64 ni = a.ninv[m], nip = a.ninvp[m];
+#pragma unroll
+      for (int i = 0; i < 16; i++) poly[(jc + PA * i) * C + c] = csub(shoup_lazy(v[i], ni, nip, 0 - q), q);
+    }
+  }
+}
+template <bool FWD, int LOGN, bool EPI>
+__device__ __forceinline__ void ntt_lds_fp(const NttArgs& a, u64* sm, const LimbRef& lr) {
+  typedef LdsShape<LOGN> H;
+  constexpr int SA = H::SA, SB = H::SB, PA = H::PA, PB = H::PB, C = H::C, CP = H::CP;
+  const int tid = threadIdx.x, m = lr.mod;
+  const int c = tid & (C - 1), jc = tid >> SB;
+  const int j = tid & (PB - 1), r = tid >> (SB - 4);
+  const FpC fc = a.fpc[m];
+  constexpr u64 Nn = 1ull << LOGN;
+  u64* poly = a.data + lr.off;
+  const u64* in = a.src + limb_src_off(a, lr);
+  const uint4* tw = a.tw + (size_t)m * Nn;
+  constexpr int NSL = ntt_round_slots(SB - 4);
+  const uint4* twr = a.twr + (((size_t)m * H::R + r) * NSL) * PB + j;
+  u64* scol = sm + swz(c);
+  u64* srow = sm + r * CP;
+  double v[16];
+  if (FWD) {
+    static_assert(fpb::ct_pass_ok(false, SA, true) && fpb::ct_pass_ok(false, SB, false), "float64 forward transform out of bounds");
+    constexpr bool A1 = fpb::ct_pass(false, SA, true, 0, true), A2 = fpb::ct_pass(false, SA, true, 1, true);
+    constexpr bool B1 = fpb::ct_pass(false, SB, false, 0, true), B2 = fpb::ct_pass(false, SB, false, 1, true);
+    {
+      RoundTw<4> T;
+      round_tw_load<true, 4>(T, 0, SA - 4 + SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_in(in[(jc + PA * i) * C + c]);
+      f_round_fwd<4, 16, A1>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) scol[(jc + PA * i) * CP] = f_bits(v[i]);
+    }
+    __syncthreads();
+    {
+      RoundTw<SA - 4> T;
+      round_tw_load<true, SA - 4>(T, (u64)(16 * jc) << SB, SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_val(scol[(16 * jc + i) * CP]);
+      f_round_fwd<SA - 4, 16, A2>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) scol[(16 * jc + i) * CP] = f_bits(v[i]);
+    }
+    __syncthreads();
+    {
+      RoundTw<4> T;
+      round_tw_load<true, 4>(T, (u64)r * C, SB - 4, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_val(srow[swz(j + PB * i)]);
+      f_round_fwd<4, 16, B1>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(j + PB * i)] = f_bits(v[i]);
+    }
+    wave_lds_sync();
+    {
+      RoundTw<SB - 4> T;
+      round_tw_load_tab<SB - 4>(T, twr, PB);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_val(srow[swz(16 * j + i)]);
+      f_round_fwd<SB - 4, 16, B2>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(16 * j + i)] = f_canon(v[i], fc);
+    }
+    wave_lds_sync();
+    row_fwd_tail<SB, EPI>(a, srow, lr, r, j, poly + (size_t)r * C);
+  } else {
+    static_assert(fpb::gs_pass_ok(false, SB, true) && fpb::gs_pass_ok(false, SA, false), "float64 inverse transform out of bounds");
+    constexpr long B0 = fpb::gs_pass(false, SB, true, 0), B1 = fpb::gs_pass(false, SB, true, 1);
+    constexpr long A0 = fpb::gs_pass(false, SA, false, 0), A1 = fpb::gs_pass(false, SA, false, 1);
+    u64 w[16];
+#pragma unroll
+    for (int i = 0; i < 16; i++) w[i] = in[r * C + j + PB * i];
+#pragma unroll
+    for (int i = 0; i < 16; i++) srow[swz(j + PB * i)] = w[i];
+    wave_lds_sync();
+    {
+      RoundTw<SB - 4> T;
+      round_tw_load_tab<SB - 4>(T, twr, PB);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_in(srow[swz(16 * j + i)]);
+      f_round_inv<SB - 4, 16, B0, false>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(16 * j + i)] = f_bits(v[i]);
+    }
+    wave_lds_sync();
+    {
+      RoundTw<4> T;
+      round_tw_load<false, 4>(T, (u64)r * C, SB - 4, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_val(srow[swz(j + PB * i)]);
+      f_round_inv<4, 16, B1, false>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) srow[swz(j + PB * i)] = f_bits(v[i]);
+    }
+    __syncthreads();
+    {
+      RoundTw<SA - 4> T;
+      round_tw_load<false, SA - 4>(T, (u64)(16 * jc) << SB, SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_val(scol[(16 * jc + i) * CP]);
+      f_round_inv<SA - 4, 16, A0, false>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) scol[(16 * jc + i) * CP] = f_bits(v[i]);
+    }
+    __syncthreads();
+    {
+      RoundTw<4> T;
+      round_tw_load<false, 4>(T, 0, SA - 4 + SB, Nn, tw);
+#pragma unroll
+      for (int i = 0; i < 16; i++) v[i] = f_val(scol[(jc + PA * i) * CP]);
+      f_round_inv<4, 16, A1, true>(v, [&](int, int, int sl) { return T.t[sl]; }, fc);
+#pragma unroll
+      for (int i = 0; i < 16; i++) poly[(jc + PA * i) * C + c] = f_canon(v[i], fc);
+    }
+  }
+}
+template <bool FWD, int LOGN, bool EPI>
+__global__ __launch_bounds__(1 << (LOGN - 4)) void ntt_lds_kernel(NttArgs a) {
+  __shared__ u64 sm[LdsShape<LOGN>::R * LdsShape<LOGN>::CP];
+  const LimbRef lr = limb_ref(a, blockIdx.x);
+  if (a.mods[lr.mod].q <= FP_QMAX) ntt_lds_fp<FWD, LOGN, EPI>(a, sm, lr);
+  else ntt_lds_int<FWD, LOGN, EPI>(a, sm, lr);
+}
+template <int LOGN>
+void launch_lds(bool forward, int nlimbs, const NttArgs& a, hipStream_t st) {
+  const dim3 grid(nlimbs), block(1 << (LOGN - 4));
+  if (!forward) hipLaunchKernelGGL((ntt_lds_kernel<false, LOGN, false>), grid, block, 0, st, a);
+  else if (a.epi) hipLaunchKernelGGL((ntt_lds_kernel<true, LOGN, true>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((ntt_lds_kernel<true, LOGN, false>), grid, block, 0, st, a);
+}
+
 template <bool FWD>
 void launch_col(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st) {
   switch (S) {
-    case 5: hipLaunchKernelGGL((ntt_col_kernel<FWD, 5>), grid, block, 0, st, a); break;
     case 6: hipLaunchKernelGGL((ntt_col_kernel<FWD, 6>), grid, block, 0, st, a); break;
     case 7: hipLaunchKernelGGL((ntt_col_kernel<FWD, 7>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((ntt_col_kernel<FWD, 8>), grid, block, 0, st, a); break;
@@ -1039,8 +1290,6 @@ void launch_col(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st) 
 template <bool FWD, bool EPI>
 void launch_row_t(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st) {
   switch (S) {
-    case 5: hipLaunchKernelGGL((ntt_row_kernel<FWD, 5, EPI>), grid, block, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((ntt_row_kernel<FWD, 6, EPI>), grid, block, 0, st, a); break;
     case 7: hipLaunchKernelGGL((ntt_row_kernel<FWD, 7, EPI>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((ntt_row_kernel<FWD, 8, EPI>), grid, block, 0, st, a); break;
   }
@@ -1053,7 +1302,6 @@ void launch_row(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st) 
 template <bool FWD>
 void launch_col8(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st) {
   switch (S) {
-    case 5: hipLaunchKernelGGL((ntt_col8_kernel<FWD, 5>), grid, block, 0, st, a); break;
     case 6: hipLaunchKernelGGL((ntt_col8_kernel<FWD, 6>), grid, block, 0, st, a); break;
     case 7: hipLaunchKernelGGL((ntt_col8_kernel<FWD, 7>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((ntt_col8_kernel<FWD, 8>), grid, block, 0, st, a); break;
@@ -1062,7 +1310,6 @@ void launch_col8(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st)
 template <bool FWD, bool EPI>
 void launch_row8_t(int S, dim3 grid, dim3 block, const NttArgs& a, hipStream_t st) {
   switch (S) {
-    case 5: hipLaunchKernelGGL((ntt_row8_kernel<FWD, 5, EPI>), grid, block, 0, st, a); break;
     case 6: hipLaunchKernelGGL((ntt_row8_kernel<FWD, 6, EPI>), grid, block, 0, st, a); break;
     case 7: hipLaunchKernelGGL((ntt_row8_kernel<FWD, 7, EPI>), grid, block, 0, st, a); break;
     default: hipLaunchKernelGGL((ntt_row8_kernel<FWD, 8, EPI>), grid, block, 0, st, a); break;
@@ -1108,10 +1355,32 @@ void launch_ntt(u64* data, size_t bstride, int batch, RowMap rm, int logN, bool 
 // special modulus: a rotation 55 -> 46 us, a whole one-table lookup 456 -> 405
 // us; a bound of 512 measures the same, and N = 2^16 always has more.
 constexpr int W8_FILL = 256;
+// Whether a launch takes the one-workgroup transform: N up to 2^11 always;
+// above, launches of at least 2^(logN - 6) limbs that the 16-word kernels would
+// take.  A limb on one CU takes longer than on several (its integer
+// butterflies alone 8 us at N = 2^13), a full chip half the memory traffic and
+// one launch.  Measured, one limb of eight on the integer path, us a transform
+// in two passes / in one workgroup: N = 2^10 9.6 / 7.4 (32 limbs); 2^12 10.5 /
+// 9.7 (96), 31.0 / 19.0 (1024); 2^13 13.1 / 15.0 (96), 15.9 / 15.2 (128),
+// 59.9 / 35.7 (1024); 2^14 25.1 / 27.9 (192), 32.8 / 28.8 (256), 109.9 / 78.3
+// (1024).
+static bool lds_transform(int logN, int nlimbs) {
+  return logN <= 11 || (logN <= 14 && nlimbs > NTT_W8_MAX_LIMBS && nlimbs >= 1 << (logN - 6));
+}
 static void ntt_launch(NttArgs a, int nlimbs, bool forward, hipStream_t st) {
   int SA, SB;
   ntt_split(a.logN, &SA, &SB);
   a.SA = SA; a.SB = SB;
+  if (lds_transform(a.logN, nlimbs)) {
+    switch (a.logN) {
+      case 10: launch_lds<10>(forward, nlimbs, a, st); break;
+      case 11: launch_lds<11>(forward, nlimbs, a, st); break;
+      case 12: launch_lds<12>(forward, nlimbs, a, st); break;
+      case 13: launch_lds<13>(forward, nlimbs, a, st); break;
+      default: launch_lds<14>(forward, nlimbs, a, st); break;
+    }
+    return;
+  }
   if (nlimbs <= NTT_W8_MAX_LIMBS) {
     const int TA = 1 << (SA - 3), TB = 1 << (SB - 3), C = 1 << SB, R = 1 << SA;
     int nsubA = std::min(512 / TA, C), nsubB = std::min(256 / TB, R);

@@ -43,6 +43,11 @@ struct RowMap {
 
 
 #if defined(__HIP_DEVICE_COMPILE__) || defined(__HIPCC__)
+// Words of a table that no kernel writes, at a wave-uniform index: read
+// through the constant address space they are scalar loads also in a kernel
+// that has stored before (where the compiler falls back to vector loads).
+typedef const u64 __attribute__((address_space(4)))* cwords;
+__device__ __forceinline__ cwords const_words(const void* p) { return (cwords)(uintptr_t)p; }
 __device__ __forceinline__ u64 add_mod(u64 a, u64 b, u64 q) { u64 r = a + b; return r >= q ? r - q : r; }
 __device__ __forceinline__ u64 sub_mod(u64 a, u64 b, u64 q) { return a >= b ? a - b : a + q - b; }
 __device__ __forceinline__ u64 shoup_mul(u64 x, u64 w, u64 wp, u64 q) {
@@ -245,8 +250,8 @@ __device__ __forceinline__ u64 acc61_redc(const Acc61& A, u64 q, u64 qinv) {
 // read for all 8 i: the table holds spare words past its last row), v <= 8
 // the overflow count: the sum is at most (2^64 - 8)(q - 1) + 8 (q - 1), so
 // below q * 2^64 as the REDC needs.
-template <class Y>
-__device__ __forceinline__ u64 bconv_word8(Y y, const u64* __restrict__ h, uint32_t v, u64 n, u64 q, u64 qinv) {
+template <class Y, class H>
+__device__ __forceinline__ u64 bconv_word8(Y y, H h, uint32_t v, u64 n, u64 q, u64 qinv) {
   Acc61 A;
 #pragma unroll
   for (int i = 0; i < 8; i++) {

@@ -6,6 +6,7 @@
 #include "hipckks.h"
 #include "kernels.h"
 #include <algorithm>
+#include <cstddef>
 
 // High word of a 128-bit sum of products of words < q < 2^62: after at most
 // 16 products (plus one earlier fold) it is below 5q; bring it below q.
@@ -352,6 +353,11 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
   }
 }
 
+static_assert(sizeof(BConvSrc) == 32 && offsetof(BConvTable, hat) == 32 * HCK_MAXSRC && offsetof(BConvTable, nS) == 32 * HCK_MAXSRC + 8 &&
+                  sizeof(ModC) == 32 && offsetof(ModC, qinv) == 8, "tables read by word");
+__device__ __forceinline__ BConvSrc bconv_src(cwords tab, int i) {
+  return BConvSrc{tab[4 * i], tab[4 * i + 1], tab[4 * i + 2], __longlong_as_double((long long)tab[4 * i + 3])};
+}
 // From one key switch's product to the next one's digits (LinkArgs).  The
 // ModDown of the first, the automorphism's sum and the ModUp of the second
 // are all coefficient-wise, so one launch does them without a transform in
@@ -361,10 +367,11 @@ __global__ __launch_bounds__(256) void bconv_lds_kernel(const u64* __restrict__ 
 // eleven.  VALU-bound as the basis extensions it is made of (2 (l+1) + dn nqp
 // rows of 8 products a coefficient).  Shape as bconv_lds_kernel: 64
 // coefficients a workgroup, four waves; a wave computes every fourth row and
-// the rows' source terms meet in LDS.  At N = 2^16 with 23 Q and 8 P rows it
-// takes 43 us where the two extensions took 38 and the transforms between
-// them 46; a fold step goes from 190 to 161 us (11 steps at 11 Q rows: 134 to
-// 100 us a step).
+// the rows' source terms meet in LDS.  Its tables are read as constant words:
+// behind its own stores the compiler read them as 90 vector loads a wave, a
+// memory round trip a row (22.7 -> 20.4 us at 11 Q rows).  A fold step of 23 Q
+// and 8 P rows at N = 2^16 takes 161 us with it against 190 with the two
+// extensions and the transforms between them.
 __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   extern __shared__ u64 sm[];
   const int lane = threadIdx.x & (BCL_X - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / BCL_X);
@@ -377,13 +384,15 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   const bool flip = ((uint32_t)x * a.ginv & (uint32_t)(2 * N - 1)) >= (uint32_t)N;
   // LDS: source terms (P rows: y and y / p of both polynomials, 8 slots each;
   // then the Q rows' y and y / q)
-  const BConvTable* __restrict__ pt = a.ptab;
+  const cwords pt = const_words(a.ptab);  // BConvTable: 4 words a source, then the pointers hat and nS
+  const cwords phat = const_words((const void*)pt[4 * HCK_MAXSRC]), pnS = const_words((const void*)pt[4 * HCK_MAXSRC + 1]);
+  const cwords mods = const_words(a.mods), pinv = const_words(a.pinv), pinvp = const_words(a.pinvp);
   for (int part = two ? 0 : 1; part < 2; part++) {
     const u64* src = part ? x1 + (size_t)nq * N : a.x0p + x;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const int i = w + 4 * k;
-      const BConvSrc s = pt->src[i];
+      const BConvSrc s = bconv_src(pt, i);
       const bool act = i < K;
       u64 yi = shoup_mul(src[(size_t)(act ? i : 0) * N], s.hinv, s.hinvp, s.q);
       if (flip && yi) yi = s.q - yi;
@@ -409,32 +418,33 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   // a row's words are loaded while the row before it is computed
   u64 zn = w < nq ? x1[(size_t)w * N] : 0, cn = a.acc && w < nq ? c1[(size_t)w * N] : 0;
   for (int r = w; r < nq; r += 4) {
-    const ModC mc = a.mods[r];
-    const u64* __restrict__ h = pt->hat + (size_t)r * K;
-    const u64 pi = a.pinv[r], pip = a.pinvp[r], n = pt->nS[r];
+    const u64 q = mods[4 * r], qinv = mods[4 * r + 1];
+    const cwords h = phat + (size_t)r * K;
+    const u64 pi = pinv[r], pip = pinvp[r], n = pnS[r];
     const u64 z = zn, c = cn;
     const int rn = min(r + 4, nq - 1);
     zn = x1[(size_t)rn * N];
     if (a.acc) cn = c1[(size_t)rn * N];
-    const u64 e1 = bconv_word8([&](int i) { return y1[i]; }, h, v1, n, mc.q, mc.qinv);
-    const u64 m = shoup_mul(flip ? add_mod(z, e1, mc.q) : sub_mod(z, e1, mc.q), pi, pip, mc.q);
-    const u64 s = add_mod(c, m, mc.q);
+    const u64 e1 = bconv_word8([&](int i) { return y1[i]; }, h, v1, n, q, qinv);
+    const u64 m = shoup_mul(flip ? add_mod(z, e1, q) : sub_mod(z, e1, q), pi, pip, q);
+    const u64 s = add_mod(c, m, q);
     c1[(size_t)r * N] = s;
-    const BConvSrc sd = a.dtab[r / K]->src[r % K];
+    const BConvSrc sd = bconv_src(const_words(a.dtab[r / K]), r % K);
     const u64 yi = shoup_mul(s, sd.hinv, sd.hinvp, sd.q);
     sm[r * BCL_X + lane] = yi;
     sm[(nq + r) * BCL_X + lane] = (u64)__double_as_longlong((double)yi / sd.qd);
     if (two) {
-      u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, v0, n, mc.q, mc.qinv);
-      e0 = shoup_mul(e0, pi, pip, mc.q);
-      a.e0[(size_t)r * N + x] = flip || e0 == 0 ? e0 : mc.q - e0;
+      u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, v0, n, q, qinv);
+      e0 = shoup_mul(e0, pi, pip, q);
+      a.e0[(size_t)r * N + x] = flip || e0 == 0 ? e0 : q - e0;
     }
   }
   __syncthreads();
   int first = w;  // this wave's first row of the digit: rows are dealt round robin over all digits
   for (int d = 0; d < a.dn; d++) {
     const int st0 = d * K, ns = min(st0 + K, nq) - st0, nrows = nqp - ns;
-    const BConvTable* __restrict__ dt = a.dtab[d];
+    const cwords dt = const_words(a.dtab[d]);
+    const cwords dhat = const_words((const void*)dt[4 * HCK_MAXSRC]), dnS = const_words((const void*)dt[4 * HCK_MAXSRC + 1]);
     u64 y[8];
     double vf = 0.0;
 #pragma unroll
@@ -450,10 +460,8 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
     for (; rr < nrows; rr += 4) {
       const int row = rr < st0 ? rr : rr + ns;
       const int m = row < nq ? row : a.L + row - nq;
-      const ModC mc = a.mods[m];
-      const u64* __restrict__ h = dt->hat + (size_t)m * ns;
       digits[((size_t)d * nqp + row) * N] =
-          bconv_word8([&](int i) { return y[i]; }, h, v, dt->nS[m], mc.q, mc.qinv);
+          bconv_word8([&](int i) { return y[i]; }, dhat + (size_t)m * ns, v, dnS[m], mods[4 * m], mods[4 * m + 1]);
     }
     first = rr - nrows;
   }

@@ -35,10 +35,10 @@ struct FftArgs {
   const int* rotgroup;
   const double *rre, *rim;
   // inverse: the column pass reads element k of plaintext p from
-  // data[src * n + ((k + rot) mod n)], or 0 past nvals; complex input: (re, im)
+  // data[src * n + ((k + rot) mod n)], or 0 from nvals on; complex input: (re, im)
   // pairs at data[2k], data[2k + 1]
   const float* data;
-  const EncodeSrc* src;
+  const EncodeSrc* src;  // nullptr: one plaintext, source 0 unrotated
   int nvals, complex_in;
   // forward: the column pass writes the real parts as float (mode 0) or double
   // (1), or (re, im) pairs of float (2)
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void fft_col_kernel(FftArgs a) {
         v = (double)a.data[2 * (size_t)k];
         vi = (double)a.data[2 * (size_t)k + 1];
       } else {
-        const EncodeSrc s = a.src[blockIdx.y];
+        const EncodeSrc s = a.src ? a.src[blockIdx.y] : EncodeSrc{0, 0};
         v = (double)a.data[(size_t)s.src * a.n + ((k + s.rot) & (a.n - 1))];
       }
     }
@@ -306,12 +306,17 @@ void launch_decode_fft(const DecodeArgs& d, int words, const int* rotgroup, cons
                        int mode, hipStream_t st) {
   const int n = d.N / 2;
   const dim3 grid(d.N / 256), block(256);
-  if (words <= 4) hipLaunchKernelGGL(decode_crt_kernel<4>, grid, block, 0, st, d);
-  else if (words <= 8) hipLaunchKernelGGL(decode_crt_kernel<8>, grid, block, 0, st, d);
-  else if (words <= 16) hipLaunchKernelGGL(decode_crt_kernel<16>, grid, block, 0, st, d);
-  else if (words <= 24) hipLaunchKernelGGL(decode_crt_kernel<24>, grid, block, 0, st, d);
-  else if (words <= 32) hipLaunchKernelGGL(decode_crt_kernel<32>, grid, block, 0, st, d);
-  else hipLaunchKernelGGL(decode_crt_kernel<DECODE_MAXW>, grid, block, 0, st, d);
+  switch (words) {
+    case 4: hipLaunchKernelGGL(decode_crt_kernel<4>, grid, block, 0, st, d); break;
+    case 8: hipLaunchKernelGGL(decode_crt_kernel<8>, grid, block, 0, st, d); break;
+    case 12: hipLaunchKernelGGL(decode_crt_kernel<12>, grid, block, 0, st, d); break;
+    case 16: hipLaunchKernelGGL(decode_crt_kernel<16>, grid, block, 0, st, d); break;
+    case 20: hipLaunchKernelGGL(decode_crt_kernel<20>, grid, block, 0, st, d); break;
+    case 24: hipLaunchKernelGGL(decode_crt_kernel<24>, grid, block, 0, st, d); break;
+    case 28: hipLaunchKernelGGL(decode_crt_kernel<28>, grid, block, 0, st, d); break;
+    case 32: hipLaunchKernelGGL(decode_crt_kernel<32>, grid, block, 0, st, d); break;
+    default: hipLaunchKernelGGL(decode_crt_kernel<DECODE_MAXW>, grid, block, 0, st, d); break;
+  }
   const FftArgs f{d.re, d.im, 0, n, 2 * d.N, rotgroup, rre, rim, nullptr, nullptr, 0, 0, out, mode};
   hipLaunchKernelGGL(fft_block_kernel<false>, dim3(n / FFT_B), dim3(FFT_B / 2), 0, st, f);
   hipLaunchKernelGGL(fft_col_kernel<false>, dim3(FFT_B / FFT_CW), dim3(256), 0, st, f);

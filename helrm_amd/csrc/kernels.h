@@ -216,7 +216,7 @@ void launch_mul_const_v(u64* out, const u64* in, size_t bstride, int batch, RowM
 // out = in +- c.w[modulus] on the rows of rm (one polynomial)
 void launch_add_scalar_v(u64* out, const u64* in, RowMap rm, const RowConst& c, const ModC* mods, int N, bool sub,
                          hipStream_t st);
-void launch_mont_mul(u64* out, size_t obstride, const u64* a, size_t abstride, const u64* bR, size_t bbstride, int batch, RowMap rm, const ModC* mods, int N, bool acc, hipStream_t st);
+void launch_mont_mul(u64* out, size_t obstride, const u64* a, size_t abstride, const u64* bR, size_t bbstride, int batch, RowMap rm, const ModC* mods, int N, const u64* add, hipStream_t st);
 void launch_mont_convert(u64* data, size_t bstride, int batch, RowMap rm, const ModC* mods, int N, bool to, hipStream_t st);
 // Basis extension of the ns source rows of `in` into the target rows rm of `out`.
 // One source group of a batched basis extension (e.g. one digit of a
@@ -265,7 +265,23 @@ void launch_moddown_rescale_spread(u64* ext, size_t e_bstride, const u64* xl, si
 void launch_sample_uniform(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, hipStream_t st);
 void launch_sample_cbd(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, bool add, hipStream_t st);
 void launch_signed_rows(u64* out, RowMap rm, const int8_t* v, const ModC* mods, int N, hipStream_t st);
+// positions small enough to travel in the kernel arguments
+struct TernaryPos {
+  uint32_t p[256];
+  __host__ __device__ uint32_t operator[](int i) const { return p[i]; }
+};
 void launch_ternary_rows(u64* out, RowMap rm, const uint32_t* pos, int npos, const ModC* mods, int N, hipStream_t st);
+void launch_ternary_rows(u64* out, RowMap rm, const TernaryPos& pos, int npos, const ModC* mods, int N, hipStream_t st);
+// x: [2][l + 2][N] coefficients (rows q_0..q_l, p_0), out: [2][l + 1][N]
+struct EncryptDownArgs {
+  const u64* x; size_t x_bstride;
+  u64* out;
+  const ModC* mods;
+  const u64 *p0inv, *p0invp;  // [mod] p_0^-1 mod q and its Shoup companion
+  u64 seed, stream[2];
+  int N, l, mp;               // mp: index of p_0
+};
+void launch_encrypt_down(const EncryptDownArgs& a, hipStream_t st);
 void launch_gk_combine(u64* b, const u64* a, const u64* soR, const u64* sR, int own0, int own1, const u64* pmod, int rows, const ModC* mods, int N, hipStream_t st);
 // Device encoder (encoder.hip): plaintext p of a batch takes element k from
 // data[src * slots + ((k + rot) mod slots)] (zero past nvals), runs the special
@@ -278,7 +294,7 @@ void launch_encode_fft(u64* out, size_t out_pstride, RowMap rm, const float* dat
                        const double* rim, const ModC* mods, int logN, hipStream_t st, bool complex_in = false);
 // Device decoder: coefficients coef[nl][N] (rows q_0 .. q_{nl-1}), tables of the
 // level: src[i] (hinv of Q / q_i), hat [nl][W] words of Q / q_i, then Q and
-// floor(Q / 2); W the first of 4, 8, 16, 24, 32, DECODE_MAXW not below `words`
+// floor(Q / 2); W the multiple of 4 up to 32 that is not below `words`, or DECODE_MAXW
 // (words of 2^8 Q; decode_words).  re / im are work buffers of N / 2 doubles;
 // out takes the slots' real parts as float (mode 0) or double (1), or (re, im)
 // pairs of float (2).
@@ -291,10 +307,7 @@ struct DecodeArgs {
   double scale;
   double *re, *im;
 };
-inline int decode_words(int words) {
-  for (int w : {4, 8, 16, 24, 32}) if (words <= w) return w;
-  return DECODE_MAXW;
-}
+inline int decode_words(int words) { return words <= 32 ? (words + 3) / 4 * 4 : DECODE_MAXW; }
 void launch_decode_fft(const DecodeArgs& d, int words, const int* rotgroup, const double* rre, const double* rim, void* out,
                        int mode, hipStream_t st);
 // multiplication by the imaginary unit (the monomial X^(N/2)) in the NTT domain:

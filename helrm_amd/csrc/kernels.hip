@@ -138,21 +138,21 @@ void launch_tensor(u64* d0, u64* d1, u64* d2, const u64* a0, const u64* a1, cons
   hipLaunchKernelGGL(tensor_kernel, dim3(N / 256, l + 1, 1), dim3(256), 0, st, d0, d1, d2, a0, a1, b0, b1, pw, pwp, mods, N);
 }
 
-// out = a * bR * R^-1 (b stored in Montgomery form); optional accumulate
-__global__ void mont_mul_kernel(u64* __restrict__ out, const u64* __restrict__ a, size_t abstride,
+// out = a * bR * R^-1 (b stored in Montgomery form), plus add (at out's stride) if given
+__global__ void mont_mul_kernel(u64* out, const u64* __restrict__ a, size_t abstride,
                                 const u64* __restrict__ bR, size_t bbstride, size_t obstride, RowMap rm,
-                                const ModC* __restrict__ mods, int N, int acc) {
+                                const ModC* __restrict__ mods, int N, const u64* add) {
   int x = blockIdx.x * blockDim.x + threadIdx.x;
   int row = rm.row(blockIdx.y);
   ModC mc = mods[rm.mod(row)];
   u64 r = mont_mul(a[(size_t)blockIdx.z * abstride + (size_t)row * N + x], bR[(size_t)blockIdx.z * bbstride + (size_t)row * N + x], mc.q, mc.qinv);
   size_t o = (size_t)blockIdx.z * obstride + (size_t)row * N + x;
-  out[o] = acc ? add_mod(out[o], r, mc.q) : r;
+  out[o] = add ? add_mod(add[o], r, mc.q) : r;
 }
 void launch_mont_mul(u64* out, size_t obstride, const u64* a, size_t abstride, const u64* bR, size_t bbstride, int batch,
-                     RowMap rm, const ModC* mods, int N, bool acc, hipStream_t st) {
+                     RowMap rm, const ModC* mods, int N, const u64* add, hipStream_t st) {
   if (rm.nact() <= 0 || batch <= 0) return;
-  hipLaunchKernelGGL(mont_mul_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, a, abstride, bR, bbstride, obstride, rm, mods, N, acc ? 1 : 0);
+  hipLaunchKernelGGL(mont_mul_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, a, abstride, bR, bbstride, obstride, rm, mods, N, add);
 }
 
 // out[row] = in[row] +- c.w[modulus of row] (a constant in every NTT slot)
@@ -1164,16 +1164,19 @@ void launch_signed_rows(u64* out, RowMap rm, const int8_t* v, const ModC* mods, 
 }
 // The polynomial with coefficient +1 at pos[i] / 2 for even pos[i], -1 for odd
 // ones (distinct places) and 0 elsewhere, reduced into every row: 1024
-// coefficients of a row a workgroup, gathered in LDS.
-__global__ __launch_bounds__(256) void ternary_rows_kernel(u64* __restrict__ out, RowMap rm, const uint32_t* __restrict__ pos,
-                                                          int npos, const ModC* __restrict__ mods, int N) {
+// coefficients of a row a workgroup, gathered in LDS.  The positions come with
+// the arguments (POS, an array of them) or from memory.
+template <class POS>
+__global__ __launch_bounds__(256) void ternary_rows_kernel(u64* __restrict__ out, RowMap rm, POS pos, int npos,
+                                                          const ModC* __restrict__ mods, int N) {
   __shared__ int v[1024];
   const int base = blockIdx.x * 1024;
   for (int i = threadIdx.x; i < 1024; i += 256) v[i] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < npos; i += 256) {
-    const int x = (int)(pos[i] >> 1) - base;
-    if (x >= 0 && x < 1024) v[x] = pos[i] & 1 ? -1 : 1;
+    const uint32_t p = pos[i];
+    const int x = (int)(p >> 1) - base;
+    if (x >= 0 && x < 1024) v[x] = p & 1 ? -1 : 1;
   }
   __syncthreads();
   const int row = rm.row(blockIdx.y);
@@ -1181,7 +1184,41 @@ __global__ __launch_bounds__(256) void ternary_rows_kernel(u64* __restrict__ out
   for (int i = threadIdx.x; i < 1024; i += 256) out[(size_t)row * N + base + i] = v[i] < 0 ? q - 1 : (u64)v[i];
 }
 void launch_ternary_rows(u64* out, RowMap rm, const uint32_t* pos, int npos, const ModC* mods, int N, hipStream_t st) {
-  hipLaunchKernelGGL(ternary_rows_kernel, dim3(N / 1024, rm.nact(), 1), dim3(256), 0, st, out, rm, pos, npos, mods, N);
+  hipLaunchKernelGGL(ternary_rows_kernel<const uint32_t*>, dim3(N / 1024, rm.nact(), 1), dim3(256), 0, st, out, rm, pos, npos,
+                     mods, N);
+}
+void launch_ternary_rows(u64* out, RowMap rm, const TernaryPos& pos, int npos, const ModC* mods, int N, hipStream_t st) {
+  hipLaunchKernelGGL(ternary_rows_kernel<TernaryPos>, dim3(N / 1024, rm.nact(), 1), dim3(256), 0, st, out, rm, pos, npos, mods,
+                     N);
+}
+// The coefficients of a fresh encryption: part b of x = pk u, with rows
+// q_0..q_l and p_0, plus its error e, divided by p_0 (Lattigo's ModDown from
+// Q + {p_0}):
+//   out_i = (x_i + e - ext_i) / p_0 mod q_i,  ext = x_{p_0} + e extended to q_i:
+// one source, so y = x_{p_0} + e itself, less p_0 where its overflow count
+// (u64)((double)y / (double)p_0) rounds to one.  One pass instead of two error
+// launches, the extension and the combination, 45 us of 25 rows at N = 2^16;
+// a thread takes every gridDim.y-th row, so that a coefficient's error and y
+// are drawn a few times and not once a row.
+__global__ __launch_bounds__(256) void encrypt_down_kernel(EncryptDownArgs a) {
+  const int x = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.z, N = a.N, nq = a.l + 1;
+  const u64* in = a.x + (size_t)b * a.x_bstride + x;
+  u64* out = a.out + (size_t)b * nq * N + x;
+  const u64 p0 = a.mods[a.mp].q;
+  const u64 r = rand64(a.seed, a.stream[b], (u64)x);
+  const int e = __popcll(r & 0x1FFFFFULL) - __popcll((r >> 21) & 0x1FFFFFULL);
+  const u64 y = add_mod(in[(size_t)nq * N], e >= 0 ? (u64)e : p0 - (u64)(-e), p0);
+  const bool over = (u64)((double)y / (double)p0) != 0;
+  for (int i = blockIdx.y; i < nq; i += gridDim.y) {
+    const ModC mc = a.mods[i];
+    const u64 xi = add_mod(in[(size_t)i * N], e >= 0 ? (u64)e : mc.q - (u64)(-e), mc.q);
+    u64 ext = mont_mul(y, mc.rmod, mc.q, mc.qinv);  // y mod q_i
+    if (over) ext = sub_mod(ext, mont_mul(p0, mc.rmod, mc.q, mc.qinv), mc.q);
+    out[(size_t)i * N] = shoup_mul(sub_mod(xi, ext, mc.q), a.p0inv[i], a.p0invp[i], mc.q);
+  }
+}
+void launch_encrypt_down(const EncryptDownArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(encrypt_down_kernel, dim3(a.N / 256, std::min(a.l + 1, 4), 2), dim3(256), 0, st, a);
 }
 // Galois-key body: b = -a*s' + e (+ P*s on own rows), in place on b; a, s', s in
 // (a standard, sR/soR Montgomery), own rows [own0, own1) of the Q chain.

@@ -371,6 +371,7 @@ struct Scheme {
   // EvaluateLinearTransform returns the rescaled result (ModDown and rescale
   // fused), as backends that advertise lt_output_prerescaled do
   bool lt_prerescale = false;
+  DU64 neg1_w, neg1_wp;     // [mod] q - 1, Shoup companion
   DU64 iu, iup, niu, niup;  // [mod] psi^(N/2) (a square root of -1), its negation, Shoup companions
   std::map<std::pair<int, int>, std::unique_ptr<BConvHost>> bconv;
   std::map<u64, DevArray<uint32_t>> perms, perm_invs;
@@ -772,7 +773,7 @@ void ensure_relin_key() {
   REQUIRE(s.dnum <= 16, "key switching needs at most 16 decomposition digits (len(Q) <= 16 * len(P))");
   const int N = s.N, nm = s.L + s.K;
   DU64 s2R((size_t)nm * N);  // s^2 in Montgomery form: mont_mul(sR, sR) = s^2 R
-  launch_mont_mul(s2R.p, 0, s.sR.p, 0, s.sR.p, 0, 1, rows_all(), s.d_mods.p, N, false, s.st);
+  launch_mont_mul(s2R.p, 0, s.sR.p, 0, s.sR.p, 0, 1, rows_all(), s.d_mods.p, N, nullptr, s.st);
   s.rlk = gen_eval_key(s2R.p, s.sR.p, [](int d) { return ST_RLK_A((u64)d); }, [](int d) { return ST_RLK_E((u64)d); });
   s.rlk_seeded = true;
 }
@@ -818,12 +819,13 @@ void encode_device(const float* h_data, size_t ndata, const std::vector<EncodeSr
   DevArray<float> dd(std::max<size_t>(ndata, 1));
   if (ndata) upload(dd.p, h_data, ndata);
   const int np = (int)src.size(), chunk = std::min(np, 64);
-  DevArray<EncodeSrc> ds(np); upload(ds.p, src.data(), np);
+  DevArray<EncodeSrc> ds;
+  if (np != 1 || src[0].src != 0 || src[0].rot != 0) { ds = DevArray<EncodeSrc>(np); upload(ds.p, src.data(), np); }
   DevArray<double> re((size_t)chunk * slots), im((size_t)chunk * slots);
   for (int c0 = 0; c0 < np; c0 += chunk) {
     const int nb = std::min(chunk, np - c0);
     u64* o = chunk_done ? out : out + (size_t)c0 * out_pstride;
-    launch_encode_fft(o, out_pstride, rm, dd.p, ds.p + c0, nb, nvals, scale, re.p, im.p, slots, s.d_rotgroup.p, s.d_rre.p,
+    launch_encode_fft(o, out_pstride, rm, dd.p, ds.p ? ds.p + c0 : nullptr, nb, nvals, scale, re.p, im.p, slots, s.d_rotgroup.p, s.d_rre.p,
                       s.d_rim.p, s.d_mods.p, s.logN, s.st, complex_in);
     ntt(o, out_pstride, nb, rm, true);
     if (chunk_done) chunk_done(c0, nb);
@@ -968,6 +970,9 @@ void build_scheme(int logN, const std::vector<u64>& q, const std::vector<u64>& p
     up(s.tw2, htw); up(s.itw2, hitw); up(s.twr2, htwr); up(s.itwr2, hitwr); up(s.ninv, hn); up(s.ninvp, hnp);
     s.fpc = DevArray<FpC>(nm); upload(s.fpc.p, hfpc.data(), nm);
     s.tw = NttTables{s.d_mods.p, s.tw2.p, s.itw2.p, s.twr2.p, s.itwr2.p, s.ninv.p, s.ninvp.p, s.fpc.p};
+    std::vector<u64> n1(nm), n1p(nm);
+    for (int m = 0; m < nm; m++) { n1[m] = s.mod[m] - 1; n1p[m] = shoup(n1[m], s.mod[m]); }
+    up(s.neg1_w, n1); up(s.neg1_wp, n1p);
     std::vector<u64> pm(nm), pmp(nm), pin(nm), pinp(nm), p0i(nm), p0ip(nm), pmr(nm);
     for (int m = 0; m < nm; m++) {
       u64 qq = s.mod[m], P = 1;
@@ -1286,7 +1291,7 @@ std::unique_ptr<Cipher> mul_plain_ct(const Cipher& ct, const Plain& pt) {
   launch_mont_convert(pR.p, 0, 1, rows_q(l), s.d_mods.p, N, true, s.st);
   auto out = new_ct(l, ct.scale * pt.scale); out->logslots = ct.logslots;
   launch_mont_mul(out->d.p, (size_t)(l + 1) * N, ct.d.p, (size_t)(ct.level + 1) * N, pR.p, 0, 2, rows_q(l), s.d_mods.p, N,
-                  false, s.st);
+                  nullptr, s.st);
   return out;
 }
 // MulRelin(a, b): tensor (a0 b0, a0 b1 + a1 b0, a1 b1) at level min, then the
@@ -1777,17 +1782,17 @@ std::unique_ptr<Cipher> eval_lt_naive(const LinTrans& t, const Cipher& ct) {
     for (int i = 0; i < n; i++) {
       const u64* dp = t.diags.p + (size_t)nz[i] * dstride;
       // the diagonal's P rows sit after its own Q rows (level t.level); multiply Q and P parts separately
-      launch_mont_mul(acc.p, qp, R.p + (size_t)i * 2 * qp, qp, dp, 0, 2, rows_q(l), s.d_mods.p, N, true, s.st);
+      launch_mont_mul(acc.p, qp, R.p + (size_t)i * 2 * qp, qp, dp, 0, 2, rows_q(l), s.d_mods.p, N, acc.p, s.st);
       launch_mont_mul(acc.p + (size_t)(l + 1) * N, qp, R.p + (size_t)i * 2 * qp + (size_t)(l + 1) * N, qp, dp + (size_t)(t.level + 1) * N, 0, 2,
-                      RowMap{K, 0, 0, s.L, 0, 0}, s.d_mods.p, N, true, s.st);
+                      RowMap{K, 0, 0, s.L, 0, 0}, s.d_mods.p, N, acc.p + (size_t)(l + 1) * N, s.st);
     }
   }
   auto out = new_ct(l, ct.scale * t.scale); out->logslots = ct.logslots;
   mod_down(l, acc.p, qp, 2, out->d.p, (size_t)(l + 1) * N);
   if (zero_p >= 0) {
     const u64* dp = t.diags.p + (size_t)zero_p * dstride;
-    launch_mont_mul(out->d.p, (size_t)(l + 1) * N, c0, 0, dp, 0, 1, rows_q(l), s.d_mods.p, N, true, s.st);
-    launch_mont_mul(out->d.p + (size_t)(l + 1) * N, 0, c1, 0, dp, 0, 1, rows_q(l), s.d_mods.p, N, true, s.st);
+    launch_mont_mul(out->d.p, (size_t)(l + 1) * N, c0, 0, dp, 0, 1, rows_q(l), s.d_mods.p, N, out->d.p, s.st);
+    launch_mont_mul(out->d.p + (size_t)(l + 1) * N, 0, c1, 0, dp, 0, 1, rows_q(l), s.d_mods.p, N, out->d.p + (size_t)(l + 1) * N, s.st);
   }
   return out;
 }
@@ -1800,28 +1805,33 @@ std::unique_ptr<Cipher> encrypt_pt(const Plain& pt) {
   REQUIRE(s.has_pk, "public key not generated");
   const int l = pt.level, N = s.N, nm = s.L + s.K, nr = l + 2;
   const u64 enc = s.enc_counter++;
-  std::vector<uint32_t> u = ternary_positions(s.seed, ST_ENC_U(enc), N, s.h);
-  DevArray<uint32_t> du(std::max<size_t>(u.size(), 1)); upload(du.p, u.data(), u.size());
+  const std::vector<uint32_t> u = ternary_positions(s.seed, ST_ENC_U(enc), N, s.h);
   RowMap rm{nr, l + 1, 0, s.L, 0, 0};
   DU64 uq((size_t)nr * N), tt((size_t)2 * nr * N);
-  launch_ternary_rows(uq.p, rm, du.p, (int)u.size(), s.d_mods.p, N, s.st);
+  TernaryPos up;
+  DevArray<uint32_t> du;
+  if (u.size() <= sizeof(up.p) / sizeof(up.p[0])) {
+    std::copy(u.begin(), u.end(), up.p);
+    launch_ternary_rows(uq.p, rm, up, (int)u.size(), s.d_mods.p, N, s.st);
+  } else {
+    du = DevArray<uint32_t>(u.size());
+    upload(du.p, u.data(), u.size());
+    launch_ternary_rows(uq.p, rm, du.p, (int)u.size(), s.d_mods.p, N, s.st);
+  }
   ntt(uq.p, 0, 1, rm, true);
   // pkR holds every modulus: rows q_0..q_l, then row p_0 of it
-  launch_mont_mul(tt.p, (size_t)nr * N, uq.p, 0, s.pkR.p, (size_t)nm * N, 2, rows_q(l), s.d_mods.p, N, false, s.st);
+  launch_mont_mul(tt.p, (size_t)nr * N, uq.p, 0, s.pkR.p, (size_t)nm * N, 2, rows_q(l), s.d_mods.p, N, nullptr, s.st);
   launch_mont_mul(tt.p + (size_t)(l + 1) * N, (size_t)nr * N, uq.p + (size_t)(l + 1) * N, 0, s.pkR.p + (size_t)s.L * N,
-                  (size_t)nm * N, 2, RowMap{1, 0, 0, s.L, 0, 0}, s.d_mods.p, N, false, s.st);
+                  (size_t)nm * N, 2, RowMap{1, 0, 0, s.L, 0, 0}, s.d_mods.p, N, nullptr, s.st);
   ntt(tt.p, (size_t)nr * N, 2, rm, false);
-  launch_sample_cbd(tt.p, rm, s.seed, ST_ENC_E0(enc), s.d_mods.p, N, true, s.st);
-  launch_sample_cbd(tt.p + (size_t)nr * N, rm, s.seed, ST_ENC_E1(enc), s.d_mods.p, N, true, s.st);
-  // ModDown from Q + {p_0} in the coefficient domain
-  DU64 ext((size_t)2 * (l + 1) * N);
-  BConvHost& bt = bconv_table(s.L, s.L + 1);
-  launch_bconv(tt.p + (size_t)(l + 1) * N, (size_t)nr * N, 1, bt.dtab.p, ext.p, (size_t)(l + 1) * N, 2, rows_q(l), s.d_mods.p, N, false, s.st);
+  // errors and ModDown from Q + {p_0} in the coefficient domain, then the
+  // transform, which adds the plaintext to part 0
+  DU64 coef((size_t)2 * (l + 1) * N);
+  launch_encrypt_down(EncryptDownArgs{tt.p, (size_t)nr * N, coef.p, s.d_mods.p, s.p0inv_w.p, s.p0inv_wp.p, s.seed,
+                                      {ST_ENC_E0(enc), ST_ENC_E1(enc)}, N, l, s.L}, s.st);
   auto out = new_ct(l, pt.scale); out->logslots = pt.logslots;
-  launch_moddown_combine(out->d.p, (size_t)(l + 1) * N, tt.p, (size_t)nr * N, ext.p, (size_t)(l + 1) * N, nullptr, 0, 0, nullptr,
-                         s.p0inv_w.p, s.p0inv_wp.p, l + 1, 2, s.d_mods.p, N, s.st);
-  ntt(out->d.p, (size_t)(l + 1) * N, 2, rows_q(l), true);
-  launch_add(out->d.p, out->d.p, pt.d.p, 0, 1, rows_q(l), s.d_mods.p, N, false, s.st);
+  launch_ntt_moddown(coef.p, (size_t)(l + 1) * N, 2, l, s.logN, nullptr, 0, out->d.p, (size_t)(l + 1) * N, pt.d.p, 0, 1, nullptr,
+                     s.neg1_w.p, s.neg1_wp.p, s.tw, s.st, nullptr, 0, 2);
   sync();
   return out;
 }
@@ -1845,7 +1855,7 @@ std::unique_ptr<Cipher> encrypt_seeded(const Plain& pt, u64 seed) {
   launch_sample_cbd(b, rows_q(l), s.seed, ST_SEED_E(enc), s.d_mods.p, N, false, s.st);
   ntt(b, 0, 1, rows_q(l), true);
   DU64 as((size_t)(l + 1) * N);
-  launch_mont_mul(as.p, 0, b + (size_t)(l + 1) * N, 0, s.sR.p, 0, 1, rows_q(l), s.d_mods.p, N, false, s.st);
+  launch_mont_mul(as.p, 0, b + (size_t)(l + 1) * N, 0, s.sR.p, 0, 1, rows_q(l), s.d_mods.p, N, nullptr, s.st);
   launch_add(b, b, as.p, 0, 1, rows_q(l), s.d_mods.p, N, true, s.st);
   launch_add(b, b, pt.d.p, 0, 1, rows_q(l), s.d_mods.p, N, false, s.st);
   sync();
@@ -1858,8 +1868,7 @@ std::unique_ptr<Plain> decrypt_ct(const Cipher& ct) {
   auto p = std::make_unique<Plain>();
   p->level = l; p->scale = ct.scale; p->logslots = ct.logslots;
   p->d = DU64((size_t)(l + 1) * N);
-  d2d(p->d.p, ct.d.p, (size_t)(l + 1) * N * 8);
-  launch_mont_mul(p->d.p, 0, ct.d.p + (size_t)(l + 1) * N, 0, s.sR.p, 0, 1, rows_q(l), s.d_mods.p, N, true, s.st);
+  launch_mont_mul(p->d.p, 0, ct.d.p + (size_t)(l + 1) * N, 0, s.sR.p, 0, 1, rows_q(l), s.d_mods.p, N, ct.d.p, s.st);
   sync();
   return p;
 }
@@ -1871,10 +1880,7 @@ std::unique_ptr<Plain> encode_values(const float* v, int n, int level, double sc
   auto p = std::make_unique<Plain>();
   p->level = level; p->scale = scale; p->logslots = s.logN - 1;
   p->d = DU64((size_t)(level + 1) * s.N);
-  // the load kernel reads a full slots-wide row: pad the values with zeros
-  std::vector<float> buf((size_t)s.N / 2, 0.0f);
-  std::copy(v, v + n, buf.begin());
-  encode_device(buf.data(), buf.size(), {EncodeSrc{0, 0}}, n, scale, rows_q(level), p->d.p, 0);
+  encode_device(v, (size_t)n, {EncodeSrc{0, 0}}, n, scale, rows_q(level), p->d.p, 0);
   return p;
 }
 // complex slot values, interleaved (re, im) pairs as EncodeComplex passes them
@@ -1885,9 +1891,7 @@ std::unique_ptr<Plain> encode_complex_values(const float* v, int n, int level, d
   auto p = std::make_unique<Plain>();
   p->level = level; p->scale = scale; p->logslots = s.logN - 1;
   p->d = DU64((size_t)(level + 1) * s.N);
-  std::vector<float> buf((size_t)s.N, 0.0f);
-  std::copy(v, v + 2 * (size_t)n, buf.begin());
-  encode_device(buf.data(), buf.size(), {EncodeSrc{0, 0}}, n, scale, rows_q(level), p->d.p, 0, true);
+  encode_device(v, 2 * (size_t)n, {EncodeSrc{0, 0}}, n, scale, rows_q(level), p->d.p, 0, true);
   return p;
 }
 // The slots of a plaintext: mode 0 real parts as float, 1 as double, 2 (re, im)

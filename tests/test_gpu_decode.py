@@ -100,3 +100,29 @@ def test_encode_encrypt_sizes(hip_lib, logn):
     finally:
         orc.close()
         hip_lib.DeleteScheme()
+
+
+@pytest.mark.parametrize("h", [255, 256, 257, 700])
+def test_encrypt_positions(hip_lib, h):
+    """The ternary polynomial's positions travel with the launch up to 256 and
+    through memory above; one limb and several, a modulus of 61 bits in P."""
+    q, p = make_params(10, [60, 50, 40, 55], [61, 61])
+    new_hip_scheme(hip_lib, 10, q, p, 40, h, 4, evaluator=False)
+    orc = O.Oracle(10, q, p, h=h, seed=4)
+    rng = np.random.default_rng(h)
+    try:
+        for index, level in enumerate((3, 1, 0)):
+            print(f"[encrypt] h {h} level {level}", flush=True)
+            vals = rng.uniform(-1, 1, 512).astype(np.float32)
+            hip_lib.SetEncryptionCounter(index)
+            pt = hip_lib.Encode(vals, level, 1 << 40)
+            ct = hip_lib.Encrypt(pt)
+            want = orc.encode(vals, level, float(1 << 40))
+            assert_equal_u64(hip_lib.export_ciphertext(ct), orc.encrypt(want, level, index), f"encrypt h {h} level {level}")
+            dec = hip_lib.Decrypt(ct)
+            got = hip_lib.decode_double(dec)
+            ref = orc.decode_f64(hip_lib.export_plaintext(dec), level, float(1 << 40))
+            np.testing.assert_array_equal(got.view(np.uint64), ref.view(np.uint64))
+    finally:
+        orc.close()
+        hip_lib.DeleteScheme()

@@ -46,22 +46,26 @@ struct FftArgs {
   int mode;
 };
 
-// one butterfly of stage len, root j: forward (u, v) -> (u + w v, u - w v),
-// inverse (u, v) -> (u + v, (u - v) conj(w))
+// the twiddle of stage len, root j (conjugate for the inverse)
 template <bool INV>
-__device__ __forceinline__ void fft_butterfly(const FftArgs& a, int len, int j, double& ur, double& ui, double& vr, double& vi) {
-#pragma clang fp contract(off)
+__device__ __forceinline__ double2 fft_root(const FftArgs& a, int len, int j) {
   const int lenq = len << 2, gap = a.M / lenq, r = a.rotgroup[j] & (lenq - 1);
   const int idx = (INV ? lenq - r : r) * gap;
-  const double wr = a.rre[idx], wi = a.rim[idx];
+  return make_double2(a.rre[idx], a.rim[idx]);
+}
+// one butterfly: forward (u, v) -> (u + w v, u - w v), inverse (u, v) ->
+// (u + v, (u - v) w)
+template <bool INV>
+__device__ __forceinline__ void fft_butterfly(double2 w, double& ur, double& ui, double& vr, double& vi) {
+#pragma clang fp contract(off)
   if (INV) {
     const double dr = ur - vr, di = ui - vi;
     ur = ur + vr;
     ui = ui + vi;
-    vr = dr * wr - di * wi;
-    vi = dr * wi + di * wr;
+    vr = dr * w.x - di * w.y;
+    vi = dr * w.y + di * w.x;
   } else {
-    const double tr = vr * wr - vi * wi, ti = vr * wi + vi * wr;
+    const double tr = vr * w.x - vi * w.y, ti = vr * w.y + vi * w.x;
     vr = ur - tr;
     vi = ui - ti;
     ur = ur + tr;
@@ -69,31 +73,51 @@ __device__ __forceinline__ void fft_butterfly(const FftArgs& a, int len, int j, 
   }
 }
 
+// Both kernels load every stage's twiddles (a table read behind another one)
+// before the first stage: the stages wait for LDS only.  A launch of one
+// plaintext has few workgroups, and the two reads a stage were most of its
+// time: 2^15 slots, columns 13.5 -> 11.1 us, blocks 6.8 -> 3.8 us.
+
 // stages len <= FFT_B of one block: 128 threads, a butterfly each per stage
 template <bool INV>
 __global__ __launch_bounds__(FFT_B / 2) void fft_block_kernel(FftArgs a) {
+  constexpr int LB = 8;
+  static_assert(FFT_B == 1 << LB, "stages of a block");
   __shared__ double sr[FFT_B], si[FFT_B];
   const int t = threadIdx.x, base = blockIdx.x * FFT_B;
   double* R = a.re + (size_t)blockIdx.y * a.pstride + base;
   double* I = a.im + (size_t)blockIdx.y * a.pstride + base;
+  double2 w[LB];
+#pragma unroll
+  for (int s = 0; s < LB; s++) w[s] = fft_root<INV>(a, 2 << s, t & ((1 << s) - 1));
   for (int k = t; k < FFT_B; k += FFT_B / 2) { sr[k] = R[k]; si[k] = I[k]; }
-  for (int len = INV ? FFT_B : 2; INV ? len >= 2 : len <= FFT_B; len = INV ? len >> 1 : len << 1) {
+#pragma unroll
+  for (int q = 0; q < LB; q++) {
+    const int s = INV ? LB - 1 - q : q, lenh = 1 << s;
     __syncthreads();
-    const int lenh = len >> 1, j = t & (lenh - 1), k = 2 * (t - j) + j;
-    fft_butterfly<INV>(a, len, j, sr[k], si[k], sr[k + lenh], si[k + lenh]);
+    const int j = t & (lenh - 1), k = 2 * (t - j) + j;
+    fft_butterfly<INV>(w[s], sr[k], si[k], sr[k + lenh], si[k + lenh]);
   }
   __syncthreads();
   for (int k = t; k < FFT_B; k += FFT_B / 2) { R[k] = sr[k]; I[k] = si[k]; }
 }
 
-// stages len > FFT_B: FFT_CW columns of the (n / FFT_B) x FFT_B view
-template <bool INV>
+// stages len > FFT_B: FFT_CW columns of the (n / FFT_B) x FFT_B view, n / FFT_B = 2^LR rows
+template <bool INV, int LR>
 __global__ __launch_bounds__(256) void fft_col_kernel(FftArgs a) {
-  constexpr int MAXE = 128 * FFT_CW;
-  __shared__ double sr[MAXE], si[MAXE];
-  const int rows = a.n / FFT_B, E = rows * FFT_CW, col0 = blockIdx.x * FFT_CW;
+  constexpr int rows = 1 << LR, E = rows * FFT_CW, NB = (E / 2 + 255) / 256;  // NB: butterflies a thread and stage
+  __shared__ double sr[E], si[E];
+  const int col0 = blockIdx.x * FFT_CW;
   double* R = a.re + (size_t)blockIdx.y * a.pstride;
   double* I = a.im + (size_t)blockIdx.y * a.pstride;
+  double2 w[LR][NB];
+#pragma unroll
+  for (int s = 0; s < LR; s++)
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      const int u = threadIdx.x + 256 * i, c = u % FFT_CW, jr = (u / FFT_CW) & ((1 << s) - 1);
+      w[s][i] = fft_root<INV>(a, (2 << s) * FFT_B, jr * FFT_B + col0 + c);
+    }
   for (int e = threadIdx.x; e < E; e += 256) {
     const int k = (e / FFT_CW) * FFT_B + col0 + e % FFT_CW;
     double v = 0.0, vi = 0.0;
@@ -112,13 +136,18 @@ __global__ __launch_bounds__(256) void fft_col_kernel(FftArgs a) {
     sr[e] = v;
     si[e] = vi;
   }
-  for (int rl = INV ? rows : 2; INV ? rl >= 2 : rl <= rows; rl = INV ? rl >> 1 : rl << 1) {
+#pragma unroll
+  for (int q = 0; q < LR; q++) {
+    const int s = INV ? LR - 1 - q : q, rh = 1 << s;
     __syncthreads();
-    const int rh = rl >> 1;
-    for (int u = threadIdx.x; u < E / 2; u += 256) {
-      const int c = u % FFT_CW, b = u / FFT_CW, jr = b & (rh - 1);
-      const int k = (2 * (b - jr) + jr) * FFT_CW + c, k2 = k + rh * FFT_CW;
-      fft_butterfly<INV>(a, rl * FFT_B, jr * FFT_B + col0 + c, sr[k], si[k], sr[k2], si[k2]);
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+      const int u = threadIdx.x + 256 * i;
+      if (u < E / 2) {
+        const int c = u % FFT_CW, b = u / FFT_CW, jr = b & (rh - 1);
+        const int k = (2 * (b - jr) + jr) * FFT_CW + c, k2 = k + rh * FFT_CW;
+        fft_butterfly<INV>(w[s][i], sr[k], si[k], sr[k2], si[k2]);
+      }
     }
   }
   __syncthreads();
@@ -135,6 +164,19 @@ __global__ __launch_bounds__(256) void fft_col_kernel(FftArgs a) {
       ((float*)a.out)[2 * (size_t)k] = (float)sr[e];
       ((float*)a.out)[2 * (size_t)k + 1] = (float)si[e];
     }
+  }
+}
+template <bool INV>
+void launch_fft_col(const FftArgs& f, int np, hipStream_t st) {
+  const dim3 grid(FFT_B / FFT_CW, np), block(256);
+  switch (f.n / FFT_B) {
+    case 2: hipLaunchKernelGGL((fft_col_kernel<INV, 1>), grid, block, 0, st, f); break;
+    case 4: hipLaunchKernelGGL((fft_col_kernel<INV, 2>), grid, block, 0, st, f); break;
+    case 8: hipLaunchKernelGGL((fft_col_kernel<INV, 3>), grid, block, 0, st, f); break;
+    case 16: hipLaunchKernelGGL((fft_col_kernel<INV, 4>), grid, block, 0, st, f); break;
+    case 32: hipLaunchKernelGGL((fft_col_kernel<INV, 5>), grid, block, 0, st, f); break;
+    case 64: hipLaunchKernelGGL((fft_col_kernel<INV, 6>), grid, block, 0, st, f); break;
+    default: hipLaunchKernelGGL((fft_col_kernel<INV, 7>), grid, block, 0, st, f); break;
   }
 }
 
@@ -187,28 +229,32 @@ __global__ void encode_finish_kernel(u64* __restrict__ out, size_t out_pstride, 
 //   acc = sum_i y_i * (Q / q_i) - k Q,  y_i = x_i (Q / q_i)^-1 mod q_i,
 // k = floor(sum_i y_i / q_i) in float64 (off by at most one, corrected), then
 // Q - acc for acc >= floor(Q / 2), the nearest double of it (ties to even) over
-// the scale, stored at its bit-reversed place of the FFT.  One thread a
-// coefficient, acc in W words (2^(64 W) > 2^8 Q) held in registers up to 32
-// words; l + 1 passes of W multiply-adds over wave-uniform table words.  One
-// wave a SIMD at N = 2^16, so the next row's word is loaded a row ahead.
+// the scale, stored at its bit-reversed place of the FFT.  A workgroup takes 64
+// coefficients: each of its four waves sums every fourth source in W words
+// (2^(64 W) > 2^8 Q, in registers up to 32 words; W multiply-adds a source over
+// wave-uniform table words), the first adds the four sums and finishes.  One
+// thread a coefficient leaves a wave a SIMD at N = 2^16, each multiply-add
+// waiting for the carry of the one before: 36 us at 23 limbs, 28 this way.
 // Decrypt and Decode of 23 limbs there took 7.5 ms with this sum on the host
-// (12 MB of residues fetched, 16 threads); 0.75 ms with it here, 0.65 of them
-// the caller's list of floats.
+// (12 MB of residues fetched, 16 threads).
 template <int W>
 __global__ __launch_bounds__(256) void decode_crt_kernel(DecodeArgs d) {
 #pragma clang fp contract(off)
   constexpr int UN = W <= 32 ? W : 1;
-  const int x = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ u64 part[3][W][64];
+  __shared__ double pest[3][64];
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int x = blockIdx.x * 64 + lane;
   const int N = d.N, n = N >> 1;
   u64 a[W];
 #pragma unroll UN
   for (int w = 0; w < W; w++) a[w] = 0;
   double est = 0.0;
-  u64 next = d.coef[x];
-  for (int i = 0; i < d.nl; i++) {
+  u64 next = d.coef[(size_t)min(wv, d.nl - 1) * N + x];
+  for (int i = wv; i < d.nl; i += 4) {
     const BConvSrc s = d.src[i];
     const u64 xi = next;
-    next = d.coef[(size_t)min(i + 1, d.nl - 1) * N + x];  // in flight while row i is multiplied
+    next = d.coef[(size_t)min(i + 4, d.nl - 1) * N + x];  // in flight while row i is multiplied
     const u64 y = shoup_mul(xi, s.hinv, s.hinvp, s.q);
     est += (double)y / s.qd;
     const u64* h = d.hat + (size_t)i * W;
@@ -219,6 +265,23 @@ __global__ __launch_bounds__(256) void decode_crt_kernel(DecodeArgs d) {
       a[w] = (u64)t;
       c = (u64)(t >> 64);
     }
+  }
+  if (wv) {
+#pragma unroll UN
+    for (int w = 0; w < W; w++) part[wv - 1][w][lane] = a[w];
+    pest[wv - 1][lane] = est;
+  }
+  __syncthreads();
+  if (wv) return;
+  for (int p = 0; p < 3; p++) {
+    u64 c = 0;
+#pragma unroll UN
+    for (int w = 0; w < W; w++) {
+      const u128 t = (u128)a[w] + part[p][w][lane] + c;
+      a[w] = (u64)t;
+      c = (u64)(t >> 64);
+    }
+    est += pest[p][lane];
   }
   const u64* Q = d.hat + (size_t)d.nl * W;
   const u64* Qh = Q + W;
@@ -296,7 +359,7 @@ void launch_encode_fft(u64* out, size_t out_pstride, RowMap rm, const float* dat
   const int N = 1 << logN, n = N >> 1, logn = logN - 1;
   const int tpb = 256;
   const FftArgs f{re, im, pstride, n, 2 * N, rotgroup, rre, rim, data, src, nvals, complex_in ? 1 : 0, nullptr, 0};
-  hipLaunchKernelGGL(fft_col_kernel<true>, dim3(FFT_B / FFT_CW, np), dim3(256), 0, st, f);
+  launch_fft_col<true>(f, np, st);
   hipLaunchKernelGGL(fft_block_kernel<true>, dim3(n / FFT_B, np), dim3(FFT_B / 2), 0, st, f);
   hipLaunchKernelGGL(encode_finish_kernel, dim3((N + tpb - 1) / tpb, np), dim3(tpb), 0, st, out, out_pstride, rm, re, im,
                      pstride, n, logn, scale, mods, N);
@@ -305,7 +368,7 @@ void launch_encode_fft(u64* out, size_t out_pstride, RowMap rm, const float* dat
 void launch_decode_fft(const DecodeArgs& d, int words, const int* rotgroup, const double* rre, const double* rim, void* out,
                        int mode, hipStream_t st) {
   const int n = d.N / 2;
-  const dim3 grid(d.N / 256), block(256);
+  const dim3 grid(d.N / 64), block(256);
   switch (words) {
     case 4: hipLaunchKernelGGL(decode_crt_kernel<4>, grid, block, 0, st, d); break;
     case 8: hipLaunchKernelGGL(decode_crt_kernel<8>, grid, block, 0, st, d); break;
@@ -319,5 +382,5 @@ void launch_decode_fft(const DecodeArgs& d, int words, const int* rotgroup, cons
   }
   const FftArgs f{d.re, d.im, 0, n, 2 * d.N, rotgroup, rre, rim, nullptr, nullptr, 0, 0, out, mode};
   hipLaunchKernelGGL(fft_block_kernel<false>, dim3(n / FFT_B), dim3(FFT_B / 2), 0, st, f);
-  hipLaunchKernelGGL(fft_col_kernel<false>, dim3(FFT_B / FFT_CW), dim3(256), 0, st, f);
+  launch_fft_col<false>(f, 1, st);
 }

@@ -192,7 +192,7 @@ void launch_ntt_rescale_pair(u64* t, size_t t_bstride, int l, int logN, const u6
 // dst[b][0..words) = src[b][0..words) for b < batch.
 void launch_copy(u64* dst, size_t dstride, const u64* src, size_t sstride, size_t words, int batch, hipStream_t st);
 void launch_add(u64* out, const u64* a, const u64* b, size_t bstride, int batch, RowMap rm, const ModC* mods, int N, bool sub, hipStream_t st);
-void launch_mul_const(u64* out, const u64* in, size_t bstride, int batch, RowMap rm, const u64* cw, const u64* cwp, const ModC* mods, int N, hipStream_t st);
+void launch_mul_const(u64* out, size_t obstride, const u64* in, size_t bstride, int batch, RowMap rm, const u64* cw, const u64* cwp, const ModC* mods, int N, hipStream_t st);
 // Packed diagonal storage: dst (packed layout, dst_stride dwords a
 // diagonal) <- src (plain [np][nrows][N], src_stride words a diagonal), and
 // back for one diagonal (dst plain [nrows][N]).
@@ -216,7 +216,7 @@ void launch_mul_const_v(u64* out, const u64* in, size_t bstride, int batch, RowM
 // out = in +- c.w[modulus] on the rows of rm (one polynomial)
 void launch_add_scalar_v(u64* out, const u64* in, RowMap rm, const RowConst& c, const ModC* mods, int N, bool sub,
                          hipStream_t st);
-void launch_mont_mul(u64* out, size_t obstride, const u64* a, size_t abstride, const u64* bR, size_t bbstride, int batch, RowMap rm, const ModC* mods, int N, const u64* add, hipStream_t st);
+void launch_mont_mul(u64* out, size_t obstride, const u64* a, size_t abstride, const u64* bR, size_t bbstride, int batch, RowMap rm, const ModC* mods, int N, const u64* add, hipStream_t st, bool bmod = false);
 void launch_mont_convert(u64* data, size_t bstride, int batch, RowMap rm, const ModC* mods, int N, bool to, hipStream_t st);
 // Basis extension of the ns source rows of `in` into the target rows rm of `out`.
 // One source group of a batched basis extension (e.g. one digit of a

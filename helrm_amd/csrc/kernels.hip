@@ -30,18 +30,19 @@ void launch_add(u64* out, const u64* a, const u64* b, size_t bstride, int batch,
 }
 
 // out = in * c_row (per-row constant in Shoup form, indexed by modulus)
-__global__ void mul_const_kernel(u64* __restrict__ out, const u64* __restrict__ in, size_t bstride, RowMap rm,
+__global__ void mul_const_kernel(u64* __restrict__ out, size_t obstride, const u64* __restrict__ in, size_t bstride, RowMap rm,
                                  const u64* __restrict__ cw, const u64* __restrict__ cwp, const ModC* __restrict__ mods, int N) {
   int x = blockIdx.x * blockDim.x + threadIdx.x;
   int row = rm.row(blockIdx.y);
   int m = rm.mod(row);
-  size_t o = (size_t)blockIdx.z * bstride + (size_t)row * N + x;
-  out[o] = shoup_mul(in[o], cw[m], cwp[m], mods[m].q);
+  size_t o = (size_t)row * N + x;
+  out[(size_t)blockIdx.z * obstride + o] = shoup_mul(in[(size_t)blockIdx.z * bstride + o], cw[m], cwp[m], mods[m].q);
 }
-void launch_mul_const(u64* out, const u64* in, size_t bstride, int batch, RowMap rm, const u64* cw, const u64* cwp,
-                      const ModC* mods, int N, hipStream_t st) {
+void launch_mul_const(u64* out, size_t obstride, const u64* in, size_t bstride, int batch, RowMap rm, const u64* cw,
+                      const u64* cwp, const ModC* mods, int N, hipStream_t st) {
   if (rm.nact() <= 0 || batch <= 0) return;
-  hipLaunchKernelGGL(mul_const_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, in, bstride, rm, cw, cwp, mods, N);
+  hipLaunchKernelGGL(mul_const_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, obstride, in, bstride, rm, cw, cwp,
+                     mods, N);
 }
 
 __global__ void mul_const_v_kernel(u64* __restrict__ out, const u64* __restrict__ in, size_t bstride, RowMap rm, RowConst c,
@@ -138,21 +139,23 @@ void launch_tensor(u64* d0, u64* d1, u64* d2, const u64* a0, const u64* a1, cons
   hipLaunchKernelGGL(tensor_kernel, dim3(N / 256, l + 1, 1), dim3(256), 0, st, d0, d1, d2, a0, a1, b0, b1, pw, pwp, mods, N);
 }
 
-// out = a * bR * R^-1 (b stored in Montgomery form), plus add (at out's stride) if given
+// out = a * bR * R^-1 (b stored in Montgomery form), plus add (at out's stride)
+// if given; with bmod, bR holds a row per modulus instead of one per row
 __global__ void mont_mul_kernel(u64* out, const u64* __restrict__ a, size_t abstride,
                                 const u64* __restrict__ bR, size_t bbstride, size_t obstride, RowMap rm,
-                                const ModC* __restrict__ mods, int N, const u64* add) {
+                                const ModC* __restrict__ mods, int N, const u64* add, int bmod) {
   int x = blockIdx.x * blockDim.x + threadIdx.x;
-  int row = rm.row(blockIdx.y);
-  ModC mc = mods[rm.mod(row)];
-  u64 r = mont_mul(a[(size_t)blockIdx.z * abstride + (size_t)row * N + x], bR[(size_t)blockIdx.z * bbstride + (size_t)row * N + x], mc.q, mc.qinv);
+  int row = rm.row(blockIdx.y), m = rm.mod(row);
+  ModC mc = mods[m];
+  u64 r = mont_mul(a[(size_t)blockIdx.z * abstride + (size_t)row * N + x],
+                   bR[(size_t)blockIdx.z * bbstride + (size_t)(bmod ? m : row) * N + x], mc.q, mc.qinv);
   size_t o = (size_t)blockIdx.z * obstride + (size_t)row * N + x;
   out[o] = add ? add_mod(add[o], r, mc.q) : r;
 }
 void launch_mont_mul(u64* out, size_t obstride, const u64* a, size_t abstride, const u64* bR, size_t bbstride, int batch,
-                     RowMap rm, const ModC* mods, int N, const u64* add, hipStream_t st) {
+                     RowMap rm, const ModC* mods, int N, const u64* add, hipStream_t st, bool bmod) {
   if (rm.nact() <= 0 || batch <= 0) return;
-  hipLaunchKernelGGL(mont_mul_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, a, abstride, bR, bbstride, obstride, rm, mods, N, add);
+  hipLaunchKernelGGL(mont_mul_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, a, abstride, bR, bbstride, obstride, rm, mods, N, add, bmod ? 1 : 0);
 }
 
 // out[row] = in[row] +- c.w[modulus of row] (a constant in every NTT slot)

@@ -1657,8 +1657,7 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
   DU64 digits((size_t)dn * qp);
   decompose_modup(l, c1, 0, 1, digits.p, false);
   DU64 pc((size_t)2 * (l + 1) * N);
-  launch_mul_const(pc.p, c0, 0, 1, rows_q(l), s.pmod_w.p, s.pmod_wp.p, s.d_mods.p, N, s.st);
-  launch_mul_const(pc.p + (size_t)(l + 1) * N, c1, 0, 1, rows_q(l), s.pmod_w.p, s.pmod_wp.p, s.d_mods.p, N, s.st);
+  launch_mul_const(pc.p, (size_t)(l + 1) * N, c0, (size_t)(c1 - c0), 2, rows_q(l), s.pmod_w.p, s.pmod_wp.p, s.d_mods.p, N, s.st);
   std::vector<int> babies;
   for (int b : t.rot2) if (b != 0) babies.push_back(b);
   const int nbr = (int)babies.size();
@@ -1760,7 +1759,7 @@ std::unique_ptr<Cipher> eval_lt_naive(const LinTrans& t, const Cipher& ct) {
   DU64 digits((size_t)dn * qp);
   decompose_modup(l, c1, 0, 1, digits.p, false);
   DU64 pc((size_t)(l + 1) * N);
-  launch_mul_const(pc.p, c0, 0, 1, rows_q(l), s.pmod_w.p, s.pmod_wp.p, s.d_mods.p, N, s.st);
+  launch_mul_const(pc.p, 0, c0, 0, 1, rows_q(l), s.pmod_w.p, s.pmod_wp.p, s.d_mods.p, N, s.st);
   std::vector<int> nz; int zero_p = -1;
   for (size_t i = 0; i < t.plain_idx.size(); i++) { if ((t.plain_idx[i] & (t.slots - 1)) == 0) zero_p = (int)i; else nz.push_back((int)i); }
   DU64 acc((size_t)2 * qp);
@@ -1819,10 +1818,7 @@ std::unique_ptr<Cipher> encrypt_pt(const Plain& pt) {
     launch_ternary_rows(uq.p, rm, du.p, (int)u.size(), s.d_mods.p, N, s.st);
   }
   ntt(uq.p, 0, 1, rm, true);
-  // pkR holds every modulus: rows q_0..q_l, then row p_0 of it
-  launch_mont_mul(tt.p, (size_t)nr * N, uq.p, 0, s.pkR.p, (size_t)nm * N, 2, rows_q(l), s.d_mods.p, N, nullptr, s.st);
-  launch_mont_mul(tt.p + (size_t)(l + 1) * N, (size_t)nr * N, uq.p + (size_t)(l + 1) * N, 0, s.pkR.p + (size_t)s.L * N,
-                  (size_t)nm * N, 2, RowMap{1, 0, 0, s.L, 0, 0}, s.d_mods.p, N, nullptr, s.st);
+  launch_mont_mul(tt.p, (size_t)nr * N, uq.p, 0, s.pkR.p, (size_t)nm * N, 2, rm, s.d_mods.p, N, nullptr, s.st, true);
   ntt(tt.p, (size_t)nr * N, 2, rm, false);
   // errors and ModDown from Q + {p_0} in the coefficient domain, then the
   // transform, which adds the plaintext to part 0

@@ -763,7 +763,81 @@ __global__ __launch_bounds__(256) void giant_acc_kernel(GiantAccArgs a) {
     a.out1[o] = redc(tlo1, add_mod(thi1, tz1, mc.q), mc.q, mc.qinv);
   }
 }
+// The same with the digit count known (up to HCK_KM1_DIG; longer
+// decompositions take the loop above).  Bound by memory: the 2 DN + 1 words of
+// a group (3 DN + 1 with the a halves read) are loaded together, behind the
+// next group's source position, where the loop waits for each digit's pair.  31
+// groups of 3 digits, 32 rows of N = 2^16: 800 -> 660 us, 5.5 TB/s over the
+// b halves, digits and accumulators; 15 groups of 5 digits, 6 rows of 2^13:
+// 17 -> 9 us.
+template <int DN, bool SEEDED>
+__global__ __launch_bounds__(256) void giant_acc_dn_kernel(GiantAccArgs a) {
+  constexpr int PER = 16 / DN;  // groups per accumulator
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  const int k = blockIdx.y;
+  const int N = a.N;
+  const int kl = k <= a.l ? k : a.L + (k - a.l - 1);
+  const ModC mc = a.mods[kl];
+  const int own_d = (a.own && k <= a.l) ? k / a.K : -1;
+  const size_t kstride = (size_t)(a.L + a.K) * N;
+  Acc128 A0, A1;
+  acc_zero(A0); acc_zero(A1);
+  u64 tlo0 = 0, thi0 = 0, tlo1 = 0, thi1 = 0, t0 = 0;
+  int next = (int)a.perm[0][i], cnt = 0;
+  for (int g = 0; g < a.ng; g++) {
+    const int src = next;
+    next = (int)a.perm[min(g + 1, a.ng - 1)][i];
+    const u64* dg = a.digits + (size_t)g * a.dig_bstride + (size_t)k * N + src;
+    const u64* own = a.own ? a.own + (size_t)g * a.own_bstride + (size_t)k * N + src : nullptr;
+    const u64* key = a.key[g] + (size_t)kl * N + src;
+    u64 x[DN], kb[DN], ka[DN];
+#pragma unroll
+    for (int d = 0; d < DN; d++) {
+      x[d] = *(d == own_d ? own : dg + (size_t)d * a.nqp * N);
+      kb[d] = __builtin_nontemporal_load(key + (size_t)d * 2 * kstride);
+      if (!SEEDED) ka[d] = __builtin_nontemporal_load(key + (size_t)d * 2 * kstride + kstride);
+    }
+    const u64 t = (a.T + (size_t)a.tg[g] * a.T_gstride)[(size_t)k * N + src];
+    if (cnt == PER) {
+      acc_flush(A0, tlo0, thi0, mc.q);
+      acc_flush(A1, tlo1, thi1, mc.q);
+      cnt = 0;
+    }
+    cnt++;
+#pragma unroll
+    for (int d = 0; d < DN; d++) {
+      acc_mac(A0, x[d], kb[d]);
+      acc_mac(A1, x[d], SEEDED ? key_a_word(a.ka[(size_t)g * DN + d], (u64)kl * N + src, mc.q) : ka[d]);
+    }
+    t0 = add_mod(t0, t, mc.q);
+  }
+  acc_flush(A0, tlo0, thi0, mc.q);
+  acc_flush(A1, tlo1, thi1, mc.q);
+  thi0 = add_mod(thi0, t0, mc.q);
+  u64 tz1 = 0;
+  if (a.t_zero >= 0) {
+    const u64* Tz = a.T + (size_t)a.t_zero * a.T_gstride;
+    thi0 = add_mod(thi0, Tz[(size_t)k * N + i], mc.q);
+    tz1 = Tz[a.T_pstride + (size_t)k * N + i];
+  }
+  const size_t o = (size_t)k * N + i;
+  a.out0[o] = redc(tlo0, thi0, mc.q, mc.qinv);
+  if (SEEDED) a.out1[o] = add_mod(mont_mul(redc(tlo1, thi1, mc.q, mc.qinv), mc.r2, mc.q, mc.qinv), tz1, mc.q);
+  else a.out1[o] = redc(tlo1, add_mod(thi1, tz1, mc.q), mc.q, mc.qinv);
+}
+template <int DN>
+static bool launch_giant_acc_t(const GiantAccArgs& a, hipStream_t st) {
+  if (DN < a.dn) {
+    if constexpr (DN < HCK_KM1_DIG) return launch_giant_acc_t<DN + 1>(a, st);
+    return false;
+  }
+  const dim3 grid(a.N / 256, a.nqp), block(256);
+  if (a.ka) hipLaunchKernelGGL((giant_acc_dn_kernel<DN, true>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((giant_acc_dn_kernel<DN, false>), grid, block, 0, st, a);
+  return true;
+}
 void launch_giant_acc(const GiantAccArgs& a, hipStream_t st) {
+  if (a.ng > 0 && launch_giant_acc_t<1>(a, st)) return;
   hipLaunchKernelGGL(giant_acc_kernel, dim3(a.N / 256, a.nqp, 1), dim3(256), 0, st, a);
 }
 

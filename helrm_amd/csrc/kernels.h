@@ -159,6 +159,7 @@ struct DiagMacArgs {
   int dn;
   const u64* bka;                 // [slot][dn] per-stream PRNG keys of the a halves (regenerated), or nullptr (read)
   const uint32_t* pkrow;          // packed layout: [row][2] descriptors, nullptr for plain [np][nqp][N]
+  int gper;  // groups of a workgroup (set by the launch)
 };
 
 // In-place NTT (forward) / inverse NTT of rows rm of `batch` polynomials.

@@ -939,6 +939,9 @@ __device__ __forceinline__ void baby_rotation_at(const DiagMacArgs& a, int slot,
   if (ka) r1 = mont_mul(r1, mc.r2, mc.q, mc.qinv);  // regenerated a halves carry no R
 }
 
+// The groups of a workgroup: a launch of few workgroups deals them out over
+// blockIdx.z (each part computes the baby rotations for itself).
+__device__ __forceinline__ int mac_g0(const DiagMacArgs& a) { return a.g0 + (int)blockIdx.z * a.gper; }
 template <int NB, bool DENSE, bool ACC>
 __global__ __launch_bounds__(256) void diag_mac_kernel(DiagMacArgs a) {
   const int x = blockIdx.x * blockDim.x + threadIdx.x;
@@ -968,11 +971,12 @@ __global__ __launch_bounds__(256) void diag_mac_kernel(DiagMacArgs a) {
   // the current group's products.
   u64 dA[NB], dB[NB], tA[2], tB[2];
   u64* Tb = a.T + (size_t)k * N + x;
-  int g = a.g0;
+  int g = mac_g0(a);
+  const int g1 = min(a.g1, g + a.gper);
   mac_load<NB, DENSE, ACC>(a, dbase, g, dA, tA, Tb);
   // (the scheduling barriers keep the machine scheduler from sinking the
   // prefetch below the products to save registers)
-  for (; g + 2 < a.g1; g += 2) {
+  for (; g + 2 < g1; g += 2) {
     mac_load<NB, DENSE, ACC>(a, dbase, g + 1, dB, tB, Tb);
     __builtin_amdgcn_sched_barrier(0);
     mac_group<NB, ACC>(a, dA, tA, s0, s1, mc, Tb + (size_t)g * a.T_gstride);
@@ -980,7 +984,7 @@ __global__ __launch_bounds__(256) void diag_mac_kernel(DiagMacArgs a) {
     __builtin_amdgcn_sched_barrier(0);
     mac_group<NB, ACC>(a, dB, tB, s0, s1, mc, Tb + (size_t)(g + 1) * a.T_gstride);
   }
-  if (g + 1 < a.g1) {
+  if (g + 1 < g1) {
     mac_load<NB, DENSE, ACC>(a, dbase, g + 1, dB, tB, Tb);
     __builtin_amdgcn_sched_barrier(0);
     mac_group<NB, ACC>(a, dA, tA, s0, s1, mc, Tb + (size_t)g * a.T_gstride);
@@ -1018,17 +1022,18 @@ __device__ __forceinline__ void mac_d16_rows(const DiagMacArgs& a, const u64 (&s
                                          (__attribute__((address_space(3))) void*)&lds[h & 1][b][0], 16, 0, 0);
     }
   };
-  issue(2 * a.g0);
-  for (int g = a.g0; g < a.g1; g++) {
+  const int g0 = mac_g0(a), g1 = min(a.g1, g0 + a.gper);
+  issue(2 * g0);
+  for (int g = g0; g < g1; g++) {
     Acc128 A0, A1;
     acc_zero(A0); acc_zero(A1);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
       const int h = 2 * g + i;
-      const bool more = i == 0 || g + 1 < a.g1;
+      const bool more = i == 0 || g + 1 < g1;
       if (more) issue(h + 1);
       if (!more) __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8));                       // vmcnt(0)
-      else if (i == 0 && g != a.g0) __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8) | 10);  // vmcnt(10)
+      else if (i == 0 && g != g0) __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8) | 10);  // vmcnt(10)
       else __builtin_amdgcn_s_waitcnt((0x7 << 4) | (0xF << 8) | 8);                         // vmcnt(8)
 #pragma unroll
       for (int b = 0; b < MAC_HALF; b++) {
@@ -1074,14 +1079,25 @@ __global__ __launch_bounds__(256) void diag_mac_d16_kernel(DiagMacArgs a) {
   if (a.pkrow[2 * krow + 1]) mac_d16_rows<true>(a, s0, s1, mc, Tb, rbase + c * PK_CHUNK, lds[w], lane);
   else mac_d16_rows<false>(a, s0, s1, mc, Tb, rbase + c * MAC_SLOT, lds[w], lane);
 }
-void launch_diag_mac(const DiagMacArgs& a, hipStream_t st) {
-  if (a.g1 <= a.g0) return;
+// Fewer workgroups than this (four on a CU) share out the giant groups, down to
+// four a part.  N = 2^13, 10 rows: a wave a SIMD went through 26 groups one
+// after the other, ten ragged tables 499 -> 436 us with four parts; N = 2^16
+// fills the GPU with one.
+constexpr long MAC_FILL = 1024;
+void launch_diag_mac(const DiagMacArgs& args, hipStream_t st) {
+  const int ng = args.g1 - args.g0;
+  if (ng <= 0) return;
+  DiagMacArgs a = args;
+  int parts = 1;
+  while ((long)(a.N / 256) * a.nqp * parts < MAC_FILL && ng >= 8 * parts) parts *= 2;
+  a.gper = (ng + parts - 1) / parts;
+  parts = (ng + a.gper - 1) / a.gper;
   if (a.pkrow) {
     // a transform stored packed (dense, 16 baby steps)
-    hipLaunchKernelGGL(diag_mac_d16_kernel, dim3(a.N / 256, a.nqp, 1), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(diag_mac_d16_kernel, dim3(a.N / 256, a.nqp, parts), dim3(256), 0, st, a);
     return;
   }
-  dim3 grid(a.N / 256, a.nqp, 1);
+  dim3 grid(a.N / 256, a.nqp, parts);
   const bool dense = a.dense && a.nb_chunk == 16 && a.b0 + 16 <= a.nbaby;
   if (a.b0 == 0) {
     if (dense) hipLaunchKernelGGL((diag_mac_kernel<16, true, false>), grid, dim3(256), 0, st, a);

@@ -262,8 +262,12 @@ class Scheme:
         if not scale:
             scale = self.params.get_default_scale()
         slots = self.params.get_slots()
-        # the slots past the values are zero in the plaintext
-        ids = [self.backend.Encode(values[i:i + slots], level, int(scale)) for i in range(0, max(len(values), 1), slots)]
+        pad = (-len(values)) % slots
+        vec = np.concatenate([values, np.zeros(pad)]) if pad or len(values) == 0 else values
+        if len(vec) == 0:
+            vec = np.zeros(slots)
+        ids = [self.backend.Encode(vec[i * slots:(i + 1) * slots], level, int(scale))
+               for i in range(len(vec) // slots)]
         return PlainTensor(self, ids, len(values))
 
     def decode(self, pt):

@@ -1676,12 +1676,14 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
       tm.d_tg = DevArray<int>(std::max(ngk, 1));
       if (nbr) { upload(tm.d_bkey.p, bk.data(), nbr); upload(tm.d_bperm.p, bp.data(), nbr); }
       if (ngk) { upload(tm.d_gkey.p, gk.data(), ngk); upload(tm.d_gperm.p, gp.data(), ngk); upload(tm.d_tg.p, tg.data(), ngk); }
-      // the stream keys depend on the Galois element alone
-      std::vector<u64> bka((size_t)std::max(nbr, 1) * dn), gka((size_t)std::max(ngk, 1) * dn);
+      // the stream keys of a key's dnum digits depend on the Galois element
+      // alone: the tables serve every level, also one of fewer digits
+      const int dnum = s.dnum;
+      std::vector<u64> bka((size_t)std::max(nbr, 1) * dnum), gka((size_t)std::max(ngk, 1) * dnum);
       for (int i = 0; i < nbr; i++)
-        for (int d = 0; d < dn; d++) bka[(size_t)i * dn + d] = stream_key(ST_GK_A(galois_element(babies[i]), (u64)d));
+        for (int d = 0; d < dnum; d++) bka[(size_t)i * dnum + d] = stream_key(ST_GK_A(galois_element(babies[i]), (u64)d));
       for (int g = 0; g < ngk; g++)
-        for (int d = 0; d < dn; d++) gka[(size_t)g * dn + d] = stream_key(ST_GK_A(galois_element(t.giant[gs + g]), (u64)d));
+        for (int d = 0; d < dnum; d++) gka[(size_t)g * dnum + d] = stream_key(ST_GK_A(galois_element(t.giant[gs + g]), (u64)d));
       tm.d_bka = DevArray<u64>(bka.size()); upload(tm.d_bka.p, bka.data(), bka.size());
       tm.d_gka = DevArray<u64>(gka.size()); upload(tm.d_gka.p, gka.data(), gka.size());
       tm.ptrs_ready = true;
@@ -1701,7 +1703,7 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
   dm.diag = t.diags.p; dm.diag_stride = lt_diag_words(t);
   dm.pkrow = t.packed ? t.d_pkrow.p : nullptr;
   dm.digits = digits.p; dm.bkey = t.d_bkey.p; dm.bperm = t.d_bperm.p; dm.own = c1; dm.dn = dn;
-  dm.bka = babies_seeded ? t.d_bka.p : nullptr;
+  dm.bka = babies_seeded ? t.d_bka.p : nullptr; dm.bka_stride = s.dnum;
   dm.pc = pc.p; dm.pc_pstride = (size_t)(l + 1) * N;
   dm.baby_is_zero = t.d_bzero.p; dm.baby_slot = t.d_bslot.p; dm.gpi = t.d_gpi.p; dm.dense = t.dense ? 1 : 0;
   dm.zero_pidx = (int)t.plain_idx.size();
@@ -1728,7 +1730,7 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
     a.T = T.p; a.T_gstride = 2 * qp; a.T_pstride = qp; a.t_zero = gs ? 0 : -1;
     a.out0 = acc.p; a.out1 = acc.p + qp; a.mods = s.d_mods.p;
     a.N = N; a.l = l; a.L = s.L; a.K = K; a.nqp = nqp; a.dn = dn;
-    a.ka = giants_seeded ? t.d_gka.p : nullptr;
+    a.ka = giants_seeded ? t.d_gka.p : nullptr; a.ka_stride = s.dnum;
     timed("giant_acc", [&] { launch_giant_acc(a, s.st); });
   } else {
     d2d(acc.p, T.p, 2 * qp * 8);

@@ -266,12 +266,15 @@ class Scheme:
         vec = np.concatenate([values, np.zeros(pad)]) if pad or len(values) == 0 else values
         if len(vec) == 0:
             vec = np.zeros(slots)
-        ids = [self.backend.Encode(vec[i * slots:(i + 1) * slots], level, int(scale))
-               for i in range(len(vec) // slots)]
+        encode = self.backend.Encode
+        if not hasattr(encode, "array"):  # a plain callable takes a list of floats, as the reference's
+            vec = vec.tolist()
+        ids = [encode(vec[i * slots:(i + 1) * slots], level, int(scale)) for i in range(len(vec) // slots)]
         return PlainTensor(self, ids, len(values))
 
     def decode(self, pt):
-        vals = [self.backend.Decode.array(i) for i in pt.ids]
+        decode = getattr(self.backend.Decode, "array", self.backend.Decode)
+        vals = [np.asarray(decode(i), dtype=np.float64) for i in pt.ids]
         return np.concatenate(vals)[: pt.n] if vals else np.zeros(0)
 
     def encrypt(self, pt):

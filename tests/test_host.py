@@ -227,3 +227,55 @@ def test_pack_lanes_pairs_chunks(n, slots):
         p = packed[m * slots:(m + 1) * slots]
         np.testing.assert_allclose(p + np.conj(p), flat[2 * m * slots:(2 * m + 1) * slots], atol=1e-15)
         np.testing.assert_allclose((-1j * (p - np.conj(p))).real, flat[(2 * m + 1) * slots:(2 * m + 2) * slots], atol=1e-15)
+
+
+class ListBackend:
+    """A caller's backend of plain callables, lists in and out as the
+    reference's bindings; every other entry point answers 0."""
+
+    def __init__(self):
+        self.pts, self.calls = [], []
+
+    def Encode(self, values, level, scale):
+        assert type(values) is list and all(type(v) is float for v in values)
+        self.pts.append(values)
+        return len(self.pts) - 1
+
+    def Decode(self, i):
+        return list(self.pts[i])
+
+    def RotateNew(self, ct, amount):
+        self.calls.append(("RotateNew", ct, amount))
+        return ct + 100
+
+    def AddCiphertext(self, a, b):
+        self.calls.append(("AddCiphertext", a, b))
+        return a
+
+    def DeleteCiphertext(self, ct):
+        self.calls.append(("DeleteCiphertext", ct))
+        return ct
+
+    def setup(self, *args):
+        return 0
+
+    setup_bindings = NewKeyGenerator = GenerateSecretKey = GeneratePublicKey = setup
+    GenerateRelinearizationKey = GenerateEvaluationKeys = NewEncoder = NewEncryptor = setup
+    NewDecryptor = NewEvaluator = NewLinearTransformEvaluator = NewPolynomialEvaluator = setup
+
+
+@pytest.mark.parametrize("n", [0, 3, 512, 1300])
+def test_scheme_over_plain_callables(n):
+    """encode, decode and the fold with a backend that has no array forms and
+    none of the library's own entry points."""
+    b = ListBackend()
+    scheme = oh.Scheme(oh.Params(10, [40, 30], [40], 30, 64), b)
+    vals = np.random.default_rng(n).uniform(-1, 1, n)
+    pt = scheme.encode(vals)
+    assert all(len(v) == 512 for v in b.pts) and len(b.pts) == max(1, -(-n // 512))
+    got = scheme.decode(pt)
+    assert got.dtype == np.float64
+    np.testing.assert_array_equal(got, vals)
+    oh.CipherTensor(scheme, [7], n).fold([4, 2])
+    assert b.calls == [c for k in (4, 2) for c in
+                       (("RotateNew", 7, k), ("AddCiphertext", 7, 107), ("DeleteCiphertext", 107))]

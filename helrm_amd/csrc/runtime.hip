@@ -159,20 +159,21 @@ inline u64 ST_RLK_A(u64 d) { return (9ULL << 56) | d; }
 inline u64 ST_RLK_E(u64 d) { return (10ULL << 56) | d; }
 constexpr u64 ST_SEED_A = 11ULL << 56;
 inline u64 ST_SEED_E(u64 e) { return (12ULL << 56) | e; }
-// ternary vector with exactly h entries +-1 (partial Fisher-Yates)
-// The drawn positions in order, each as 2 * position + (1 for -1).  The
-// shuffle's array is kept only where a swap has touched it.
+// ternary vector with exactly h entries +-1 (partial Fisher-Yates): the drawn
+// positions in order, each as 2 * position + (1 for -1).  The whole shuffled
+// array is made: with a map of its touched places alone, Encrypt took 357 us
+// against 97 at h = 8192 of N = 2^13 (584 against 184 at 24 limbs of 2^16),
+// and no less at h = 192 (60 against 61, 159 against 146).
 std::vector<uint32_t> ternary_positions(u64 seed, u64 stream, int N, int h) {
-  std::unordered_map<int, int> moved;
-  auto at = [&](int i) { auto it = moved.find(i); return it == moved.end() ? i : it->second; };
+  std::vector<int> idx(N);
+  for (int i = 0; i < N; i++) idx[i] = i;
   if (h > N) h = N;
   std::vector<uint32_t> pos(h);
   for (int k = 0; k < h; k++) {
-    u64 r = rand64(seed, stream, (u64)k);
-    int j = k + (int)(((u128)r * (u64)(N - k)) >> 64);
-    const int a = at(k), b = at(j);
-    moved[j] = a;  // place k is drawn and not read again
-    pos[k] = 2 * (uint32_t)b + (uint32_t)(rand64(seed, stream, (1ULL << 32) + (u64)k) & 1);
+    const u64 r = rand64(seed, stream, (u64)k);
+    const int j = k + (int)(((u128)r * (u64)(N - k)) >> 64);
+    std::swap(idx[k], idx[j]);
+    pos[k] = 2 * (uint32_t)idx[k] + (uint32_t)(rand64(seed, stream, (1ULL << 32) + (u64)k) & 1);
   }
   return pos;
 }

@@ -102,10 +102,11 @@ def test_encode_encrypt_sizes(hip_lib, logn):
         hip_lib.DeleteScheme()
 
 
-@pytest.mark.parametrize("h", [255, 256, 257, 700])
+@pytest.mark.parametrize("h", [255, 256, 257, 700, 1024])
 def test_encrypt_positions(hip_lib, h):
     """The ternary polynomial's positions travel with the launch up to 256 and
-    through memory above; one limb and several, a modulus of 61 bits in P."""
+    through memory above, up to every place of the ring; one limb and several, a
+    modulus of 61 bits in P."""
     q, p = make_params(10, [60, 50, 40, 55], [61, 61])
     new_hip_scheme(hip_lib, 10, q, p, 40, h, 4, evaluator=False)
     orc = O.Oracle(10, q, p, h=h, seed=4)

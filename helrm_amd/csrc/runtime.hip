@@ -2202,12 +2202,10 @@ int RotateAdd(int ctID, int amount) {
     return ctID;
   });
 }
-// RotateNew into an existing ciphertext with no allocation: the key switch's
-// temporaries live in the device scratch array, the automorphism tables and
-// basis-conversion tables were built with the key and the scheme.  The
-// rotation key must exist already.  A call on the other stream of the
-// scheme waits for the previous call's key switch; calls from several host
-// threads or processes sharing the GPU race on the array.
+// [ext] RotateAdd by each amount in turn: a Linear's whole output fold.  Two or
+// more steps run as one chain (fold_rotations) where its kernels take the
+// level, else step by step, with the same words.  Every key is made before the
+// first step, and ct is replaced after the last.
 int RotateAddMany(int ctID, const int* amounts, int lenAmounts) {
   return guard([&] {
     Scheme& s = sch();
@@ -2223,16 +2221,26 @@ int RotateAddMany(int ctID, const int* amounts, int lenAmounts) {
       if (fold_chains(ct.level, ge.size())) {
         fold_rotations(ct, ge);
       } else {
+        // ct keeps its words until the last step is queued, as in fold_rotations
+        std::unique_ptr<Cipher> sum;
         for (u64 g : ge) {
+          const Cipher& in = sum ? *sum : ct;
           auto out = new_ct(ct.level, ct.scale);
-          automorphism_core(ct, g, key_ptr(g, false), perm_inv_for(g), out->d.p, nullptr, ct.d.p);
-          std::swap(ct.d, out->d);
+          automorphism_core(in, g, key_ptr(g, false), perm_inv_for(g), out->d.p, nullptr, in.d.p);
+          sum = std::move(out);
         }
+        if (sum) std::swap(ct.d, sum->d);
       }
     });
     return ctID;
   });
 }
+// RotateNew into an existing ciphertext with no allocation: the key switch's
+// temporaries live in the device scratch array, the automorphism tables and
+// basis-conversion tables were built with the key and the scheme.  The
+// rotation key must exist already.  A call on the other stream of the
+// scheme waits for the previous call's key switch; calls from several host
+// threads or processes sharing the GPU race on the array.
 int RotateInto(int ctID, int amount, int outID) {
   return guard([&] {
     Scheme& s = sch();

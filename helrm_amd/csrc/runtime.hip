@@ -2211,6 +2211,7 @@ int RotateAddMany(int ctID, const int* amounts, int lenAmounts) {
     Scheme& s = sch();
     Cipher& ct = get_ct(ctID);
     REQUIRE(lenAmounts >= 0, "RotateAddMany: negative number of rotations");
+    REQUIRE(amounts || lenAmounts == 0, "RotateAddMany: no rotations given");
     std::vector<u64> ge;
     for (int i = 0; i < lenAmounts; i++) {
       ge.push_back(galois_element(amounts[i]));

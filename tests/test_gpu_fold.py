@@ -95,6 +95,8 @@ def test_fold_refuses_and_leaves_input(hip_lib):
         with pytest.raises(HipError, match="ciphertext not found"):
             hip_lib.RotateAddMany(ct + 100, [1, 2])
         assert hip_lib.RotateAddMany(ct, []) == ct
+        for amounts, length in ((None, 2), (None, -1)):
+            assert hip_lib.RotateAddMany.func(ct, amounts, length) == -1
         assert_equal_u64(hip_lib.export_ciphertext(ct), before, "empty fold")
     finally:
         hip_lib.DeleteScheme()

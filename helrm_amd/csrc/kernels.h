@@ -233,8 +233,8 @@ struct BConvJob {
 #define HCK_MAXJOBS 16
 // ginv: 0, or the inverse of a Galois element whose automorphism the source
 // already carries (LinkArgs): at the positions whose sign it changed the
-// extension is taken of the negated sources and negated (launches of the
-// shared-source form only).
+// extension is taken of the negated sources and negated (at most 8 sources a
+// job: such a launch takes the shared-source form whatever its size).
 struct BConvJobs { BConvJob j[HCK_MAXJOBS]; int n, rows_per_block; uint32_t ginv; };
 // Basis extension of every job for every batch entry, in one launch.
 void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, size_t out_bstride, int batch,

@@ -7,6 +7,7 @@
 #include "kernels.h"
 #include <algorithm>
 #include <cstddef>
+#include <stdexcept>
 
 // High word of a 128-bit sum of products of words < q < 2^62: after at most
 // 16 products (plus one earlier fold) it is below 5q; bring it below q.
@@ -484,8 +485,11 @@ void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, si
   if (nrows <= 0) return;
   // all destination rows in one thread unless that leaves too few workgroups
   const int cols = N / 256;
-  // a launch of at most a few waves per SIMD: the shared-source form
-  if (nsmax <= 8 && N % BCL_X == 0 && (long)cols * batch * jobs.n < BCL_MAX_BLOCKS) {
+  // a launch of at most a few waves per SIMD: the shared-source form; also any
+  // under an automorphism, which the other form knows nothing of
+  const bool shared_ok = nsmax <= 8 && N % BCL_X == 0;
+  if (jobs.ginv && !shared_ok) throw std::invalid_argument("basis extension under an automorphism: more than 8 sources");
+  if (shared_ok && (jobs.ginv || (long)cols * batch * jobs.n < BCL_MAX_BLOCKS)) {
     hipLaunchKernelGGL(bconv_lds_kernel, dim3(N / BCL_X, 1, batch * jobs.n), dim3(256), 0, st, in, in_bstride, jobs, out,
                        out_bstride, mods, N);
     return;

@@ -83,31 +83,32 @@ struct KeyMac1Args {
 };
 
 // From the product of one key switch to the digits of the next, in the
-// coefficient domain (link_kernel): per batch entry, with z the coefficients
-// of the QP polynomial x1 (level l) and M = (z - [z]_P) * P^-1 its ModDown,
-//   c1 = M (+ c1, with acc), and every digit of c1 extended to its other QP rows.
-// With x0p (P rows of a second QP polynomial) also e0 = -[x0p]_P * P^-1 on
+// coefficient domain (link_kernel): with z the coefficients of the QP
+// polynomial x1 (level l) and M = (z - [z]_P) * P^-1 its ModDown,
+//   c1 += M, every digit of c1 extended to its other QP rows,
+// and from x0p, the P rows of a second QP polynomial, e0 = -[x0p]_P * P^-1 on
 // the Q rows.  ginv: 0, or the inverse of the Galois element whose
 // automorphism x0p and x1 already carry: ModDown rounds down, so at the
 // positions where the automorphism changed the sign it is taken of the
 // negated word and the result is negated.
 struct LinkArgs {
-  const u64* x1; size_t x1_bstride;    // [nqp][N]
-  const u64* x0p;                      // [K][N] or nullptr (batch 1 only)
-  u64* c1; size_t c1_bstride;          // [l+1][N]
+  const u64* x1;                       // [nqp][N]
+  const u64* x0p;                      // [K][N]
+  u64* c1;                             // [l+1][N]
   u64* e0;                             // [l+1][N]
-  u64* digits; size_t dig_bstride;     // [dn][nqp][N]
+  u64* digits;                         // [dn][nqp][N]
   const struct BConvTable* ptab;       // P -> Q
   const struct BConvTable* dtab[HCK_MAXDIG];  // per digit
   const u64 *pinv, *pinvp;
   const ModC* mods;
-  int N, l, L, K, nqp, dn, acc;
+  int N, l, L, K, nqp, dn;
   uint32_t ginv;
 };
-// LDS bytes of a link launch; at most LINK_LDS_MAX (K <= 8, dn <= HCK_MAXDIG) can be launched
+// LDS bytes of a link launch, at most LINK_LDS_MAX: its caller's limits, K <= 8
+// and dn <= HCK_KM1_DIG, leave up to 64 Q rows, 64 KB
 #define LINK_LDS_MAX 65536
 size_t link_lds_bytes(int l);
-void launch_link(const LinkArgs& a, int batch, hipStream_t st);
+void launch_link(const LinkArgs& a, hipStream_t st);
 
 struct GiantAccArgs {
   const u64* digits;  // [ng][dn][nqp][N]
@@ -241,8 +242,7 @@ void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, si
                   const ModC* mods, int N, hipStream_t st);
 // Single source group: the sources are rows [0, ns) of in.
 void launch_bconv(const u64* in, size_t in_bstride, int ns, const BConvTable* dtab, u64* out, size_t out_bstride, int batch,
-                  const RowMap& rm, const ModC* mods, int N, bool force_v0, hipStream_t st);
-void launch_moddown_combine(u64* out, size_t o_bstride, const u64* x, size_t x_bstride, const u64* ext, size_t e_bstride, const u64* add, size_t a_bstride, int add_batches, const uint32_t* perm, const u64* pinv, const u64* pinvp, int qrows, int batch, const ModC* mods, int N, hipStream_t st);
+                  const RowMap& rm, const ModC* mods, int N, hipStream_t st);
 void launch_keymac(const KeyMacArgs& a, int batch, hipStream_t st);
 void launch_keymac1(const KeyMac1Args& a, hipStream_t st);
 void launch_giant_acc(const GiantAccArgs& a, hipStream_t st);
@@ -266,7 +266,7 @@ void launch_moddown_rescale_spread(u64* ext, size_t e_bstride, const u64* xl, si
                                    u64 pinvlp, const u64* pmod_w, const u64* pmod_wp, const ModC* mods, int N, int batch,
                                    hipStream_t st);
 void launch_sample_uniform(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, hipStream_t st);
-void launch_sample_cbd(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, bool add, hipStream_t st);
+void launch_sample_cbd(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, hipStream_t st);
 void launch_signed_rows(u64* out, RowMap rm, const int8_t* v, const ModC* mods, int N, hipStream_t st);
 // positions small enough to travel in the kernel arguments
 struct TernaryPos {

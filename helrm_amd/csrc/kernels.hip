@@ -379,19 +379,18 @@ __device__ __forceinline__ BConvSrc bconv_src(cwords tab, int i) {
 __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   extern __shared__ u64 sm[];
   const int lane = threadIdx.x & (BCL_X - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / BCL_X);
-  const int N = a.N, K = a.K, nq = a.l + 1, nqp = a.nqp, b = blockIdx.y;
+  const int N = a.N, K = a.K, nq = a.l + 1, nqp = a.nqp;
   const int x = blockIdx.x * BCL_X + lane;
-  const u64* x1 = a.x1 + (size_t)b * a.x1_bstride + x;
-  u64* c1 = a.c1 + (size_t)b * a.c1_bstride + x;
-  u64* digits = a.digits + (size_t)b * a.dig_bstride + x;
-  const bool two = a.x0p != nullptr;
+  const u64* x1 = a.x1 + x;
+  u64* c1 = a.c1 + x;
+  u64* digits = a.digits + x;
   const bool flip = ((uint32_t)x * a.ginv & (uint32_t)(2 * N - 1)) >= (uint32_t)N;
   // LDS: source terms (P rows: y and y / p of both polynomials, 8 slots each;
   // then the Q rows' y and y / q)
   const cwords pt = const_words(a.ptab);  // BConvTable: 4 words a source, then the pointers hat and nS
   const cwords phat = const_words((const void*)pt[4 * HCK_MAXSRC]), pnS = const_words((const void*)pt[4 * HCK_MAXSRC + 1]);
   const cwords mods = const_words(a.mods), pinv = const_words(a.pinv), pinvp = const_words(a.pinvp);
-  for (int part = two ? 0 : 1; part < 2; part++) {
+  for (int part = 0; part < 2; part++) {
     const u64* src = part ? x1 + (size_t)nq * N : a.x0p + x;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
@@ -412,15 +411,13 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   for (int i = 0; i < 8; i++) {
     y1[i] = sm[(16 + i) * BCL_X + lane];
     v1f += __longlong_as_double((long long)sm[(24 + i) * BCL_X + lane]);
-    if (two) {
-      y0[i] = sm[i * BCL_X + lane];
-      v0f += __longlong_as_double((long long)sm[(8 + i) * BCL_X + lane]);
-    }
+    y0[i] = sm[i * BCL_X + lane];
+    v0f += __longlong_as_double((long long)sm[(8 + i) * BCL_X + lane]);
   }
   const uint32_t v1 = (uint32_t)(u64)v1f, v0 = (uint32_t)(u64)v0f;
   __syncthreads();
   // a row's words are loaded while the row before it is computed
-  u64 zn = w < nq ? x1[(size_t)w * N] : 0, cn = a.acc && w < nq ? c1[(size_t)w * N] : 0;
+  u64 zn = w < nq ? x1[(size_t)w * N] : 0, cn = w < nq ? c1[(size_t)w * N] : 0;
   for (int r = w; r < nq; r += 4) {
     const u64 q = mods[4 * r], qinv = mods[4 * r + 1];
     const cwords h = phat + (size_t)r * K;
@@ -428,7 +425,7 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
     const u64 z = zn, c = cn;
     const int rn = min(r + 4, nq - 1);
     zn = x1[(size_t)rn * N];
-    if (a.acc) cn = c1[(size_t)rn * N];
+    cn = c1[(size_t)rn * N];
     const u64 e1 = bconv_word8([&](int i) { return y1[i]; }, h, v1, n, q, qinv);
     const u64 m = shoup_mul(flip ? add_mod(z, e1, q) : sub_mod(z, e1, q), pi, pip, q);
     const u64 s = add_mod(c, m, q);
@@ -437,11 +434,9 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
     const u64 yi = shoup_mul(s, sd.hinv, sd.hinvp, sd.q);
     sm[r * BCL_X + lane] = yi;
     sm[(nq + r) * BCL_X + lane] = (u64)__double_as_longlong((double)yi / sd.qd);
-    if (two) {
-      u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, v0, n, q, qinv);
-      e0 = shoup_mul(e0, pi, pip, q);
-      a.e0[(size_t)r * N + x] = flip || e0 == 0 ? e0 : q - e0;
-    }
+    u64 e0 = bconv_word8([&](int i) { return y0[i]; }, h, v0, n, q, qinv);
+    e0 = shoup_mul(e0, pi, pip, q);
+    a.e0[(size_t)r * N + x] = flip || e0 == 0 ? e0 : q - e0;
   }
   __syncthreads();
   int first = w;  // this wave's first row of the digit: rows are dealt round robin over all digits
@@ -471,8 +466,8 @@ __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   }
 }
 size_t link_lds_bytes(int l) { return (size_t)std::max(4 * 8, 2 * (l + 1)) * BCL_X * 8; }
-void launch_link(const LinkArgs& a, int batch, hipStream_t st) {
-  hipLaunchKernelGGL(link_kernel, dim3(a.N / BCL_X, batch), dim3(256), link_lds_bytes(a.l), st, a);
+void launch_link(const LinkArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL(link_kernel, dim3(a.N / BCL_X), dim3(256), link_lds_bytes(a.l), st, a);
 }
 void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, size_t out_bstride, int batch,
                   const ModC* mods, int N, hipStream_t st) {
@@ -507,10 +502,10 @@ void launch_bconv(const u64* in, size_t in_bstride, BConvJobs jobs, u64* out, si
     hipLaunchKernelGGL((bconv_kernel<HCK_MAXSRC>), grid, dim3(256), 0, st, in, in_bstride, jobs, out, out_bstride, mods, N);
 }
 void launch_bconv(const u64* in, size_t in_bstride, int ns, const BConvTable* dtab, u64* out, size_t out_bstride, int batch,
-                  const RowMap& rm, const ModC* mods, int N, bool force_v0, hipStream_t st) {
+                  const RowMap& rm, const ModC* mods, int N, hipStream_t st) {
   BConvJobs jobs{};
   jobs.n = 1;
-  jobs.j[0] = BConvJob{dtab, 0, ns, force_v0 ? 1 : 0, 0, rm, 0};
+  jobs.j[0] = BConvJob{dtab, 0, ns, 0, 0, rm, 0};
   launch_bconv(in, in_bstride, jobs, out, out_bstride, batch, mods, N, st);
 }
 
@@ -528,29 +523,6 @@ void launch_mul_i(u64* out, const u64* in, size_t bstride, int batch, RowMap rm,
   if (batch <= 0 || rm.nact() <= 0) return;
   hipLaunchKernelGGL(mul_i_kernel, dim3(N / 256, rm.nact(), batch), dim3(256), 0, st, out, in, bstride, rm, iu, iup, niu, niup,
                      mods, N);
-}
-
-// ModDown combine: out = (x - ext) * P^-1 (+ add) [gathered through perm]
-// x rows = Q rows of a QP poly (stride x_bstride), ext rows = Q rows.
-__global__ void moddown_combine_kernel(u64* __restrict__ out, size_t o_bstride, const u64* __restrict__ x, size_t x_bstride,
-                                       const u64* __restrict__ ext, size_t e_bstride, const u64* __restrict__ add, size_t a_bstride,
-                                       int add_batches, const uint32_t* __restrict__ perm, const u64* __restrict__ pinv,
-                                       const u64* __restrict__ pinvp, const ModC* __restrict__ mods, int N) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  int r = blockIdx.y, b = blockIdx.z;
-  int src = perm ? (int)perm[i] : i;
-  u64 q = mods[r].q;
-  u64 v = sub_mod(x[(size_t)b * x_bstride + (size_t)r * N + src], ext[(size_t)b * e_bstride + (size_t)r * N + src], q);
-  v = shoup_mul(v, pinv[r], pinvp[r], q);
-  if (add && b < add_batches) v = add_mod(v, add[(size_t)b * a_bstride + (size_t)r * N + src], q);
-  out[(size_t)b * o_bstride + (size_t)r * N + i] = v;
-}
-void launch_moddown_combine(u64* out, size_t o_bstride, const u64* x, size_t x_bstride, const u64* ext, size_t e_bstride,
-                            const u64* add, size_t a_bstride, int add_batches, const uint32_t* perm, const u64* pinv,
-                            const u64* pinvp, int qrows, int batch, const ModC* mods, int N, hipStream_t st) {
-  if (qrows <= 0 || batch <= 0) return;
-  hipLaunchKernelGGL(moddown_combine_kernel, dim3(N / 256, qrows, batch), dim3(256), 0, st, out, o_bstride, x, x_bstride, ext,
-                     e_bstride, add, a_bstride, add_batches, perm, pinv, pinvp, mods, N);
 }
 
 // The counter PRNG of the key generator (see rand64 below).
@@ -1234,19 +1206,17 @@ __global__ void sample_uniform_kernel(u64* __restrict__ out, RowMap rm, u64 seed
 void launch_sample_uniform(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, hipStream_t st) {
   hipLaunchKernelGGL(sample_uniform_kernel, dim3(N / 256, rm.nact(), 1), dim3(256), 0, st, out, rm, seed, stream, mods, N);
 }
-// centred binomial (eta = 21) error, the same integer reduced into every row; optionally added
-__global__ void sample_cbd_kernel(u64* __restrict__ out, RowMap rm, u64 seed, u64 stream, const ModC* __restrict__ mods, int N, int add) {
+// centred binomial (eta = 21) error, the same integer reduced into every row
+__global__ void sample_cbd_kernel(u64* __restrict__ out, RowMap rm, u64 seed, u64 stream, const ModC* __restrict__ mods, int N) {
   int x = blockIdx.x * blockDim.x + threadIdx.x;
   int row = rm.row(blockIdx.y);
   u64 q = mods[rm.mod(row)].q;
   u64 r = rand64(seed, stream, (u64)x);
   int e = __popcll(r & 0x1FFFFFULL) - __popcll((r >> 21) & 0x1FFFFFULL);
-  u64 v = e >= 0 ? (u64)e : q - (u64)(-e);
-  size_t o = (size_t)row * N + x;
-  out[o] = add ? add_mod(out[o], v, q) : v;
+  out[(size_t)row * N + x] = e >= 0 ? (u64)e : q - (u64)(-e);
 }
-void launch_sample_cbd(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, bool add, hipStream_t st) {
-  hipLaunchKernelGGL(sample_cbd_kernel, dim3(N / 256, rm.nact(), 1), dim3(256), 0, st, out, rm, seed, stream, mods, N, add ? 1 : 0);
+void launch_sample_cbd(u64* out, RowMap rm, u64 seed, u64 stream, const ModC* mods, int N, hipStream_t st) {
+  hipLaunchKernelGGL(sample_cbd_kernel, dim3(N / 256, rm.nact(), 1), dim3(256), 0, st, out, rm, seed, stream, mods, N);
 }
 // small signed integers (int8, e.g. ternary) reduced into every row
 __global__ void signed_rows_kernel(u64* __restrict__ out, RowMap rm, const int8_t* __restrict__ v, const ModC* __restrict__ mods, int N) {

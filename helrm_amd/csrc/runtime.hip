@@ -653,7 +653,7 @@ void mod_down(int l, const u64* x, size_t x_bstride, int batch, u64* out, size_t
   // P rows of x (rows l+1.. of each batch entry) -> coefficient domain in pc
   ntt_oop(x + (size_t)(l + 1) * N, x_bstride, pc, (size_t)K * N, batch, rows_p(), false);
   BConvHost& bt = bconv_table_cached(s.L, s.L + K);
-  launch_bconv(pc, (size_t)K * N, K, bt.dtab.p, ext, (size_t)(l + 1) * N, batch, rows_q(l), s.d_mods.p, N, false, s.st);
+  launch_bconv(pc, (size_t)K * N, K, bt.dtab.p, ext, (size_t)(l + 1) * N, batch, rows_q(l), s.d_mods.p, N, s.st);
   // forward transform of the extension fused with (x - ext) * P^-1 (+ add), gathered through perm
   launch_ntt_moddown(ext, (size_t)(l + 1) * N, batch, l, s.logN, x, x_bstride, out, o_bstride, add, a_bstride,
                      add_batches, perm_inv, s.pinv_w.p, s.pinv_wp.p, s.tw, s.st, acc, o_bstride);
@@ -674,8 +674,7 @@ void mod_down_rescale(int l, const u64* x, size_t x_bstride, int batch, u64* out
   // rows l (q_l) and l+1.. (P) of x are consecutive: one inverse transform
   ntt_oop(x + (size_t)l * N, x_bstride, pcq.p, (size_t)(K + 1) * N, batch, RowMap{K + 1, 1, l, s.L, 0, 0}, false);
   BConvHost& bt = bconv_table(s.L, s.L + K);
-  launch_bconv(pcq.p + N, (size_t)(K + 1) * N, K, bt.dtab.p, ext.p, (size_t)(l + 1) * N, batch, rows_q(l), s.d_mods.p, N, false,
-               s.st);
+  launch_bconv(pcq.p + N, (size_t)(K + 1) * N, K, bt.dtab.p, ext.p, (size_t)(l + 1) * N, batch, rows_q(l), s.d_mods.p, N, s.st);
   launch_moddown_rescale_spread(ext.p, (size_t)(l + 1) * N, pcq.p, (size_t)(K + 1) * N, l, s.mod[l] >> 1, s.pinv_h[l],
                                 s.pinv_hp[l], s.pmod_w.p, s.pmod_wp.p, s.d_mods.p, N, batch, s.st);
   launch_ntt_moddown(ext.p, (size_t)(l + 1) * N, batch, l - 1, s.logN, x, x_bstride, out, o_bstride, nullptr, 0, 0, nullptr,
@@ -711,7 +710,7 @@ void gen_public() {
   DU64 b((size_t)nm * N), a((size_t)nm * N);
   launch_sample_uniform(a.p, rows_all(), s.seed, ST_PK_A, s.d_mods.p, N, s.st);
   ntt(a.p, 0, 1, rows_all(), true);
-  launch_sample_cbd(b.p, rows_all(), s.seed, ST_PK_E, s.d_mods.p, N, false, s.st);
+  launch_sample_cbd(b.p, rows_all(), s.seed, ST_PK_E, s.d_mods.p, N, s.st);
   ntt(b.p, 0, 1, rows_all(), true);
   launch_gk_combine(b.p, a.p, s.sR.p, s.sR.p, 0, 0, s.pmod_plain.p, nm, s.d_mods.p, N, s.st);
   s.pkR = DU64((size_t)2 * nm * N);
@@ -735,7 +734,7 @@ std::unique_ptr<DU64> gen_eval_key(const u64* s_inR, const u64* s_outR, FA st_a,
     // uniform in either domain; Lattigo's key generator samples it there too),
     // so any word of it is a function of (seed, stream, modulus, position)
     launch_sample_uniform(a, rows_all(), s.seed, st_a(d), s.d_mods.p, N, s.st);
-    launch_sample_cbd(b, rows_all(), s.seed, st_e(d), s.d_mods.p, N, false, s.st);
+    launch_sample_cbd(b, rows_all(), s.seed, st_e(d), s.d_mods.p, N, s.st);
     ntt(b, 0, 1, rows_all(), true);
     launch_gk_combine(b, a, s_outR, s_inR, d * K, std::min((d + 1) * K, s.L), s.pmod_plain.p, nm, s.d_mods.p, N, s.st);
   }
@@ -1193,7 +1192,7 @@ void fold_rotations(Cipher& ct, const std::vector<u64>& ge) {
   BConvHost& bt = bconv_table_cached(s.L, s.L + K);
   lk.x1 = dd + (size_t)nqp * N; lk.x0p = ddp; lk.c1 = coef; lk.e0 = ws + w.e0; lk.digits = digits; lk.ptab = bt.dtab.p;
   lk.pinv = s.pinv_w.p; lk.pinvp = s.pinv_wp.p; lk.mods = s.d_mods.p;
-  lk.N = N; lk.l = l; lk.L = s.L; lk.K = K; lk.nqp = nqp; lk.dn = dn; lk.acc = 1;
+  lk.N = N; lk.l = l; lk.L = s.L; lk.K = K; lk.nqp = nqp; lk.dn = dn;
   const u64 M = 2 * (u64)N;
   for (size_t i = 0; i < ge.size(); i++) {
     const uint32_t ginv = (uint32_t)invmod_odd(ge[i], M);
@@ -1221,7 +1220,7 @@ void fold_rotations(Cipher& ct, const std::vector<u64>& ge) {
     }
     launch_ntt_list(ws, fr.inv.p, fr.ninv, s.logN, false, s.tw, s.st);
     lk.ginv = ginv;
-    launch_link(lk, 1, s.st);
+    launch_link(lk, s.st);
     launch_ntt_list(ws, fr.fwd.p, fr.nfwd, s.logN, true, s.tw, s.st);
     own = ws + w.c1n; c0 = c0cur; e0 = ws + w.e0;
   }
@@ -1851,7 +1850,7 @@ std::unique_ptr<Cipher> encrypt_seeded(const Plain& pt, u64 seed) {
   auto out = new_ct(l, pt.scale); out->logslots = pt.logslots;
   u64* b = out->d.p;
   expand_seeded_a(*out, seed);
-  launch_sample_cbd(b, rows_q(l), s.seed, ST_SEED_E(enc), s.d_mods.p, N, false, s.st);
+  launch_sample_cbd(b, rows_q(l), s.seed, ST_SEED_E(enc), s.d_mods.p, N, s.st);
   ntt(b, 0, 1, rows_q(l), true);
   DU64 as((size_t)(l + 1) * N);
   launch_mont_mul(as.p, 0, b + (size_t)(l + 1) * N, 0, s.sR.p, 0, 1, rows_q(l), s.d_mods.p, N, nullptr, s.st);

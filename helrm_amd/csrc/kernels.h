@@ -125,8 +125,7 @@ struct GiantAccArgs {
   u64 *out0, *out1;            // QP accumulators [nqp][N]
   const ModC* mods;
   int N, l, L, K, nqp, dn;
-  const u64* ka;               // [ng][ka_stride] per-stream PRNG keys of the keys' a halves (regenerated), or nullptr (read)
-  int ka_stride;               // a key's digits: dn at the top level, more than dn below
+  const u64* ka;               // [ng][dn] per-stream PRNG keys of the keys' a halves (regenerated), or nullptr (read)
 };
 
 // Diagonals of a dense 16-baby transform are stored packed: a row whose
@@ -159,8 +158,7 @@ struct DiagMacArgs {
   const uint32_t* const* bperm;   // per baby slot: automorphism gather
   const u64* own;                 // c1 (Q rows, NTT): a digit's own rows
   int dn;
-  const u64* bka;                 // [slot][bka_stride] per-stream PRNG keys of the a halves (regenerated), or nullptr (read)
-  int bka_stride;                 // a key's digits, as GiantAccArgs::ka_stride
+  const u64* bka;                 // [slot][dn] per-stream PRNG keys of the a halves (regenerated), or nullptr (read)
   const uint32_t* pkrow;          // packed layout: [row][2] descriptors, nullptr for plain [np][nqp][N]
   int gper;  // groups of a workgroup (set by the launch)
 };

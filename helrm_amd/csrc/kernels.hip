@@ -709,7 +709,7 @@ __global__ __launch_bounds__(256) void giant_acc_kernel(GiantAccArgs a) {
     const int src = (int)perm[i];
     const u64* dg = a.digits + (size_t)g * a.dig_bstride;
     const u64* own = a.own ? a.own + (size_t)g * a.own_bstride + (size_t)k * N : nullptr;
-    const u64* ka = a.ka ? a.ka + (size_t)g * a.ka_stride : nullptr;
+    const u64* ka = a.ka ? a.ka + (size_t)g * a.dn : nullptr;
     for (int d = 0; d < a.dn; d++) {
       const u64 x = d == own_d ? own[src] : dg[((size_t)d * a.nqp + k) * N + src];
       const u64* kb = key + (size_t)d * 2 * kstride + (size_t)kl * N + src;
@@ -783,7 +783,7 @@ __global__ __launch_bounds__(256) void giant_acc_dn_kernel(GiantAccArgs a) {
 #pragma unroll
     for (int d = 0; d < DN; d++) {
       acc_mac(A0, x[d], kb[d]);
-      acc_mac(A1, x[d], SEEDED ? key_a_word(a.ka[(size_t)g * a.ka_stride + d], (u64)kl * N + src, mc.q) : ka[d]);
+      acc_mac(A1, x[d], SEEDED ? key_a_word(a.ka[(size_t)g * DN + d], (u64)kl * N + src, mc.q) : ka[d]);
     }
     t0 = add_mod(t0, t, mc.q);
   }
@@ -893,7 +893,7 @@ __device__ __forceinline__ void baby_rotation_at(const DiagMacArgs& a, int slot,
   const int N = a.N;
   const int src = (int)a.bperm[slot][x];
   const u64* key = a.bkey[slot];
-  const u64* ka = a.bka ? a.bka + (size_t)slot * a.bka_stride : nullptr;
+  const u64* ka = a.bka ? a.bka + (size_t)slot * a.dn : nullptr;
   const int own_d = k <= a.l ? k / a.K : -1;
   const size_t kstride = (size_t)(a.L + a.K) * N;
   Acc128 A0, A1;

@@ -334,7 +334,8 @@ struct LinTrans {
   double scale = 0;
   // device arrays of key / permutation pointers (baby and giant rotations), built on first use
   DevArray<const u64*> d_bkey, d_gkey; DevArray<const uint32_t*> d_bperm, d_gperm; DevArray<int> d_tg;
-  DevArray<u64> d_bka, d_gka;  // [key][dnum] stream keys of the keys' a halves (used when every key was generated here)
+  // by digit count: [baby key][dn] and [giant key][dn] stream keys of the keys' a halves (used when every key was generated here)
+  std::map<int, std::pair<DU64, DU64>> d_ka;
   bool ptrs_ready = false;
 };
 
@@ -1676,17 +1677,23 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
       tm.d_tg = DevArray<int>(std::max(ngk, 1));
       if (nbr) { upload(tm.d_bkey.p, bk.data(), nbr); upload(tm.d_bperm.p, bp.data(), nbr); }
       if (ngk) { upload(tm.d_gkey.p, gk.data(), ngk); upload(tm.d_gperm.p, gp.data(), ngk); upload(tm.d_tg.p, tg.data(), ngk); }
-      // the stream keys of a key's dnum digits depend on the Galois element
-      // alone: the tables serve every level, also one of fewer digits
-      const int dnum = s.dnum;
-      std::vector<u64> bka((size_t)std::max(nbr, 1) * dnum), gka((size_t)std::max(ngk, 1) * dnum);
-      for (int i = 0; i < nbr; i++)
-        for (int d = 0; d < dnum; d++) bka[(size_t)i * dnum + d] = stream_key(ST_GK_A(galois_element(babies[i]), (u64)d));
-      for (int g = 0; g < ngk; g++)
-        for (int d = 0; d < dnum; d++) gka[(size_t)g * dnum + d] = stream_key(ST_GK_A(galois_element(t.giant[gs + g]), (u64)d));
-      tm.d_bka = DevArray<u64>(bka.size()); upload(tm.d_bka.p, bka.data(), bka.size());
-      tm.d_gka = DevArray<u64>(gka.size()); upload(tm.d_gka.p, gka.data(), gka.size());
       tm.ptrs_ready = true;
+    }
+    // the stream keys depend on the Galois element alone; a table a digit
+    // count, since the kernels read one key's dn words after another's (a
+    // stride of all dnum digits instead cost giant_acc_dn_kernel<3> 33 -> 43 us
+    // at N = 2^13)
+    auto& ka = tm.d_ka[dn];
+    if (!ka.first.p) {
+      std::vector<u64> bka((size_t)std::max(nbr, 1) * dn), gka((size_t)std::max(ngk, 1) * dn);
+      for (int i = 0; i < nbr; i++)
+        for (int d = 0; d < dn; d++) bka[(size_t)i * dn + d] = stream_key(ST_GK_A(galois_element(babies[i]), (u64)d));
+      for (int g = 0; g < ngk; g++)
+        for (int d = 0; d < dn; d++) gka[(size_t)g * dn + d] = stream_key(ST_GK_A(galois_element(t.giant[gs + g]), (u64)d));
+      DU64 b(bka.size()), g(gka.size());
+      upload(b.p, bka.data(), bka.size());
+      upload(g.p, gka.data(), gka.size());
+      ka = {std::move(b), std::move(g)};
     }
   }
   // the a halves are regenerated in the kernels when every key of the group
@@ -1703,7 +1710,7 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
   dm.diag = t.diags.p; dm.diag_stride = lt_diag_words(t);
   dm.pkrow = t.packed ? t.d_pkrow.p : nullptr;
   dm.digits = digits.p; dm.bkey = t.d_bkey.p; dm.bperm = t.d_bperm.p; dm.own = c1; dm.dn = dn;
-  dm.bka = babies_seeded ? t.d_bka.p : nullptr; dm.bka_stride = s.dnum;
+  dm.bka = babies_seeded ? t.d_ka.at(dn).first.p : nullptr;
   dm.pc = pc.p; dm.pc_pstride = (size_t)(l + 1) * N;
   dm.baby_is_zero = t.d_bzero.p; dm.baby_slot = t.d_bslot.p; dm.gpi = t.d_gpi.p; dm.dense = t.dense ? 1 : 0;
   dm.zero_pidx = (int)t.plain_idx.size();
@@ -1730,7 +1737,7 @@ std::unique_ptr<Cipher> eval_lt_bsgs(const LinTrans& t, const Cipher& ct, bool r
     a.T = T.p; a.T_gstride = 2 * qp; a.T_pstride = qp; a.t_zero = gs ? 0 : -1;
     a.out0 = acc.p; a.out1 = acc.p + qp; a.mods = s.d_mods.p;
     a.N = N; a.l = l; a.L = s.L; a.K = K; a.nqp = nqp; a.dn = dn;
-    a.ka = giants_seeded ? t.d_gka.p : nullptr; a.ka_stride = s.dnum;
+    a.ka = giants_seeded ? t.d_ka.at(dn).second.p : nullptr;
     timed("giant_acc", [&] { launch_giant_acc(a, s.st); });
   } else {
     d2d(acc.p, T.p, 2 * qp * 8);

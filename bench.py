@@ -103,6 +103,45 @@ def keyswitch_pass_rows(level, K, fold_add=False, key_parts=KEY_PARTS):
     return rows
 
 
+def fold_pass_rows(level, K, steps, key_parts=KEY_PARTS):
+    """Rows of N words that a fold of `steps` (two or more) rotations at
+    `level` moves as one chain (RotateAddMany), pass by pass as in
+    keyswitch_pass_rows: the first decomposition, a key product a step, a link
+    with its two transforms between steps, and the last step's ModDown."""
+    ql = level + 1
+    nqp = ql + K
+    dn = (nqp - 1) // K
+    ext = dn * nqp - ql
+    mid = steps - 1
+    return {
+        "inverse NTT of c1": 4 * ql,
+        "extension of the digits": ql + ext,
+        "forward NTT of the extended rows": 4 * ext,
+        # digits and keys read; part 1, part 0's P rows and the new c0 written;
+        # c0 (and after a link its correction e0) read straight and permuted
+        "key products": steps * ((dn * key_parts + dn + 2) * nqp + 2 * ql) + mid * 2 * ql,
+        "inverse NTT of part 1 and part 0's P rows": mid * 4 * (nqp + K),
+        "links": mid * (nqp + K + ql + 2 * ql + ext),
+        "forward NTT of the digits, c1 and e0": mid * 4 * (ext + 2 * ql),
+        "inverse NTT of the last P rows, both parts": 4 * 2 * K,
+        "last extension P -> Q, both parts": 2 * K + 2 * ql,
+        "forward NTT with the last ModDown epilogue": 2 * 2 * ql + (2 * ql + ql + 2 * ql + 2 * ql),
+    }
+
+
+def kernel_times(lib, names):
+    """Launches and mean time of the named kernel timers; a timer that the
+    timed work should have run and that counted nothing is an error, not a
+    figure left out."""
+    kt = {}
+    for name in names:
+        c, tot = lib.kernel_time(name)
+        if not c:
+            raise RuntimeError(f"kernel timer '{name}' counted no launch in the timed passes")
+        kt[name] = {"launches": c, "avg_ms": tot / c}
+    return kt
+
+
 def read_traffic(kernel="diag_mac"):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 PMC summary, if present."""
     path = os.path.join(ROOT, "profiles", f"{kernel}_pcmm26_traffic.json")
@@ -590,20 +629,36 @@ def main():
         o = w.run()
         o.free()
     lib.Synchronize()
-    kt = {}
-    for name in ("diag_mac", "giant_acc", "rotate"):
-        c, tot = lib.kernel_time(name)
-        kt[name] = {"launches": c, "avg_ms": tot / c if c else None}
+    layers = w.linear_layers()
+    folds = [layer.output_rotations for layer in layers if layer.output_rotations]
+    giants = any(lib.lt_info(t)["giant"] > 1 for layer in layers for t in layer.transform_ids.values())
+    kt = kernel_times(lib, ["diag_mac"] + ["giant_acc"] * giants + ["fold"] * bool(folds))
     lib.KernelTimingEnable(0)
     time.sleep(0.05)
     if concurrent:
         w.concurrent = True
+    # the single rotation with the fold's add (RotateAdd), which no workload's
+    # own pass runs any more: the fold's amounts on the layer's output, whose
+    # level is the fold's
+    if folds and len(layers) == 1:
+        amounts = [w.params.get_slots() // 2 ** i for i in range(1, folds[0] + 1)]
+        o = w.run()
+        for r in range(nprof + 1):
+            if r == 1:  # the first pass is not timed
+                lib.Synchronize()
+                lib.KernelTimingEnable(1)
+            for a in amounts:
+                for c in o.ids:
+                    lib.RotateAdd(c, a)
+        lib.Synchronize()
+        kt.update(kernel_times(lib, ["rotate"]))
+        lib.KernelTimingEnable(0)
+        o.free()
 
     L, K = len(cfg["logq"]), len(cfg["logp"])
     N = 1 << cfg["logn"]
     # diagonal-MAC launches per step (one per 32 baby steps of every Linear)
-    launches = max(1, round(kt["diag_mac"]["launches"] / nprof)) if kt["diag_mac"]["launches"] else 1
-    layers = w.linear_layers()
+    launches = max(1, round(kt["diag_mac"]["launches"] / nprof))
     step_bytes, mac_bytes, mac_unit, lt_shapes = 0, 0, 0, []
     ks_bytes = {"giant_acc": 0}
     for layer in layers:
@@ -650,20 +705,27 @@ def main():
                                      "kernel_count_bytes_per_launch": mac_per_launch,
                                      "kernel_count_frac": roofline["kernel_count"]["frac"]}}
     for name, total in ks_bytes.items():
-        n_l = kt[name]["launches"] / nprof if kt[name]["launches"] else 0
-        if not n_l or not kt[name]["avg_ms"]:
+        if name not in kt:
             continue
-        per = total / n_l
+        per = total / (kt[name]["launches"] / nprof)
         gbs = per / (kt[name]["avg_ms"] / 1000.0) / 1e9
         kernel_rooflines[name] = {"algorithmic_bytes_per_launch": per, "avg_ms": kt[name]["avg_ms"],
                                   "achieved_GBs": gbs, "frac": gbs / HBM_PEAK_GBS}
 
-    # the single-ciphertext key switch: the fold's rotations (one key switch
-    # each at the transform's output level, the fold's add inside its last
-    # pass) against the per-rotation bytes
-    if kt["rotate"]["launches"] and len(layers) == 1:
+    # the fold (one chain of key switches at the transform's output level) and
+    # the single key switch with the fold's add, against the bytes of a
+    # rotation and those that their passes move
+    if "rotate" in kt:
         lf = layers[0].level - 1  # the fold runs on the rescaled transform output
         nqp, dn = lf + 1 + K, (lf + 1 + K - 1) // K
+        f_ms, f_n = kt["fold"]["avg_ms"], folds[0]
+        fb, fp = f_n * keyswitch_rotation_bytes(lf, K, N), sum(fold_pass_rows(lf, K, f_n).values()) * N * 8
+        kernel_rooflines["fold"] = {
+            "level": lf, "steps": f_n, "avg_ms": f_ms, "ms_per_step": f_ms / f_n, "algorithmic_bytes_per_fold": fb,
+            "achieved_GBs": fb / (f_ms / 1000.0) / 1e9, "frac": fb / (f_ms / 1000.0) / 1e9 / HBM_PEAK_GBS}
+        if f_n >= 2 and K <= 8 and dn <= 8:  # otherwise it runs step by step
+            kernel_rooflines["fold"].update({"pass_bytes_per_fold": fp, "pass_GBs": fp / (f_ms / 1000.0) / 1e9,
+                                             "pass_frac": fp / (f_ms / 1000.0) / 1e9 / HBM_PEAK_GBS})
         rb = keyswitch_rotation_bytes(lf, K, N)
         r_ms = kt["rotate"]["avg_ms"]
         pb = sum(keyswitch_pass_rows(lf, K, fold_add=True).values()) * N * 8
@@ -671,7 +733,7 @@ def main():
         ub = keyswitch_rotation_bytes(lf, K, N, key_parts=2)
         kernel_rooflines["keyswitch_rotation"] = {
             "level": lf, "algorithmic_bytes_per_rotation": rb, "avg_ms": r_ms,
-            "rotations_per_step": kt["rotate"]["launches"] / nprof,
+            "rotations_timed": kt["rotate"]["launches"],
             "achieved_GBs": rb / (r_ms / 1000.0) / 1e9, "frac": rb / (r_ms / 1000.0) / 1e9 / HBM_PEAK_GBS,
             "per_unit_bytes_per_rotation": ub, "per_unit_frac": ub / (r_ms / 1000.0) / 1e9 / HBM_PEAK_GBS,
             "pass_bytes_per_rotation": pb, "pass_GBs": pb / (r_ms / 1000.0) / 1e9,

@@ -2224,6 +2224,7 @@ int RotateAddMany(int ctID, const int* amounts, int lenAmounts) {
       ensure_galois_key(ge.back());
       s.rot_keys.insert(ge.back());
     }
+    if (ge.empty()) return ctID;
     timed("fold", [&] {
       if (fold_chains(ct.level, ge.size())) {
         fold_rotations(ct, ge);
@@ -2236,7 +2237,7 @@ int RotateAddMany(int ctID, const int* amounts, int lenAmounts) {
           automorphism_core(in, g, key_ptr(g, false), perm_inv_for(g), out->d.p, nullptr, in.d.p);
           sum = std::move(out);
         }
-        if (sum) std::swap(ct.d, sum->d);
+        std::swap(ct.d, sum->d);
       }
     });
     return ctID;

@@ -104,6 +104,41 @@ def test_keyswitch_pass_rows():
     assert sum(folded.values()) == 1092 + 2 * 23
 
 
+def test_fold_pass_rows():
+    """A fold of six steps at level 22 (23 Q + 8 P rows, three digits, 70
+    extended rows): the decomposition 92 + 93 + 280; six key products of 248
+    rows with c0 read twice, five of them e0 too; five links (31 + 8 read, c1
+    and e0 of 23 rows, 70 digit rows) between inverse transforms of 39 and
+    forward ones of 116 limbs; the last ModDown 64 + 62 and 46 limbs whose last
+    pass reads x of part 1 and both addends."""
+    rows = bench.fold_pass_rows(22, 8, 6)
+    assert list(rows.values()) == [92, 93, 280, 6 * (248 + 46) + 5 * 46, 5 * 156, 5 * 178, 5 * 464, 64, 62, 92 + 161]
+    # a step inside the chain moves what a rotation by itself with the add moves, in six launches of eleven
+    step = [a - b for a, b in zip(bench.fold_pass_rows(22, 8, 7).values(), rows.values())]
+    assert sum(step) == 1138 == sum(bench.keyswitch_pass_rows(22, 8, fold_add=True).values())
+    two = bench.fold_pass_rows(22, 8, 2, key_parts=2)
+    assert two["key products"] == 2 * (341 + 46) + 46
+
+
+class Timers:
+    def __init__(self, counts):
+        self.counts = counts
+
+    def kernel_time(self, name):
+        c = self.counts.get(name, 0)
+        return c, 0.5 * c
+
+
+def test_kernel_times_refuse_an_idle_timer():
+    """A timer that the timed passes should have run is never reported as
+    zero launches."""
+    lib = Timers({"diag_mac": 4, "fold": 2})
+    assert bench.kernel_times(lib, ["diag_mac", "fold"]) == {"diag_mac": {"launches": 4, "avg_ms": 0.5},
+                                                             "fold": {"launches": 2, "avg_ms": 0.5}}
+    with pytest.raises(RuntimeError, match="'rotate'"):
+        bench.kernel_times(lib, ["diag_mac", "rotate"])
+
+
 def test_measured_step_traffic():
     """The whole-PCMM traffic of the committed PMC summary, as a rate at a step time."""
     r = bench.measured_step_traffic("pcmm26", 7.0)

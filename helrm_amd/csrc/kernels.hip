@@ -550,7 +550,8 @@ __device__ __forceinline__ u64 key_a_word(u64 kd, u64 ctr, u64 q) {
 // Keys are in Montgomery form; the sum is accumulated lazily in 128 bits.
 // With a.seeded the a halves (k1) are regenerated (key_a_word) instead of
 // read: their products carry no factor R, so part 1 is multiplied by R
-// after its REDC.
+// after its REDC.  Launched for the naive transform's batches and for single
+// key switches of more than HCK_KM1_DIG digits (keymac1_kernel below that).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void keymac_kernel(KeyMacArgs a) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;

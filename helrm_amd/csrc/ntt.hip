@@ -1353,7 +1353,9 @@ void launch_ntt(u64* data, size_t bstride, int batch, RowMap rm, int logN, bool 
 // N = 2^13 then runs on 32 or 64 CUs instead of 8 or 16, and its waves have a
 // SIMD each instead of sharing one with another.  N = 2^13, 4 limbs and one
 // special modulus: a rotation 55 -> 46 us, a whole one-table lookup 456 -> 405
-// us; a bound of 512 measures the same, and N = 2^16 always has more.
+// us; a bound of 512 measures the same.  At N = 2^16 a column tile has its 16
+// words already, and the row passes of up to 7 limbs are halved: a rescale's
+// inverse of 2 limbs 5.3 -> 4.6 us.
 constexpr int W8_FILL = 256;
 // Whether a launch takes the one-workgroup transform: N up to 2^11 always;
 // above, launches of at least 2^(logN - 6) limbs that the 16-word kernels would

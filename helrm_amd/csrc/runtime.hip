@@ -1,11 +1,11 @@
 // runtime.hip -- host runtime and C ABI of the MI355X CKKS backend.
 //
 // One global scheme per process (as the Lattigo wrapper's `scheme`,
-// orion/backend/lattigo/scheme.go:32), one HIP stream, ID-handle registries
-// with lowest-free-id reuse (orion/backend/lattigo/minheap.go:27-98).  All
-// polynomial arithmetic runs on the GPU through kernels.hip; the host does
-// only parameter set-up, the encoder's float64 FFT, the decoder's CRT and
-// sampling of the small ternary vectors.  Every entry point returns -1 (or an
+// orion/backend/lattigo/scheme.go:32), work on one of its two HIP streams,
+// ID-handle registries with lowest-free-id reuse
+// (orion/backend/lattigo/minheap.go:27-98).  All polynomial arithmetic,
+// encoding and decoding run on the GPU; the host does only parameter set-up
+// and sampling of the small ternary vectors.  Every entry point returns -1 (or an
 // empty array) and records a message for GetLastError() instead of aborting.
 #include <hip/hip_runtime.h>
 #include <algorithm>
@@ -784,9 +784,8 @@ u64 stream_key(u64 stream) { return mix64(sch().seed + 0x9e3779b97f4a7c15ULL * (
 
 
 // ============================================================================
-// encoder: root and rotation-group tables (Lattigo ckks.Encoder); the special
-// inverse FFT, fixed-point rounding and residues run on the GPU (encoder.hip),
-// the decoder's forward special FFT on the host
+// encoder: root and rotation-group tables (Lattigo ckks.Encoder) of the special
+// FFTs, which run on the GPU in both directions (encoder.hip)
 // ============================================================================
 void init_encoder(Scheme& s) {
   const int M = 2 * s.N, slots = s.N / 2, quarm = M >> 2;

@@ -102,8 +102,9 @@ int RotateNew(int ciphertextID, int amount); /* evaluator.go:89-101 */
 int RotateAdd(int ciphertextID, int amount);
 /* [ext] RotateAdd by each amount in turn: a Linear's whole output fold in one
  * call.  Same words as the single steps; the key switches of consecutive
- * steps share their transforms.  Every key is made first, so a failure leaves
- * the ciphertext as it was.  Returns ciphertextID. */
+ * steps share their transforms.  Every key is made before the first step and
+ * the ciphertext replaced after the last, so a failure leaves it as it was.
+ * Returns ciphertextID. */
 int RotateAddMany(int ciphertextID, const int* amounts, int lenAmounts);
 /* [ext] No counterpart in the reference.  For callers that cannot allocate
  * device memory (code under HIP graph capture, tight serving loops): RotateNew

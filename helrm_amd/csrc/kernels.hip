@@ -374,8 +374,8 @@ __device__ __forceinline__ BConvSrc bconv_src(cwords tab, int i) {
 // the rows' source terms meet in LDS.  Its tables are read as constant words:
 // behind its own stores the compiler read them as 90 vector loads a wave, a
 // memory round trip a row (22.7 -> 20.4 us at 11 Q rows).  A fold step of 23 Q
-// and 8 P rows at N = 2^16 takes 161 us with it against 190 with the two
-// extensions and the transforms between them.
+// and 8 P rows at N = 2^16 takes 163 us with it against 181 by RotateAdd, with
+// the two extensions and the transforms between them.
 __global__ __launch_bounds__(256) void link_kernel(LinkArgs a) {
   extern __shared__ u64 sm[];
   const int lane = threadIdx.x & (BCL_X - 1), w = __builtin_amdgcn_readfirstlane(threadIdx.x / BCL_X);

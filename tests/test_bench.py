@@ -1,6 +1,8 @@
 """bench.py's contract pieces that need no GPU: the refusal of more than one
 GPU and the algorithmic byte counts its rooflines divide by."""
+import json
 import os
+import re
 import subprocess
 import sys
 
@@ -146,3 +148,14 @@ def test_measured_step_traffic():
     assert r["measured_traffic_bytes"] > 2 * bench.algorithmic_bytes(packed_rows=23)[0]
     assert abs(r["measured_traffic_GBs"] - r["measured_traffic_bytes"] / 7e-3 / 1e9) < 1e-6
     assert bench.measured_step_traffic("dlrm", 7.0) == {}
+
+
+def test_traffic_and_trace_are_of_one_state():
+    """The committed traffic summary, which the bench divides by its step time,
+    and the committed kernel trace count the same launches a query."""
+    with open(os.path.join(ROOT, "profiles", "pcmm26_traffic.json")) as f:
+        dispatches = json.load(f)["dispatches"]
+    with open(os.path.join(ROOT, "profiles", "pcmm26_kernel_trace.md")) as f:
+        text = f.read()
+    assert int(re.search(r"(\d+) launches\.", text).group(1)) == dispatches
+    assert sum(int(n) for n in re.findall(r"^\| `.*` \| (\d+) \|", text, re.M)) == dispatches
